@@ -224,8 +224,10 @@ __device__ __forceinline__ void crt_body(const CrtArgs& a, uint32_t bx) {
 }
 
 template <int NL, bool CPLX>
-__global__ void __launch_bounds__(256) crt_kernel(CrtArgs a) {
+__global__ void __launch_bounds__(256) crt_kernel(CrtArgs a, uint64_t* ts) {
+    const Stamp st(ts);
     crt_body<NL, CPLX>(a, blockIdx.x);
+    st.end();
 }
 
 template <int NL, bool CPLX>
@@ -261,15 +263,15 @@ __global__ void scale_c_kernel(double* C, int64_t ldc, int64_t m, int64_t n, dou
 }
 
 template <int NL>
-void launch_crt_nl(hipStream_t st, const CrtArgs& a) {
+void launch_crt_nl(const Stream& st, const CrtArgs& a) {
     const unsigned blocks = crt_blocks(a);
-    if (a.cplx) hipLaunchKernelGGL((crt_kernel<NL, true>), dim3(blocks), dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((crt_kernel<NL, false>), dim3(blocks), dim3(256), 0, st, a);
+    if (a.cplx) launch(st, crt_kernel<NL, true>, dim3(blocks), dim3(256), a);
+    else launch(st, crt_kernel<NL, false>, dim3(blocks), dim3(256), a);
 }
 
 }  // namespace
 
-void crt(hipStream_t st, const CrtArgs& a) {
+void crt(const Stream& st, const CrtArgs& a) {
     if (a.mb <= 0 || a.nb <= 0) return;
     switch (a.L16 / 2) {
         case 2: launch_crt_nl<2>(st, a); break;

@@ -19,12 +19,16 @@ void hip_check(hipError_t e, const char* what) {
 }  // namespace
 
 Engine::Engine(hipStream_t stream) : stream_(stream) {
-    std::vector<TabSet> host(kMaxModuli + 1);
-    make_tabsets(host.data());
+    // the tables and, behind them, the first block of stamps (zeros), in one allocation and one copy
+    constexpr size_t kTabs = (kMaxModuli + 1) * sizeof(TabSet), kStampsAt = (kTabs + 255) / 256 * 256;
+    std::vector<uint64_t> host((kStampsAt + kStampSlots0 * k::kStampWords * sizeof(uint64_t)) / sizeof(uint64_t), 0);
+    make_tabsets(reinterpret_cast<TabSet*>(host.data()));
+    const size_t bytes = host.size() * sizeof(uint64_t);
     void* p = nullptr;
-    hip_check(hipMalloc(&p, host.size() * sizeof(TabSet)), "table allocation");
+    hip_check(hipMalloc(&p, bytes), "table allocation");
     dtabs_ = static_cast<TabSet*>(p);
-    const hipError_t e = hipMemcpy(dtabs_, host.data(), host.size() * sizeof(TabSet), hipMemcpyHostToDevice);
+    stamps_.push_back({reinterpret_cast<uint64_t*>(static_cast<std::byte*>(p) + kStampsAt), 0, kStampSlots0});
+    const hipError_t e = hipMemcpy(p, host.data(), bytes, hipMemcpyHostToDevice);
     if (e != hipSuccess) {
         (void)hipFree(dtabs_);
         hip_check(e, "table upload");
@@ -33,6 +37,8 @@ Engine::Engine(hipStream_t stream) : stream_(stream) {
     if (hipGetDevice(&dev) == hipSuccess) {
         dev_ = dev;
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0) cus_ = cus;
+        int khz = 0;  // rate of the clock that the kernels stamp
+        if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) == hipSuccess && khz > 0) clock_khz_ = khz;
     }
     if (hipEventCreateWithFlags(&switch_ev_, hipEventDisableTiming) != hipSuccess) {
         (void)hipFree(dtabs_);
@@ -51,7 +57,7 @@ Engine::~Engine() {
     if (aux_) (void)hipStreamSynchronize(aux_);
     release_workspace();
     if (aux_) (void)hipStreamDestroy(aux_);
-    for (auto e : events_) (void)hipEventDestroy(e);
+    for (size_t i = 1; i < stamps_.size(); ++i) (void)hipFree(stamps_[i].p);
     for (auto e : sync_events_) (void)hipEventDestroy(e);
     if (switch_ev_) (void)hipEventDestroy(switch_ev_);
     if (dtabs_) (void)hipFree(dtabs_);
@@ -100,24 +106,36 @@ const Plan& Engine::plan_for(int s, int64_t k) {
     return plan_;
 }
 
-hipEvent_t Engine::timing_event(size_t idx) {
-    while (events_.size() <= idx) {
-        hipEvent_t e;
-        hip_check(hipEventCreate(&e), "event create");
-        events_.push_back(e);
+uint64_t* Engine::stamp_slot(size_t mark) {
+    for (const StampBlock& b : stamps_)
+        if (mark - b.first < b.slots) return b.p + (mark - b.first) * k::kStampWords;
+    // the end stamps are maxima: a block starts at zero (a copy from pageable memory has landed when it returns)
+    const std::vector<uint64_t> zero(k::kStampWords * kStampSlots, 0);
+    const size_t bytes = zero.size() * sizeof(uint64_t);
+    void* p = nullptr;
+    hip_check(hipMalloc(&p, bytes), "stage time allocation");
+    const hipError_t e = hipMemcpy(p, zero.data(), bytes, hipMemcpyHostToDevice);
+    if (e != hipSuccess) {
+        (void)hipFree(p);
+        hip_check(e, "stage time allocation");
     }
-    return events_[idx];
+    stamps_.push_back({static_cast<uint64_t*>(p), mark, kStampSlots});
+    return stamps_.back().p;
 }
 
-size_t Engine::stage_begin(Stage st, hipStream_t on) {
-    const size_t idx = 2 * marks_.size();
-    hip_check(hipEventRecord(timing_event(idx), on), "event record");
-    marks_.push_back(Mark{st, idx});
-    return marks_.size() - 1;
+bool Engine::capturing() const {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream_, &cap) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return cap == hipStreamCaptureStatusActive;
 }
 
-void Engine::stage_end(size_t mark, hipStream_t on) {
-    hip_check(hipEventRecord(timing_event(marks_[mark].ev + 1), on), "event record");
+uint64_t* Engine::StageTimer::next() {
+    uint64_t* ts = e.stamp_slot(e.marks_.size());
+    e.marks_.push_back(st);
+    return ts;
 }
 
 hipEvent_t Engine::sync_event() {
@@ -139,14 +157,26 @@ void Engine::order_after(hipStream_t to, hipStream_t from) {
 StageTimes Engine::stage_times() {
     StageTimes t;
     if (!profiling_ || marks_.empty()) return t;
-    for (const Mark& mk : marks_) {
-        (void)hipEventSynchronize(events_[mk.ev + 1]);
-        float ms = 0;
-        if (hipEventElapsedTime(&ms, events_[mk.ev], events_[mk.ev + 1]) != hipSuccess) {
+    // (a stream under capture cannot be waited for)
+    if (capturing() || hipStreamSynchronize(stream_) != hipSuccess) {
+        (void)hipGetLastError();
+        return t;
+    }
+    constexpr size_t kW = k::kStampWords;
+    std::vector<uint64_t> ts(marks_.size() * kW);
+    for (const StampBlock& b : stamps_) {
+        if (b.first >= marks_.size()) break;
+        const size_t n = std::min(b.slots, marks_.size() - b.first);
+        if (hipMemcpy(ts.data() + b.first * kW, b.p, n * kW * sizeof(uint64_t), hipMemcpyDeviceToHost) != hipSuccess) {
             (void)hipGetLastError();
-            ms = 0;
+            return t;
         }
-        switch (mk.st) {
+    }
+    for (size_t i = 0; i < marks_.size(); ++i) {
+        const uint64_t* w = ts.data() + i * kW;
+        const uint64_t b = w[0], e = *std::max_element(w + 1, w + kW);
+        const double ms = e > b ? static_cast<double>(e - b) / static_cast<double>(clock_khz_) : 0.0;
+        switch (marks_[i]) {
             case Stage::Scale: t.scale_ms += ms; break;
             case Stage::Split: t.split_ms += ms; break;
             case Stage::Gemm: t.gemm_ms += ms; break;
@@ -247,16 +277,11 @@ void Engine::gemm_fixed(std::byte* ws, size_t ws_bytes, Op ta, Op tb, int64_t m,
 void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, double ai, const double* A, int64_t lda,
                  const double* B, int64_t ldb, double br, double bi, double* C, int64_t ldc, int s, bool cplx,
                  std::byte* fixed_ws, size_t fixed_bytes) {
-    // a call into a fixed workspace creates nothing: no stage events either
-    // under stream capture: no timing events, and the panels are planned for the workspace as it
-    // is (it cannot grow there: that needs a synchronization and an allocation)
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream_, &cap) != hipSuccess) {
-        (void)hipGetLastError();
-        cap = hipStreamCaptureStatusNone;
-    }
-    const bool capturing = cap == hipStreamCaptureStatusActive;
-    const bool timed = profiling_ && !fixed_ws && !capturing;
+    // a call into a fixed workspace and one under stream capture are not timed; under capture the
+    // panels are planned for the workspace as it is (it cannot grow there: that needs a
+    // synchronization and an allocation)
+    const bool capture = capturing();
+    const bool timed = profiling_ && !fixed_ws && !capture;
     if (!accumulate_) marks_.clear();
     sync_used_ = 0;
     ++calls_;
@@ -285,7 +310,7 @@ void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, doubl
                                         std::to_string((need + (size_t{1} << 20) - 1) >> 20) + " MiB, it holds " +
                                         std::to_string(fixed_bytes >> 20) + " MiB");
     }
-    const size_t limit = fixed_ws ? fixed_bytes : capturing && ws_limit_ == 0 ? ws_size_ : budget();
+    const size_t limit = fixed_ws ? fixed_bytes : capture && ws_limit_ == 0 ? ws_size_ : budget();
     const TileInfo ti = plan_for_call(cs, limit);
     const int64_t mb = ti.mb, nb = ti.nb;
     const Layout L = layout(cs, mb, nb);
@@ -304,18 +329,13 @@ void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, doubl
     uint8_t* R = reinterpret_cast<uint8_t*>(ws + L.oR);
     const int64_t cw = cplx ? 2 : 1;  // doubles per element
 
-    // one stage's launches on stream `on`, bracketed by timing events when timed
+    // one stage's launches on stream `on`, stamped when timed
     auto timed_on = [&](Stage st, hipStream_t on, auto&& launch) {
-        if (!timed) {
-            launch();
-            return;
-        }
-        const size_t mk = stage_begin(st, on);
-        launch();
-        stage_end(mk, on);
+        StageTimer timer(*this, st);
+        launch(k::Stream(on, timed ? &timer : nullptr));
     };
     // split of `rows` rows of op(X) starting at row r0 into the planes from plane row prow
-    auto split_rows = [&](hipStream_t on, bool is_b, int64_t r0, int64_t rows, int64_t prow) {
+    auto split_rows = [&](const k::Stream& on, bool is_b, int64_t r0, int64_t rows, int64_t prow) {
         const Op op = is_b ? tb : ta;
         const double* X = is_b ? B : A;
         const int64_t ldx = is_b ? ldb : lda;
@@ -339,7 +359,7 @@ void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, doubl
         k::split(on, sp);
     };
     // INT8 GEMMs of `rows` rows of the A panel by columns c0 .. c0 + cols of the B panel
-    auto gemm_block = [&](hipStream_t on, int64_t rows, int64_t c0, int64_t cols) {
+    auto gemm_block = [&](const k::Stream& on, int64_t rows, int64_t c0, int64_t cols) {
         k::GemmArgs ga{};
         ga.A = Ap;
         ga.B = Bp + c0 * kp;
@@ -374,7 +394,7 @@ void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, doubl
         }
     };
     // CRT + alpha/beta epilogue of rows i0 .. i0 + rows by panel columns c0 .. c0 + cols of panel j0
-    auto crt_block = [&](hipStream_t on, int64_t i0, int64_t rows, int64_t j0, int64_t c0, int64_t cols) {
+    auto crt_block = [&](const k::Stream& on, int64_t i0, int64_t rows, int64_t j0, int64_t c0, int64_t cols) {
         k::CrtArgs ca{};
         ca.R = R + c0 * L.mpad;
         ca.plane_r = L.planeR;
@@ -399,9 +419,9 @@ void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, doubl
     };
 
     // scale: exponents of the rows of op(A) and the columns of op(B) (hpp:974-989)
-    timed_on(Stage::Scale, stream_, [&] {
-        k::scale(stream_, A, lda, m, k, ta != Op::N, cplx, tk, PA, D);
-        k::scale(stream_, B, ldb, n, k, tb == Op::N, cplx, tk, PB, E);
+    timed_on(Stage::Scale, stream_, [&](const k::Stream& on) {
+        k::scale(on, A, lda, m, k, ta != Op::N, cplx, tk, PA, D);
+        k::scale(on, B, ldb, n, k, tb == Op::N, cplx, tk, PB, E);
     });
     // Column blocks of a panel pair: with more than one, the B blocks are split and the CRTs run on
     // the second stream while the GEMM of the next block runs on the caller's (a fixed workspace
@@ -412,13 +432,13 @@ void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, doubl
         const int64_t nbj = std::min(nb, n - j0);
         const int64_t wb = nblocks > 1 ? round_up((nbj + nblocks - 1) / nblocks, L.TN) : nbj;
         const int64_t nblk = (nbj + wb - 1) / wb;
-        if (nblk == 1) timed_on(Stage::Split, stream_, [&] { split_rows(stream_, true, j0, nbj, 0); });
+        if (nblk == 1) timed_on(Stage::Split, stream_, [&](const k::Stream& on) { split_rows(on, true, j0, nbj, 0); });
         for (int64_t i0 = 0; i0 < m; i0 += mb) {
             const int64_t mbi = std::min(mb, m - i0);
-            if (ti.pm > 1 || j0 == 0) timed_on(Stage::Split, stream_, [&] { split_rows(stream_, false, i0, mbi, 0); });
+            if (ti.pm > 1 || j0 == 0) timed_on(Stage::Split, stream_, [&](const k::Stream& on) { split_rows(on, false, i0, mbi, 0); });
             if (nblk == 1) {
-                timed_on(Stage::Gemm, stream_, [&] { gemm_block(stream_, mbi, 0, nbj); });
-                timed_on(Stage::Crt, stream_, [&] { crt_block(stream_, i0, mbi, j0, 0, nbj); });
+                timed_on(Stage::Gemm, stream_, [&](const k::Stream& on) { gemm_block(on, mbi, 0, nbj); });
+                timed_on(Stage::Crt, stream_, [&](const k::Stream& on) { crt_block(on, i0, mbi, j0, 0, nbj); });
                 continue;
             }
             if (!forked) {  // the second stream starts after everything before it on the caller's
@@ -429,21 +449,21 @@ void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, doubl
             if (i0 == 0)  // the B panel's blocks, once per panel column, ahead of the CRTs
                 for (int64_t c = 0; c < nblk; ++c) {
                     const int64_t c0 = c * wb, cols = std::min(wb, nbj - c0);
-                    timed_on(Stage::Split, aux_, [&] { split_rows(aux_, true, j0 + c0, cols, c0); });
+                    timed_on(Stage::Split, aux_, [&](const k::Stream& on) { split_rows(on, true, j0 + c0, cols, c0); });
                     split_done[c] = sync_event();
                     hip_check(hipEventRecord(split_done[c], aux_), "event record");
                 }
             for (int64_t c = 0; c < nblk; ++c) {
                 const int64_t c0 = c * wb, cols = std::min(wb, nbj - c0);
                 if (i0 == 0) hip_check(hipStreamWaitEvent(stream_, split_done[c], 0), "stream wait");
-                timed_on(Stage::Gemm, stream_, [&] { gemm_block(stream_, mbi, c0, cols); });
+                timed_on(Stage::Gemm, stream_, [&](const k::Stream& on) { gemm_block(on, mbi, c0, cols); });
                 gemm_done[c] = sync_event();
                 hip_check(hipEventRecord(gemm_done[c], stream_), "event record");
             }
             for (int64_t c = 0; c < nblk; ++c) {
                 const int64_t c0 = c * wb, cols = std::min(wb, nbj - c0);
                 hip_check(hipStreamWaitEvent(aux_, gemm_done[c], 0), "stream wait");
-                timed_on(Stage::Crt, aux_, [&] { crt_block(aux_, i0, mbi, j0, c0, cols); });
+                timed_on(Stage::Crt, aux_, [&](const k::Stream& on) { crt_block(on, i0, mbi, j0, c0, cols); });
             }
             // the next panel pair rewrites the residues the CRTs read, and its B split the planes
             // the GEMMs read (the GEMMs are done once the CRTs are: each waited for its GEMM)

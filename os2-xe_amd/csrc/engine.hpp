@@ -89,16 +89,18 @@ public:
 
 private:
     enum class Stage { Scale, Split, Gemm, Crt };
-    struct Mark {
+    // hands every launch of one stage its own stamps
+    struct StageTimer final : k::LaunchTimer {
+        Engine& e;
         Stage st;
-        size_t ev;  // events_[ev], events_[ev + 1]: begin and end on the stream the stage ran on
+        StageTimer(Engine& eng, Stage stage) : e(eng), st(stage) {}
+        uint64_t* next() override;
     };
     void run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, double ai, const double* A, int64_t lda,
              const double* B, int64_t ldb, double br, double bi, double* C, int64_t ldc, int s, bool cplx,
              std::byte* fixed_ws, size_t fixed_bytes);
-    hipEvent_t timing_event(size_t idx);
-    size_t stage_begin(Stage st, hipStream_t on);
-    void stage_end(size_t mark, hipStream_t on);
+    uint64_t* stamp_slot(size_t mark);
+    bool capturing() const;
     hipEvent_t sync_event();  // from a pool reused by every call (a wait binds the record before it)
     void order_after(hipStream_t to, hipStream_t from);
     int overlap_blocks() const;  // column blocks per panel pair (Tuning::overlap_blocks; automatic: 1)
@@ -126,8 +128,16 @@ private:
     TileInfo memo_ti_{};
     k::Tile tile_ = k::Tile::T256;
     hipStream_t aux_ = nullptr;  // second stream of the column-block overlap
-    std::vector<hipEvent_t> events_;        // timing events
-    std::vector<Mark> marks_;
+    // stamps of the timed launches, kStampWords words each, in device blocks: the first behind the tables
+    // (enough for any call of a few panels), more when many panels or profile_begin() need them
+    static constexpr size_t kStampSlots0 = 256, kStampSlots = 4096;
+    struct StampBlock {
+        uint64_t* p;
+        size_t first, slots;  // stamps of marks first .. first + slots - 1
+    };
+    std::vector<StampBlock> stamps_;
+    int64_t clock_khz_ = 100000;
+    std::vector<Stage> marks_;              // stage of every timed launch; mark i has entry i of stamps_
     std::vector<hipEvent_t> sync_events_;   // ordering events between the two streams
     size_t sync_used_ = 0;
     bool accumulate_ = false;

@@ -299,12 +299,14 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint32_t plane, uin
 }
 
 template <int BM, int BN, int MINB, int NS>
-__global__ void __launch_bounds__(256, MINB) igemm_residue_kernel(GemmArgs p) {
+__global__ void __launch_bounds__(256, MINB) igemm_residue_kernel(GemmArgs p, uint64_t* ts) {
     __shared__ v4i smem[TileShape<BM, BN, NS>::SMEM / 16];
+    const Stamp st(ts);
     uint32_t plane, tm, tn;
     const uint32_t tiles = static_cast<uint32_t>(p.tiles_m) * static_cast<uint32_t>(p.tiles_n);
     tile_coords(p, plane_xcd_remap(blockIdx.x, tiles, gridDim.x), plane, tm, tn);
     gemm_tile<BM, BN, NS>(p, plane, tm, tn, smem);
+    st.end();
 }
 
 template <int BM, int BN, int MINB, int NS>
@@ -468,11 +470,11 @@ void igemm_int32(hipStream_t st, Tile tile, const GemmArgs& a) {
 #undef OZ2_LAUNCH
 }
 
-void igemm_residue(hipStream_t st, Tile tile, const GemmArgs& a) {
+void igemm_residue(const Stream& st, Tile tile, const GemmArgs& a) {
     const uint32_t nblk = static_cast<uint32_t>(a.tiles_m) * a.tiles_n * a.nplanes;
     if (nblk == 0 || a.klen <= 0) return;
 #define OZ2_LAUNCH(BM, BN, MINB, NS) \
-    hipLaunchKernelGGL((igemm_residue_kernel<BM, BN, MINB, NS>), dim3(nblk), dim3(256), 0, st, a)
+    launch(st, igemm_residue_kernel<BM, BN, MINB, NS>, dim3(nblk), dim3(256), a)
     switch (tile) {
         case Tile::T256: OZ2_LAUNCH(256, 256, 1, 4); break;
         case Tile::T128: OZ2_LAUNCH(128, 128, 2, 4); break;

@@ -19,6 +19,51 @@
 namespace oz2 {
 namespace k {
 
+// Source of a timed launch's stamps (stage times): kStampWords device words of its own.
+inline constexpr uint32_t kStampWords = 16;
+struct LaunchTimer {
+    virtual uint64_t* next() = 0;
+
+protected:
+    ~LaunchTimer() = default;
+};
+
+// Where a launch goes: a stream and, for timed calls, the timer of its stage.  The kernel stamps the
+// GPU's constant-rate clock itself (Stamp below).  Events recorded around the launches are barrier
+// packets of their own, about 10 us of idle GPU between any two stages (DGEMM 64^3 s = 16: 68 us a call
+// with them, 29 us with timing off; 1024^3 s = 14: 112 and 76 us), and events handed to the launch cost
+// 12 us of host time each; the stamps cost nothing that shows.
+struct Stream {
+    hipStream_t s;
+    LaunchTimer* timer = nullptr;
+    Stream(hipStream_t st, LaunchTimer* t = nullptr) : s(st), timer(t) {}
+};
+
+#if defined(__HIPCC__)
+// Begin of a kernel in ts[0], ends in the other words (ts null: not timed).  Workgroups start in order,
+// so the first one stamps the begin; the end is the latest of the last kStampWords - 1 workgroups, each
+// with a word of its own (one word for all of 256 workgroups, by atomicMax, cost 1.5 us a launch).  The
+// clock only grows, so words left by an earlier launch do not count.
+struct Stamp {
+    uint64_t* ts;
+    uint32_t b, n;
+    __device__ __forceinline__ explicit Stamp(uint64_t* t)
+        : ts(t), b(blockIdx.y * gridDim.x + blockIdx.x), n(gridDim.x * gridDim.y) {
+        if (ts && b == 0 && threadIdx.x == 0) ts[0] = wall_clock64();
+    }
+    __device__ __forceinline__ void end() const {
+        if (ts && n - b < kStampWords && threadIdx.x == 0) ts[n - b] = wall_clock64();
+    }
+};
+
+// kernels launched this way take the stamps as their last parameter
+template <typename... P, typename... A>
+void launch(const Stream& st, void (*kernel)(P...), dim3 grid, dim3 block, A&&... args) {
+    uint64_t* ts = st.timer ? st.timer->next() : nullptr;
+    hipLaunchKernelGGL(kernel, grid, block, 0, st.s, args..., ts);
+}
+#endif
+
 // Byte offset of element (row r, k p) inside one operand plane with kp columns:
 // 16-row bands of kp/64 consecutive 1 KB blocks; inside a block, 64 bytes per row
 // as four 16-byte chunks.  Byte b of chunk c holds k = block_k(c, b) of the block:
@@ -43,7 +88,7 @@ __host__ __device__ inline int64_t plane_offset(int64_t r, int64_t p, int64_t kp
 // Complex data (interleaved re, im) scales by the max over both parts.
 // `partial` needs partial_elems(len, k) u64 entries when !kcontig.
 size_t scale_partial_elems(int64_t len, int64_t k, bool kcontig);
-void scale(hipStream_t st, const double* X, int64_t ldx, int64_t len, int64_t k, bool kcontig, bool cplx, int tk,
+void scale(const Stream& st, const double* X, int64_t ldx, int64_t len, int64_t k, bool kcontig, bool cplx, int tk,
            uint64_t* partial, int32_t* ex);
 
 // ---- split -------------------------------------------------------------------
@@ -63,7 +108,7 @@ struct SplitArgs {
     int form;             // limb_form(tk): octets of the offset value 8, 12 or 14
     const TabSet* tab;    // device tables of this s
 };
-void split(hipStream_t st, const SplitArgs& a);
+void split(const Stream& st, const SplitArgs& a);
 
 // ---- INT8 GEMM with residue epilogue ------------------------------------------
 struct GemmArgs {
@@ -82,7 +127,7 @@ struct GemmArgs {
     int64_t kb_extra;     // op(B) reads k range k0 + kb_extra .. (0 for Scheme II)
     int32_t* R32;         // igemm_int32: sums [nplanes][npad_c][ldr] as int32 (R unused)
 };
-void igemm_residue(hipStream_t st, Tile tile, const GemmArgs& a);
+void igemm_residue(const Stream& st, Tile tile, const GemmArgs& a);
 // the same GEMM with the int32 sums stored as they are (|sums| < 2^31 is the caller's to keep):
 // the digit products of Ozaki Scheme I
 void igemm_int32(hipStream_t st, Tile tile, const GemmArgs& a);
@@ -104,7 +149,7 @@ struct CrtArgs {
     int s, L16;
     const TabSet* tab;    // device tables of this s
 };
-void crt(hipStream_t st, const CrtArgs& a);
+void crt(const Stream& st, const CrtArgs& a);
 
 // ---- Ozaki Scheme I (the accuracy benchmark's comparison baseline) --------------------
 // L balanced base-128 digits of RNE(op(X)[r][p] 2^ex[r]) per element into one extended

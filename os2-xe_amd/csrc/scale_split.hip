@@ -166,11 +166,21 @@ __device__ __forceinline__ void scale_finalize_body(const ScaleFinItem& it, uint
     it.ex[r] = exponent_from_maxbits(mx, it.tk);
 }
 
-__global__ void __launch_bounds__(256) scale_kcontig_kernel(ScaleKcItem it) { scale_kcontig_body(it, blockIdx.x); }
-__global__ void __launch_bounds__(256) scale_kstrided_kernel(ScaleKsItem it) {
-    scale_kstrided_body(it, blockIdx.x, blockIdx.y);
+__global__ void __launch_bounds__(256) scale_kcontig_kernel(ScaleKcItem it, uint64_t* ts) {
+    const Stamp st(ts);
+    scale_kcontig_body(it, blockIdx.x);
+    st.end();
 }
-__global__ void __launch_bounds__(256) scale_finalize_kernel(ScaleFinItem it) { scale_finalize_body(it, blockIdx.x); }
+__global__ void __launch_bounds__(256) scale_kstrided_kernel(ScaleKsItem it, uint64_t* ts) {
+    const Stamp st(ts);
+    scale_kstrided_body(it, blockIdx.x, blockIdx.y);
+    st.end();
+}
+__global__ void __launch_bounds__(256) scale_finalize_kernel(ScaleFinItem it, uint64_t* ts) {
+    const Stamp st(ts);
+    scale_finalize_body(it, blockIdx.x);
+    st.end();
+}
 
 constexpr int64_t kScaleRowsPerBlock = 64;
 
@@ -386,7 +396,11 @@ __device__ __forceinline__ void split_body(const SplitItem& it, uint32_t bx, uin
     else split_real_body<FM, KC, split_q(FM, false)>(it.a, it.lg, bx, by);
 }
 template <int V>
-__global__ void __launch_bounds__(256) split_kernel(SplitItem it) { split_body<V>(it, blockIdx.x, blockIdx.y); }
+__global__ void __launch_bounds__(256) split_kernel(SplitItem it, uint64_t* ts) {
+    const Stamp st(ts);
+    split_body<V>(it, blockIdx.x, blockIdx.y);
+    st.end();
+}
 
 int split_variant(const SplitArgs& a) {
     return a.form | (a.kcontig ? 4 : 0) | (a.cplx ? 8 : 0) | (a.cplx && a.conj ? 16 : 0);
@@ -418,8 +432,8 @@ SplitItem split_item(const SplitArgs& a, uint32_t& gy) {
 }
 
 template <int V>
-void launch_split_v(hipStream_t st, const SplitItem& it, uint32_t gy) {
-    hipLaunchKernelGGL((split_kernel<V>), dim3(it.gx, gy), dim3(256), 0, st, it);
+void launch_split_v(const Stream& st, const SplitItem& it, uint32_t gy) {
+    launch(st, split_kernel<V>, dim3(it.gx, gy), dim3(256), it);
 }
 
 // ---- grouped forms: block b of the launch runs block (b - start[p]) of item p
@@ -452,24 +466,24 @@ size_t scale_partial_elems(int64_t len, int64_t k, bool kcontig) {
     return static_cast<size_t>(scale_kblocks(len, k)) * static_cast<size_t>(len);
 }
 
-void scale(hipStream_t st, const double* X, int64_t ldx, int64_t len, int64_t k, bool kcontig, bool cplx, int tk,
+void scale(const Stream& st, const double* X, int64_t ldx, int64_t len, int64_t k, bool kcontig, bool cplx, int tk,
            uint64_t* partial, int32_t* ex) {
     if (len <= 0) return;
     if (kcontig) {
         const ScaleKcItem it{X, ldx, len, cplx ? 2 * k : k, cplx ? 1 : 0, tk, ex, static_cast<uint32_t>((len + 3) / 4)};
-        hipLaunchKernelGGL(scale_kcontig_kernel, dim3(it.gx), dim3(256), 0, st, it);
+        launch(st, scale_kcontig_kernel, dim3(it.gx), dim3(256), it);
     } else {
         const int64_t nkb = scale_kblocks(len, k);
         const int64_t kper = (k + nkb - 1) / nkb;
         const ScaleKsItem it{X, ldx, len, k, kper, cplx ? 1 : 0, partial,
                              static_cast<uint32_t>((len + kScaleRowsPerBlock - 1) / kScaleRowsPerBlock)};
-        hipLaunchKernelGGL(scale_kstrided_kernel, dim3(it.gx, static_cast<unsigned>(nkb)), dim3(256), 0, st, it);
+        launch(st, scale_kstrided_kernel, dim3(it.gx, static_cast<unsigned>(nkb)), dim3(256), it);
         const ScaleFinItem fin{partial, len, static_cast<int>(nkb), tk, ex, static_cast<uint32_t>((len + 255) / 256)};
-        hipLaunchKernelGGL(scale_finalize_kernel, dim3(fin.gx), dim3(256), 0, st, fin);
+        launch(st, scale_finalize_kernel, dim3(fin.gx), dim3(256), fin);
     }
 }
 
-void split(hipStream_t st, const SplitArgs& a) {
+void split(const Stream& st, const SplitArgs& a) {
     uint32_t gy = 0;
     const SplitItem it = split_item(a, gy);
     switch (split_variant(a)) {
