@@ -1,16 +1,20 @@
 // crt.hip - CRT reconstruction fused with the alpha/beta epilogue, for gfx950.
 //
+// Bounds: HBM up to s = 16 (s + 8 or 16 bytes an entry; 5.2 TB/s at 8192 x 8192 s = 16, the rate of a plain
+// copy), the VALU above (3.6 TB/s at s = 24).
+//
 // Reference behaviour: src/ozaki2_gpu.hpp:526-664.  For each entry the s
 // residues r_t (bytes from the GEMM epilogue; k-chunks are summed mod m_t)
 // determine the exact integer C' with |C'| <= M/4:
 //   q  = round(sum_t r_t F_t / 2^16)            (F_t = round(2^16 y_t / m_t); error < 0.05, so q is exact)
-//   C' = sum_t r_t W_t - q M                     (16-bit limbs, 32-bit sums)
+//   C' = sum_t r_t W_t - q M                     (limb sums of crt_tile.hpp or 16-bit dot products)
 // C' is rounded once to 53 bits (sticky bit) and scaled by 2^-(D_i + E_j),
 // which rounds again only for subnormal results, as in the reference.
 // Rows / columns with a non-finite exponent give NaN.  The epilogue is
 // C = alpha*v (beta == 0, C not read) or fma(alpha, v, beta*C); complex:
 // Re = P0 - P1, Im = P2 - P0 - P1 in residue space (3M form), then
 // (ar*vr - ai*vi, ar*vi + ai*vr) + beta*C, each product pair fused as one fma.
+#include "crt_tile.hpp"
 #include "grouped.hpp"
 #include "kernels.hpp"
 #include "math.hpp"
@@ -21,163 +25,173 @@ using namespace math;
 
 namespace {
 
-// residue r_t of one entry, summing k-chunks mod m_t
-__device__ __forceinline__ uint32_t chunk_sum(uint32_t s, uint32_t m) {
-    // s < kch * 256; reduce by repeated folding (kch is small)
-    while (s >= m) s -= m;
-    return s;
+// Residue words (4 entries) of SC moduli summed over the k-chunks mod m_t: all words of a chunk are
+// loaded before they are added, as bytes 0, 2 and bytes 1, 3 in 16-bit halves.
+template <int SC>
+__device__ __forceinline__ void chunk_words(const uint8_t* base, const CrtArgs& a, ConstTab tb,
+                                            uint32_t (&r)[SC]) {
+    uint32_t even[SC] = {}, odd[SC] = {};
+    auto reduce = [&](uint32_t x, int t) {  // both halves mod m_t
+        const uint32_t m = tb->m[t], mu = tb->mu[t];
+        return m == 256 ? x & 0x00FF00FFu : mod_m23(x & 0xFFFFu, m, mu) | mod_m23(x >> 16, m, mu) << 16;
+    };
+    for (int c = 0; c < a.kch; ++c) {
+        uint32_t w[SC];
+#pragma unroll
+        for (int t = 0; t < SC; ++t)
+            w[t] = t < a.s ? *reinterpret_cast<const uint32_t*>(base + c * a.chunk_r + t * a.plane_r) : 0u;
+#pragma unroll
+        for (int t = 0; t < SC; ++t) {
+            even[t] += w[t] & 0x00FF00FFu;
+            odd[t] += (w[t] >> 8) & 0x00FF00FFu;
+        }
+        if ((c & 127) == 127) {  // sums stay below 256 + 128 * 255 < 2^16
+#pragma unroll
+            for (int t = 0; t < SC; ++t)
+                if (t < a.s) {
+                    even[t] = reduce(even[t], t);
+                    odd[t] = reduce(odd[t], t);
+                }
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < SC; ++t) r[t] = t < a.s ? reduce(even[t], t) | reduce(odd[t], t) << 8 : 0u;
 }
 
-// 4 consecutive rows per thread; residues are bytes packed 4 per 32-bit load.
-template <int NL, bool CPLX>
+// 3M residues of modulus m: Re = P0 - P1 and Im = P2 - P0 - P1, reduced into [0, m)
+__device__ __forceinline__ void from_3m(uint32_t w0, uint32_t w1, uint32_t w2, uint32_t m, uint32_t& re, uint32_t& im) {
+    uint32_t xr[4], xi[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const uint32_t x0 = (w0 >> (8 * e)) & 0xFFu, x1 = (w1 >> (8 * e)) & 0xFFu, x2 = (w2 >> (8 * e)) & 0xFFu;
+        uint32_t r = x0 + m - x1;  // [0, 2m)
+        xr[e] = r >= m ? r - m : r;
+        r = x2 + 2 * m - x0 - x1;  // [0, 3m)
+        r = r >= m ? r - m : r;
+        xi[e] = r >= m ? r - m : r;
+    }
+    re = pack_lo_bytes(xr[0], xr[1], xr[2], xr[3]);
+    im = pack_lo_bytes(xi[0], xi[1], xi[2], xi[3]);
+}
+
+// Matrix cores or dot products for the limb and quotient sums.  With few moduli the kernel is bound by its
+// loads, and the dot products' registers (44 to 68, against 87 to 100) keep more waves in flight; with many
+// it is bound by the sums.  Measured on MI355X, beta != 0, matrix / dot products, us: 4096 x 4096
+// s = 8 72 / 62, s = 16 124 / 109, s = 20 131 / 160, s = 24 150 / 192; 8192 x 8192 s = 16 459 / 414
+// (5.2 TB/s); complex 4096 x 4096 s = 16 324 / 357, s = 24 430 / 489.
+constexpr bool crt_matrix(int nl, bool cplx) { return cplx ? nl >= 4 : nl >= 5; }
+
+template <int NL, bool MAT>
+struct CrtSums : CrtTile<NL> {
+    using CrtTile<NL>::CrtTile;
+};
+template <int NL>
+struct CrtSums<NL, false> {
+    ConstTab tb;
+    __device__ __forceinline__ explicit CrtSums(const TabSet* tab) : tb(const_tab(tab)) {}
+    template <typename Out>
+    __device__ __forceinline__ void four(const uint32_t (&r)[4 * NL], const Out& out) const {
+        CrtAcc<NL> acc[4];
+#pragma unroll
+        for (int t = 0; t < 4 * NL; t += 2) {
+            if (t >= tb->s) break;  // (also keeps the tables' scalar loads apart: together they spill)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[e].add2(tb, t >> 1, (r[t] >> (8 * e)) & 0xFFu, (r[t + 1] >> (8 * e)) & 0xFFu);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            uint32_t w[NL];
+            acc[e].words(tb, w);
+            out(e, w);
+        }
+    }
+};
+
+// 4 consecutive rows per thread; residues are bytes packed 4 per 32-bit load.  CHUNKS: k-chunks to sum.
+template <int NL, bool CPLX, bool CHUNKS>
 __device__ __forceinline__ void crt_body(const CrtArgs& a, uint32_t bx) {
+    constexpr int SC = 4 * NL;
     const auto tb = const_tab(a.tab);
-    const int64_t mq = (a.mb + 3) >> 2;
-    const int64_t idx = static_cast<int64_t>(bx) * 256 + threadIdx.x;
-    const int64_t j = idx / mq;
-    const int64_t i0 = (idx - j * mq) * 4;
-    if (j >= a.nb) return;
+    const CrtSums<NL, crt_matrix(NL, CPLX)> sums(a.tab);
+    // row quads of a column; the block's first quad by one uniform division, the lane's from there in
+    // 32 bits (a 64-bit division per lane is about as long as the reconstruction of an entry)
+    const uint32_t mq = static_cast<uint32_t>((a.mb + 3) >> 2);
+    const uint64_t first = static_cast<uint64_t>(bx) * 256;
+    const int64_t jb = static_cast<int64_t>(first / mq);
+    const uint32_t in = static_cast<uint32_t>(first - static_cast<uint64_t>(jb) * mq) + threadIdx.x;
+    const uint32_t dj = in / mq;
+    // every lane takes part in the matrix products: the ones past the end repeat the last column's start
+    const bool ok = jb + dj < a.nb;
+    const int64_t j = ok ? jb + dj : a.nb - 1;
+    const int64_t i0 = ok ? static_cast<int64_t>(in - dj * mq) * 4 : 0;
     const int32_t Ej = a.E[j];
     const uint8_t* base = a.R + j * a.ldr + i0;
     const int s = a.s;
+    const int64_t gs = static_cast<int64_t>(s) * a.plane_r;
 
-    CrtAcc<NL> re[4];
-    CrtAcc<NL> im[4];
+    uint32_t re[SC], im[CPLX ? SC : 1];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        re[e].init();
-        if (CPLX) im[e].init();
+    for (int t = 0; t < SC; ++t) {
+        re[t] = 0;
+        if (CPLX) im[t] = 0;
     }
-    if (!CPLX && a.kch == 1) {
-        // one k-chunk: the s residue words (4 entries each) are all loaded before any
-        // arithmetic, then summed in modulus pairs (2 residues per dot2 step); r = 0 past s
-        uint32_t w[kMaxModuli];
+    if (!CPLX && !CHUNKS) {
+        // all s residue words are loaded before any arithmetic
 #pragma unroll
-        for (int t = 0; t < kMaxModuli; ++t)
-            w[t] = t < s ? *reinterpret_cast<const uint32_t*>(base + t * a.plane_r) : 0u;
-#pragma unroll
-        for (int t = 0; t < kMaxModuli; t += 2) {
-            if (t < s) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    re[e].add2(tb, t >> 1, (w[t] >> (8 * e)) & 0xFFu, (w[t + 1] >> (8 * e)) & 0xFFu);
-            }
-        }
-    }
-    if (CPLX && a.kch == 1) {
-        // the same for the three 3M groups, in two halves of the moduli to bound the
-        // words held at once; Re = P0 - P1 and Im = P2 - P0 - P1 reduced into [0, m)
-        const int64_t gs = static_cast<int64_t>(s) * a.plane_r;
+        for (int t = 0; t < SC; ++t)
+            if (t < s) re[t] = *reinterpret_cast<const uint32_t*>(base + t * a.plane_r);
+    } else if (!CPLX) {
+        chunk_words<SC>(base, a, tb, re);
+    } else if (!CHUNKS) {
+        // the same for the three 3M groups, in two halves of the moduli to bound the words held at once
 #pragma unroll
         for (int half = 0; half < 2; ++half) {
-            constexpr int H = kMaxModuli / 2;
-            const int t0 = half * H;
-            if (t0 >= s) break;
+            constexpr int H = SC / 2;
             uint32_t w0[H], w1[H], w2[H];
 #pragma unroll
             for (int u = 0; u < H; ++u) {
-                const uint8_t* b = base + (t0 + u) * a.plane_r;
-                const bool in = t0 + u < s;
-                w0[u] = in ? *reinterpret_cast<const uint32_t*>(b) : 0u;
-                w1[u] = in ? *reinterpret_cast<const uint32_t*>(b + gs) : 0u;
-                w2[u] = in ? *reinterpret_cast<const uint32_t*>(b + 2 * gs) : 0u;
+                const int t = half * H + u;
+                const uint8_t* b = base + t * a.plane_r;
+                w0[u] = t < s ? *reinterpret_cast<const uint32_t*>(b) : 0u;
+                w1[u] = t < s ? *reinterpret_cast<const uint32_t*>(b + gs) : 0u;
+                w2[u] = t < s ? *reinterpret_cast<const uint32_t*>(b + 2 * gs) : 0u;
             }
 #pragma unroll
-            for (int u = 0; u < H; u += 2) {
-                if (t0 + u < s) {
-                    const uint32_t m[2] = {tb->m[t0 + u], tb->m[t0 + u + 1]};  // 0 past s (residues 0 there)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        uint32_t xr[2], xi[2];
-#pragma unroll
-                        for (int h = 0; h < 2; ++h) {
-                            const uint32_t x0 = (w0[u + h] >> (8 * e)) & 0xFFu;
-                            const uint32_t x1 = (w1[u + h] >> (8 * e)) & 0xFFu;
-                            const uint32_t x2 = (w2[u + h] >> (8 * e)) & 0xFFu;
-                            uint32_t r = x0 + m[h] - x1;  // [0, 2m)
-                            xr[h] = r >= m[h] ? r - m[h] : r;
-                            r = x2 + 2 * m[h] - x0 - x1;  // [0, 3m)
-                            r = r >= m[h] ? r - m[h] : r;
-                            xi[h] = r >= m[h] ? r - m[h] : r;
-                        }
-                        re[e].add2(tb, (t0 + u) >> 1, xr[0], xr[1]);
-                        im[e].add2(tb, (t0 + u) >> 1, xi[0], xi[1]);
-                    }
-                }
+            for (int u = 0; u < H; ++u) {
+                const int t = half * H + u;
+                if (t < s) from_3m(w0[u], w1[u], w2[u], tb->m[t], re[t], im[CPLX ? t : 0]);
             }
         }
+    } else {
+        uint32_t w[3][SC];
+#pragma unroll
+        for (int g = 0; g < 3; ++g) chunk_words<SC>(base + g * gs, a, tb, w[g]);
+#pragma unroll
+        for (int t = 0; t < SC; ++t)
+            if (t < s) from_3m(w[0][t], w[1][t], w[2][t], tb->m[t], re[t], im[CPLX ? t : 0]);
     }
-    // moduli in pairs (2 residues per dot2 step of the limb sums); r = 0 past s
-    for (int t = 0; t < s && a.kch > 1; t += 2) {
-        const bool two = t + 1 < s;
-        const uint32_t m0 = tb->m[t], m1 = two ? tb->m[t + 1] : 1u;
-        if (!CPLX) {
-            uint32_t r0[4] = {0, 0, 0, 0}, r1[4] = {0, 0, 0, 0};
-            for (int c = 0; c < a.kch; ++c) {
-                const uint8_t* b = base + c * a.chunk_r + t * a.plane_r;
-                const uint32_t w0 = *reinterpret_cast<const uint32_t*>(b);
-                const uint32_t w1 = two ? *reinterpret_cast<const uint32_t*>(b + a.plane_r) : 0u;
+
+    int32_t shift[4];
+    bool nonfinite[4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    r0[e] += (w0 >> (8 * e)) & 0xFFu;
-                    r1[e] += (w1 >> (8 * e)) & 0xFFu;
-                }
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const uint32_t x0 = a.kch > 1 ? chunk_sum(r0[e], m0) : r0[e];
-                const uint32_t x1 = a.kch > 1 ? chunk_sum(r1[e], m1) : r1[e];
-                re[e].add2(tb, t >> 1, x0, x1);
-            }
-        } else {
-            uint32_t p0[2][4] = {}, p1[2][4] = {}, p2[2][4] = {};
-            const int64_t gs = static_cast<int64_t>(s) * a.plane_r;
-            for (int c = 0; c < a.kch; ++c) {
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    if (h == 1 && !two) break;
-                    const uint8_t* b = base + c * a.chunk_r + (t + h) * a.plane_r;
-                    const uint32_t w0 = *reinterpret_cast<const uint32_t*>(b);
-                    const uint32_t w1 = *reinterpret_cast<const uint32_t*>(b + gs);
-                    const uint32_t w2 = *reinterpret_cast<const uint32_t*>(b + 2 * gs);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        p0[h][e] += (w0 >> (8 * e)) & 0xFFu;
-                        p1[h][e] += (w1 >> (8 * e)) & 0xFFu;
-                        p2[h][e] += (w2 >> (8 * e)) & 0xFFu;
-                    }
-                }
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                uint32_t xr[2] = {0, 0}, xi[2] = {0, 0};
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    if (h == 1 && !two) break;
-                    const uint32_t m = h ? m1 : m0;
-                    const uint32_t x0 = a.kch > 1 ? chunk_sum(p0[h][e], m) : p0[h][e];
-                    const uint32_t x1 = a.kch > 1 ? chunk_sum(p1[h][e], m) : p1[h][e];
-                    const uint32_t x2 = a.kch > 1 ? chunk_sum(p2[h][e], m) : p2[h][e];
-                    xr[h] = chunk_sum(x0 + m - x1, m);           // Re = P0 - P1
-                    xi[h] = chunk_sum(x2 + 2 * m - x0 - x1, m);  // Im = P2 - P0 - P1
-                }
-                re[e].add2(tb, t >> 1, xr[0], xr[1]);
-                im[e].add2(tb, t >> 1, xi[0], xi[1]);
-            }
-        }
+    for (int e = 0; e < 4; ++e) {
+        const int32_t Di = a.D[min(i0 + e, a.mb - 1)];
+        nonfinite[e] = Di == INT32_MIN || Ej == INT32_MIN;
+        shift[e] = nonfinite[e] ? 0 : Di + Ej;
     }
-    if (!CPLX && i0 + 4 <= a.mb) {
-        // four entries of one column: 16-byte accesses to C when it is aligned for them
-        double v[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int32_t Di = a.D[i0 + e];
-            const bool nonfinite = Di == INT32_MIN || Ej == INT32_MIN;
-            v[e] = re[e].finish(tb, nonfinite ? 0 : Di + Ej);
-            if (nonfinite) v[e] = __builtin_nan("");
-        }
+    double v[4], vi[4];
+    sums.four(re, [&](int e, const uint32_t (&w)[NL]) {
+        v[e] = nonfinite[e] ? __builtin_nan("") : crt_round<NL>(w, shift[e]);
+    });
+    if constexpr (CPLX)
+        sums.four(im, [&](int e, const uint32_t (&w)[NL]) {
+            vi[e] = nonfinite[e] ? __builtin_nan("") : crt_round<NL>(w, shift[e]);
+        });
+    if (!ok) return;
+    if constexpr (!CPLX) {
         double* cp = a.C + i0 + j * a.ldc;
-        if ((reinterpret_cast<uintptr_t>(cp) & 15) == 0) {
+        if (i0 + 4 <= a.mb && (reinterpret_cast<uintptr_t>(cp) & 15) == 0) {
+            // four entries of one column: 16-byte accesses to C when it is aligned for them
             double2* c2 = reinterpret_cast<double2*>(cp);
             if (a.br == 0.0) {
                 c2[0] = make_double2(a.ar * v[0], a.ar * v[1]);
@@ -187,31 +201,19 @@ __device__ __forceinline__ void crt_body(const CrtArgs& a, uint32_t bx) {
                 c2[0] = make_double2(__builtin_fma(a.ar, v[0], a.br * x0.x), __builtin_fma(a.ar, v[1], a.br * x0.y));
                 c2[1] = make_double2(__builtin_fma(a.ar, v[2], a.br * x1.x), __builtin_fma(a.ar, v[3], a.br * x1.y));
             }
-        } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                cp[e] = a.br == 0.0 ? a.ar * v[e] : __builtin_fma(a.ar, v[e], a.br * cp[e]);
+            return;
         }
-        return;
-    }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const int64_t i = i0 + e;
-        if (i >= a.mb) break;
-        const int32_t Di = a.D[i];
-        const bool nonfinite = Di == INT32_MIN || Ej == INT32_MIN;
-        const int shift = nonfinite ? 0 : Di + Ej;
-        if (!CPLX) {
-            double v = re[e].finish(tb, shift);
-            if (nonfinite) v = __builtin_nan("");
-            double* cp = a.C + i + j * a.ldc;
-            *cp = a.br == 0.0 ? a.ar * v : __builtin_fma(a.ar, v, a.br * *cp);
-        } else {
-            double vr = re[e].finish(tb, shift), vi = im[e].finish(tb, shift);
-            if (nonfinite) vr = vi = __builtin_nan("");
+        for (int e = 0; e < 4; ++e)
+            if (i0 + e < a.mb) cp[e] = a.br == 0.0 ? a.ar * v[e] : __builtin_fma(a.ar, v[e], a.br * cp[e]);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int64_t i = i0 + e;
+            if (i >= a.mb) break;
             double* cp = a.C + 2 * (i + j * a.ldc);
-            double orr = __builtin_fma(a.ar, vr, -(a.ai * vi));
-            double oi = __builtin_fma(a.ar, vi, a.ai * vr);
+            double orr = __builtin_fma(a.ar, v[e], -(a.ai * vi[e]));
+            double oi = __builtin_fma(a.ar, vi[e], a.ai * v[e]);
             if (a.br != 0.0 || a.bi != 0.0) {
                 const double cr = cp[0], ci = cp[1];
                 orr = orr + __builtin_fma(a.br, cr, -(a.bi * ci));
@@ -223,18 +225,24 @@ __device__ __forceinline__ void crt_body(const CrtArgs& a, uint32_t bx) {
     }
 }
 
-template <int NL, bool CPLX>
-__global__ void __launch_bounds__(256) crt_kernel(CrtArgs a, uint64_t* ts) {
+// waves per SIMD to compile for (below 256 registers the products' results stay out of the accumulation
+// registers, which the VALU cannot read)
+constexpr int crt_waves(int nl, bool cplx, bool chunks) {
+    return cplx ? (nl > 4 ? 2 : 3) : nl > 4 || chunks ? 4 : 6;
+}
+
+template <int NL, bool CPLX, bool CHUNKS>
+__global__ void __launch_bounds__(256, crt_waves(NL, CPLX, CHUNKS)) crt_kernel(CrtArgs a, uint64_t* ts) {
     const Stamp st(ts);
-    crt_body<NL, CPLX>(a, blockIdx.x);
+    crt_body<NL, CPLX, CHUNKS>(a, blockIdx.x);
     st.end();
 }
 
-template <int NL, bool CPLX>
-__global__ void __launch_bounds__(256) crt_grouped_kernel(const CrtArgs* __restrict__ items,
+template <int NL, bool CHUNKS>
+__global__ void __launch_bounds__(256, crt_waves(NL, false, CHUNKS)) crt_grouped_kernel(const CrtArgs* __restrict__ items,
                                                           const uint32_t* __restrict__ start, uint32_t n) {
     const uint32_t p = owner_of(start, n, blockIdx.x);
-    crt_body<NL, CPLX>(items[p], blockIdx.x - start[p]);
+    crt_body<NL, false, CHUNKS>(items[p], blockIdx.x - start[p]);
 }
 
 uint32_t crt_blocks(const CrtArgs& a) {
@@ -265,8 +273,10 @@ __global__ void scale_c_kernel(double* C, int64_t ldc, int64_t m, int64_t n, dou
 template <int NL>
 void launch_crt_nl(const Stream& st, const CrtArgs& a) {
     const unsigned blocks = crt_blocks(a);
-    if (a.cplx) launch(st, crt_kernel<NL, true>, dim3(blocks), dim3(256), a);
-    else launch(st, crt_kernel<NL, false>, dim3(blocks), dim3(256), a);
+    if (a.cplx && a.kch > 1) launch(st, crt_kernel<NL, true, true>, dim3(blocks), dim3(256), a);
+    else if (a.cplx) launch(st, crt_kernel<NL, true, false>, dim3(blocks), dim3(256), a);
+    else if (a.kch > 1) launch(st, crt_kernel<NL, false, true>, dim3(blocks), dim3(256), a);
+    else launch(st, crt_kernel<NL, false, false>, dim3(blocks), dim3(256), a);
 }
 
 }  // namespace
@@ -283,12 +293,12 @@ void crt(const Stream& st, const CrtArgs& a) {
     }
 }
 
-// grouped CRT: one launch per (limb count, real/complex)
+// grouped CRT (real products): one launch per (limb count, one k-chunk / several)
 void prep_crt(std::vector<GroupedLaunch>& out, const std::vector<CrtArgs>& jobs) {
     GroupedLaunch by[14];
     for (const CrtArgs& a : jobs) {
         if (a.mb <= 0 || a.nb <= 0) continue;
-        const int v = (a.L16 / 2) * 2 + (a.cplx ? 1 : 0);
+        const int v = (a.L16 / 2) * 2 + (a.kch > 1 ? 1 : 0);
         by[v].kind = v;
         by[v].add(a, crt_blocks(a));
     }

@@ -1,7 +1,7 @@
 // math.hpp - per-element integer arithmetic of the Ozaki Scheme II path,
 // shared by the gfx950 kernels and by the host build used to test it on the
 // CPU (csrc/test/emu.cpp).  Everything here is exact integer work except the
-// fp32 CRT quotient estimate, whose error is bounded far below its margin.
+// fixed-point CRT quotient estimate, whose error is bounded far below its margin.
 #pragma once
 #include <cstdint>
 
@@ -10,9 +10,11 @@
 #if defined(__HIPCC__)
 #include <hip/hip_runtime.h>
 #define OZ2_HD __host__ __device__ __forceinline__
+#define OZ2_UNROLL _Pragma("unroll")
 #else
 #include <cmath>
 #define OZ2_HD inline
+#define OZ2_UNROLL
 #endif
 
 namespace oz2 {
@@ -36,14 +38,6 @@ extern "C" __device__ uint32_t oz2_llvm_mulhi_u24(uint32_t, uint32_t) __asm("llv
 extern "C" __device__ int32_t oz2_llvm_mul_i24(int32_t, int32_t) __asm("llvm.amdgcn.mul.i24");
 #endif
 
-// v_mul_u32_u24 / v_mul_hi_u32_u24: low 32 and high 16 bits of a 24 x 24-bit product
-OZ2_HD uint32_t mul24(uint32_t a, uint32_t b) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    return __umul24(a, b);
-#else
-    return static_cast<uint32_t>(static_cast<uint64_t>(a & 0xFFFFFFu) * static_cast<uint64_t>(b & 0xFFFFFFu));
-#endif
-}
 // v_mad_i32_i24: a * b + c with a, b sign-extended from 24 bits (low 32 bits of the result)
 OZ2_HD uint32_t mad_i24(int32_t a, int32_t b, uint32_t c) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -54,6 +48,7 @@ OZ2_HD uint32_t mad_i24(int32_t a, int32_t b, uint32_t c) {
     return static_cast<uint32_t>(static_cast<uint64_t>(sa * sb)) + c;
 #endif
 }
+// v_mul_hi_u32_u24: high 16 bits of a 24 x 24-bit product
 OZ2_HD uint32_t mulhi24(uint32_t a, uint32_t b) {
 #if defined(__HIP_DEVICE_COMPILE__)
     return oz2_llvm_mulhi_u24(a, b);
@@ -257,85 +252,84 @@ OZ2_HD double ldexp_(double v, int e) {
 #endif
 }
 
-// Exact reconstruction of one entry from residues r_t in [0, m_t); NL = 32-bit words of M.
-// The quotient q = round(sum_t r_t y_t / m_t) is taken in 16.16 fixed point: with
+// Exact reconstruction of one entry from its limb and quotient sums (as rows of the
+// matrix product of TabSet::Wd and Kc, or by dot products); NL = 32-bit words of M.  The quotient q = round(sum_t r_t y_t / m_t) is taken in 16.16 fixed point: with
 // F_t = round(2^16 y_t / m_t) the sum sum_t r_t F_t / 2^16 is within s * 255 * 2^-17 < 0.05 of
 // the exact one, which lies within 1/4 of q whenever |C'| <= M/4 (the scaling guarantees it),
 // so rounding it gives q (the reference's fp32 estimate gives the same q for the same reason).
-// The fixed-point sum is one more dot2 per modulus pair in the limb sums.
+//
+// C' = sum_t r_t W_t - q M as NL little-endian words (two's complement, mod 2^(32 NL)) from its 2 NL limb
+// sums, each with q Mc16 below 2^30 in magnitude.
+template <int NL, typename Tab, typename Limb>
+OZ2_HD void crt_carry(Tab tb, uint32_t uq, Limb limb, uint32_t (&w)[NL]) {
+    const int32_t q = static_cast<int32_t>(uq >> 16);
+    int32_t carry = 0;
+    OZ2_UNROLL for (int l = 0; l < 2 * NL; ++l) {
+        const int32_t v = static_cast<int32_t>(mad_i24(q, static_cast<int32_t>(tb->Mc16[l]), limb(l))) + carry;
+        const uint32_t lo = static_cast<uint32_t>(v) & 0xFFFFu;
+        if (l & 1) w[l >> 1] |= lo << 16;
+        else w[l >> 1] = lo;
+        carry = v >> 16;
+    }
+}
+
+// from the rows of the matrix product: limb l is x[2l] + 256 x[2l+1] (24 * 128 * 128 * 257 + 24 * 128 * 65535
+// + 24 * 255 * 65535 < 2^30); the 2^15 of q's rounding is in Kc
+template <int NL, typename Tab, typename Row>
+OZ2_HD void crt_words(Tab tb, Row x, uint32_t (&w)[NL]) {
+    const uint32_t uq = static_cast<uint32_t>(x(4 * NL)) + ((static_cast<uint32_t>(x(4 * NL + 1)) +
+                                                            (static_cast<uint32_t>(x(4 * NL + 2)) << 8)) << 8);
+    crt_carry<NL>(tb, uq, [&](int l) { return static_cast<uint32_t>(x(2 * l)) + (static_cast<uint32_t>(x(2 * l + 1)) << 8); }, w);
+}
+
+// the limb and quotient sums by 16-bit dot products: moduli 2i and 2i+1 at once (r1 = 0 past s), one dot2
+// per limb (r < 256, W16 < 2^16: sums below 2^29)
 template <int NL>
 struct CrtAcc {
-    static constexpr int L = 2 * NL;
-    uint32_t uq;  // sum r_t F_t < 24 * 255 * 2^16 < 2^29
-    uint32_t acc[L];
-    OZ2_HD void init() {
-        uq = 0;
-        for (int l = 0; l < L; ++l) acc[l] = 0;
-    }
-    // uq += r F_t; acc_l += r W16[t][l]  (r < 256, W16 < 2^16: products < 2^24, sums < 2^29)
-    template <typename Tab>
-    OZ2_HD void add(Tab tb, int t, uint32_t r) {
-        uq += mul24(r, tb->F16[t]);
-        for (int l = 0; l < L; ++l) acc[l] += mul24(r, tb->W16[t][l]);
-    }
-    // moduli 2i and 2i+1 at once (r1 = 0 past s): one dot2 per limb with the paired table
+    uint32_t uq = 0x8000u, acc[2 * NL] = {};
     template <typename Tab>
     OZ2_HD void add2(Tab tb, int i, uint32_t r0, uint32_t r1) {
         const uint32_t rr = r0 | (r1 << 16);
         uq = udot2(rr, tb->F16p[i], uq);
-        for (int l = 0; l < L; ++l) acc[l] = udot2(rr, tb->W16p[i][l], acc[l]);
+        OZ2_UNROLL for (int l = 0; l < 2 * NL; ++l) acc[l] = udot2(rr, tb->W16p[i][l], acc[l]);
     }
-    // RNE(C') * 2^-shift with C' = sum r_t W_t - q M
     template <typename Tab>
-    OZ2_HD double finish(Tab tb, int shift) const {
-        const int32_t q = static_cast<int32_t>((uq + 0x8000u) >> 16);
-        uint32_t w[NL];
-        int32_t carry = 0;
-        for (int l = 0; l < L; ++l) {
-            // 0 <= q <= s * 255 and M16 < 2^16: one v_mad_i32_i24
-            const int32_t v = static_cast<int32_t>(mad_i24(-q, static_cast<int32_t>(tb->M16[l]), acc[l] + static_cast<uint32_t>(carry)));
-            const uint32_t lo = static_cast<uint32_t>(v) & 0xFFFFu;
-            if (l & 1) w[l >> 1] |= lo << 16;
-            else w[l >> 1] = lo;
-            carry = v >> 16;
-        }
-        const bool neg = (w[NL - 1] >> 31) != 0;
-        if (neg) {
-            uint32_t cy = 1;
-            for (int l = 0; l < NL; ++l) {
-                const uint64_t s = static_cast<uint64_t>(~w[l]) + cy;
-                w[l] = static_cast<uint32_t>(s);
-                cy = static_cast<uint32_t>(s >> 32);
-            }
-        }
-        // |C'| as G 64-bit groups; the window is the top 64 bits of the leading nonzero group
-        // and the one below it, every lower bit folded into a sticky bit
-        constexpr int G = (NL + 1) / 2;
-        static_assert(G <= 3, "at most 6 words");
-        uint64_t g[G];
-        for (int i = 0; i < G; ++i)
-            g[i] = w[2 * i] | (2 * i + 1 < NL ? static_cast<uint64_t>(w[2 * i + 1]) << 32 : 0);
-        uint64_t hi = g[G - 1], lo = G >= 2 ? g[G - 2] : 0;
-        bool below = G == 3 && g[0] != 0;
-        int base = 64 * (G - 1);  // log2 weight of hi's lowest bit
-        for (int step = 0; step + 1 < G; ++step) {  // step down past zero groups
-            const bool z = hi == 0;
-            const int idx = G - 2 - step;            // lo is group idx
-            hi = z ? lo : hi;
-            lo = z ? (idx >= 1 ? g[idx - 1] : 0) : lo;
-            base -= z ? 64 : 0;
-            below = z ? false : below;               // with G <= 3 nothing lies below the new lo
-        }
-        if (hi == 0) return 0.0;
-        const int z = clz64(hi);
-        uint64_t top = z ? (hi << z) | (lo >> (64 - z)) : hi;
-        const uint64_t rest = z ? (lo << z) : lo;
-        top |= (below || rest != 0) ? 1u : 0u;
-        // the window's lsb weighs 2^(base - z); one RNE here, a second only if subnormal
-        const double v = ldexp_(static_cast<double>(top), base - z - shift);
-        return neg ? -v : v;
+    OZ2_HD void words(Tab tb, uint32_t (&w)[NL]) const {
+        crt_carry<NL>(tb, uq, [&](int l) { return acc[l]; }, w);
     }
 };
+
+// RNE(C') * 2^-shift.  The window is 64 bits of C' from its sign bit on, every lower bit folded into the
+// window's last one (sticky).  It stays in two's complement: the fold moves the value towards the next odd
+// number, and the rounding boundaries of a 53-bit result are even, so negative values round as their
+// magnitudes do.
+template <int NL>
+OZ2_HD double crt_round(const uint32_t (&w)[NL], int shift) {
+    constexpr int G = (NL + 1) / 2;
+    static_assert(G <= 3, "at most 6 words");
+    int64_t g[G];
+    OZ2_UNROLL for (int i = 0; i < G; ++i) {
+        const uint32_t top = 2 * i + 1 < NL ? w[2 * i + 1] : static_cast<uint32_t>(static_cast<int32_t>(w[NL - 1]) >> 31);
+        g[i] = static_cast<int64_t>(w[2 * i] | static_cast<uint64_t>(top) << 32);
+    }
+    int64_t hi = g[G - 1], lo = G >= 2 ? g[G - 2] : 0;
+    bool below = G == 3 && g[0] != 0;
+    int base = 64 * (G - 1);  // log2 weight of hi's lowest bit
+    OZ2_UNROLL for (int step = 0; step + 1 < G; ++step) {  // step down past groups that only extend the sign
+        const bool z = hi == lo >> 63;
+        const int idx = G - 2 - step;            // lo is group idx
+        hi = z ? lo : hi;
+        lo = z ? (idx >= 1 ? g[idx - 1] : 0) : lo;
+        base -= z ? 64 : 0;
+        below = z ? false : below;               // with G <= 3 nothing lies below the new lo
+    }
+    const int sh = clz64(static_cast<uint64_t>(hi ^ (hi >> 63))) - 1;  // sign bits but one: 0 .. 63
+    uint64_t top = (static_cast<uint64_t>(hi) << sh) | ((static_cast<uint64_t>(lo) >> 1) >> (63 - sh));
+    const uint64_t rest = static_cast<uint64_t>(lo) << sh;
+    top |= (below || rest != 0) ? 1u : 0u;
+    // the window's lsb weighs 2^(base - sh); one RNE here, a second only if subnormal
+    return ldexp_(static_cast<double>(static_cast<int64_t>(top)), base - sh - shift);
+}
 
 }  // namespace math
 }  // namespace oz2

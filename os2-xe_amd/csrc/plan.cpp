@@ -160,14 +160,33 @@ void make_tabsets(TabSet* out) {
             tb.h2[t] = 2 * h;
             for (int j = 0; j < 16; ++j) tb.c8[t][j >> 2] |= static_cast<uint32_t>(pow2_mod(8 * j, m)) << (8 * (j & 3));
             tb.c30[t] = m == 256 ? 0 : m * static_cast<uint32_t>(((uint64_t{1} << 30) + m - 1) / m);
-            tb.F16[t] = static_cast<uint32_t>((static_cast<uint64_t>(p.y[t]) * (1u << 17) + m) / (2u * m));
-            for (int l = 0; l < tb.L16; ++l) tb.W16[t][l] = (p.W[t].word32(l / 2) >> (16 * (l % 2))) & 0xFFFFu;
+            // balanced digits in [-128, 127]; the carry out of the last one is dropped (mod 2^(32 NL))
+            auto digits = [&](auto byte, int row0, int n) {
+                int carry = 0;
+                for (int i = 0; i < n; ++i) {
+                    int d = byte(i) + carry;
+                    carry = d > 127;
+                    d -= carry ? 256 : 0;
+                    tb.Wd[row0 + i][t] = static_cast<int8_t>(d);
+                }
+            };
+            const uint32_t F = static_cast<uint32_t>((static_cast<uint64_t>(p.y[t]) * (1u << 17) + m) / (2u * m));
+            digits([&](int i) { return static_cast<int>((p.W[t].word32(i / 4) >> (8 * (i % 4))) & 0xFFu); }, 0, 4 * p.NL);
+            digits([&](int i) { return static_cast<int>((F >> (8 * i)) & 0xFFu); }, 4 * p.NL, 3);
+            tb.F16p[t / 2] |= F << (16 * (t % 2));
+            for (int l = 0; l < tb.L16; ++l) {
+                const uint32_t limb = (p.W[t].word32(l / 2) >> (16 * (l % 2))) & 0xFFFFu;
+                tb.Kc[2 * l] += static_cast<int32_t>(128u * limb);
+                tb.W16p[t / 2][l] |= limb << (16 * (t % 2));
+            }
+            tb.Kc[4 * p.NL] += static_cast<int32_t>(128u * F);
         }
-        for (int l = 0; l < tb.L16; ++l) tb.M16[l] = (p.M.word32(l / 2) >> (16 * (l % 2))) & 0xFFFFu;
-        for (int t = 0; t < s; t += 2) {
-            for (int l = 0; l < tb.L16; ++l)
-                tb.W16p[t / 2][l] = tb.W16[t][l] | (t + 1 < s ? tb.W16[t + 1][l] << 16 : 0u);
-            tb.F16p[t / 2] = tb.F16[t] | (t + 1 < s ? tb.F16[t + 1] << 16 : 0u);
+        tb.Kc[4 * p.NL] += 0x8000;
+        uint32_t borrow = 1;  // 2^(32 NL) - M = ~M + 1
+        for (int l = 0; l < tb.L16; ++l) {
+            const uint32_t v = (~(p.M.word32(l / 2) >> (16 * (l % 2))) & 0xFFFFu) + borrow;
+            tb.Mc16[l] = v & 0xFFFFu;
+            borrow = v >> 16;
         }
     }
 }

@@ -80,6 +80,7 @@ int moduli_for_bits(int64_t k, int bits);
 // One TabSet per s (2..24), built on the host and copied to device memory once
 // per engine; kernels read it through a const __restrict__ pointer, so the
 // per-modulus constants come in through scalar loads.
+inline constexpr int kCrtRows = 32;      // rows of the CRT's matrix product (4 NL + 3 <= 27 used)
 struct TabSet {
     int32_t s;
     int32_t L16;                            // 16-bit limbs of M: 2 * NL
@@ -93,12 +94,16 @@ struct TabSet {
     uint32_t h2[kMaxModuli];                // 2 h
     uint32_t c8[kMaxModuli][4];             // bytes 2^(8 j) mod m, j = 0..15, four to a word (low first)
     uint32_t c30[kMaxModuli];               // m * ceil(2^30 / m) (GEMM residue epilogue offset; 0 for m = 256)
-    // CRT (hpp:222-236)
-    uint32_t F16[kMaxModuli];               // round(2^16 y_t / m_t): fixed-point quotient weights
-    uint32_t F16p[kMaxModuli / 2];          // F16[2i] | F16[2i+1] << 16 (0 past s)
-    uint32_t W16[kMaxModuli][2 * kMaxLimbs];  // 16-bit limbs of W_t
-    uint32_t W16p[kMaxModuli / 2][2 * kMaxLimbs];  // W16[2i][l] | W16[2i+1][l] << 16 (0 past s)
-    uint32_t M16[2 * kMaxLimbs];            // 16-bit limbs of M
+    // CRT (hpp:222-236) as an int8 matrix product over the moduli: row r of the sums is
+    // sum_t (r_t - 128) Wd[r][t] + Kc[r].  Rows 0 .. 4 NL - 1 are the balanced base-256 digits of
+    // W_t mod 2^(32 NL), rows 4 NL .. 4 NL + 2 those of the quotient weight F_t = round(2^16 y_t / m_t);
+    // Kc adds the 128 W_t (per 16-bit limb, in the limb's even row) and 128 F_t + 2^15 back.
+    alignas(16) int8_t Wd[kCrtRows][32];
+    alignas(16) int32_t Kc[kCrtRows];
+    uint32_t Mc16[2 * kMaxLimbs];           // 16-bit limbs of 2^(32 NL) - M
+    // the same sums by 16-bit dot products, two moduli a step
+    uint32_t F16p[kMaxModuli / 2];          // F_2i | F_2i+1 << 16 (0 past s)
+    uint32_t W16p[kMaxModuli / 2][2 * kMaxLimbs];  // 16-bit limbs l of W_2i | W_2i+1 << 16 (0 past s)
 };
 // tables for s = 0..24 (entries 0 and 1 unused); y_t and W_t do not depend on k
 void make_tabsets(TabSet* out /* [kMaxModuli + 1] */);
