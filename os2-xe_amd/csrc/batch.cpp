@@ -154,6 +154,7 @@ BatchPlan::BatchPlan(Engine& eng, std::vector<GemmDesc> descs, const std::vector
             c.cplx = false;
             c.s = s_[i];
             c.L16 = 2 * q.plan.NL;
+            c.up = q.plan.up();
             c.tab = tabs + s_[i];
             cj.push_back(c);
         }

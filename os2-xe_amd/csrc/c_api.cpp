@@ -516,6 +516,7 @@ int oz2_unit_crt(void* stream, const uint8_t* R, int64_t ldr, int64_t mb, int64_
         a.br = beta;
         a.s = num_moduli;
         a.L16 = 2 * oz2::limbs_for(num_moduli);
+        a.up = oz2::make_plan(num_moduli, 1).up();
         a.tab = unit_tables() + num_moduli;
         oz2::k::crt(static_cast<hipStream_t>(stream), a);
         if (hipGetLastError() != hipSuccess) throw std::runtime_error("oz2: crt launch failed");

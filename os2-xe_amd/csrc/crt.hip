@@ -1,7 +1,7 @@
 // crt.hip - CRT reconstruction fused with the alpha/beta epilogue, for gfx950.
 //
-// Bounds: HBM up to s = 16 (s + 8 or 16 bytes an entry; 5.2 TB/s at 8192 x 8192 s = 16, the rate of a plain
-// copy), the VALU above (3.6 TB/s at s = 24).
+// Bounds: HBM up to s = 16 (s + 8 or 16 bytes an entry; 5.3 TB/s at 8192 x 8192 s = 16, the rate of a plain
+// copy), the VALU above (4.0 TB/s at s = 24).
 //
 // Reference behaviour: src/ozaki2_gpu.hpp:526-664.  For each entry the s
 // residues r_t (bytes from the GEMM epilogue; k-chunks are summed mod m_t)
@@ -75,10 +75,13 @@ __device__ __forceinline__ void from_3m(uint32_t w0, uint32_t w1, uint32_t w2, u
 }
 
 // Matrix cores or dot products for the limb and quotient sums.  With few moduli the kernel is bound by its
-// loads, and the dot products' registers (44 to 68, against 87 to 100) keep more waves in flight; with many
+// loads, and the dot products' registers (44 to 78, against 87 and more) keep more waves in flight; with many
 // it is bound by the sums.  Measured on MI355X, beta != 0, matrix / dot products, us: 4096 x 4096
-// s = 8 72 / 62, s = 16 124 / 109, s = 20 131 / 160, s = 24 150 / 192; 8192 x 8192 s = 16 459 / 414
-// (5.2 TB/s); complex 4096 x 4096 s = 16 324 / 357, s = 24 430 / 489.
+// s = 8 72 / 62, s = 16 124 / 109, s = 20 131 / 160, s = 24 150 / 192; 8192 x 8192 s = 16 459 / 414;
+// complex 4096 x 4096 s = 16 324 / 357, s = 24 430 / 489 (before the two-double rounding of crt_round, which
+// took 2 to 7 % off each: 8192 x 8192 s = 16 404, 4096 x 4096 s = 24 135, complex 315 and 411).
+// No scalar load may be left for the end of the kernel: one (the scaling exponent, from the tables) made it
+// 30 % slower, so that comes as an argument.
 constexpr bool crt_matrix(int nl, bool cplx) { return cplx ? nl >= 4 : nl >= 5; }
 
 template <int NL, bool MAT>
@@ -177,16 +180,15 @@ __device__ __forceinline__ void crt_body(const CrtArgs& a, uint32_t bx) {
     for (int e = 0; e < 4; ++e) {
         const int32_t Di = a.D[min(i0 + e, a.mb - 1)];
         nonfinite[e] = Di == INT32_MIN || Ej == INT32_MIN;
-        shift[e] = nonfinite[e] ? 0 : Di + Ej;
+        shift[e] = Di + Ej + a.up;
     }
     double v[4], vi[4];
-    sums.four(re, [&](int e, const uint32_t (&w)[NL]) {
-        v[e] = nonfinite[e] ? __builtin_nan("") : crt_round<NL>(w, shift[e]);
-    });
+    crt_four<NL>(sums, re, shift, v);
     if constexpr (CPLX)
-        sums.four(im, [&](int e, const uint32_t (&w)[NL]) {
-            vi[e] = nonfinite[e] ? __builtin_nan("") : crt_round<NL>(w, shift[e]);
-        });
+        crt_four<NL>(sums, im, shift, vi);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        if (nonfinite[e]) v[e] = vi[e] = __builtin_nan("");
     if (!ok) return;
     if constexpr (!CPLX) {
         double* cp = a.C + i0 + j * a.ldc;

@@ -49,7 +49,7 @@ struct CrtTile {
     }
 
     // r[t]: residues of modulus t of the lane's four entries, one byte each (any value past s);
-    // out(e, w): words of C' of entry e.  All lanes of the wave take part.
+    // out(e, w): words of V of entry e.  All lanes of the wave take part.
     template <typename Out>
     __device__ __forceinline__ void four(const uint32_t (&r)[SC], const Out& out) const {
         // 4 x 4 byte transposes: b[e] = residues of entry e, minus 128, by modulus
@@ -93,6 +93,23 @@ struct CrtTile {
         }
     }
 };
+
+// RNE(V) 2^-shift of four entries from their sums (CrtTile or the dot products)
+template <int NL, typename Sums>
+__device__ __forceinline__ void crt_four(const Sums& sums, const uint32_t (&r)[4 * NL], const int32_t (&shift)[4],
+                                         double (&v)[4]) {
+    // entries far below their bound, rare, take the general window: up to 16 moduli the wave takes the quad
+    // again (all lanes are needed), above, where holding the residues for that would spill, entry by entry
+    bool any = false;
+    sums.four(r, [&](int e, const uint32_t (&w)[NL]) {
+        bool f;
+        v[e] = math::crt_round<NL>(w, shift[e], f);
+        if (NL > 4 && f) v[e] = math::crt_round_any<NL>(w, shift[e]);
+        any |= f;
+    });
+    if (NL == 4 && __any(any))
+        sums.four(r, [&](int e, const uint32_t (&w)[NL]) { v[e] = math::crt_round_any<NL>(w, shift[e]); });
+}
 
 }  // namespace k
 }  // namespace oz2

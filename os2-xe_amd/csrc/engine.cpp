@@ -414,6 +414,7 @@ void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, doubl
         ca.cplx = cplx;
         ca.s = s;
         ca.L16 = 2 * p.NL;
+        ca.up = p.up();
         ca.tab = tab;
         k::crt(on, ca);
     };

@@ -147,9 +147,23 @@ struct CrtArgs {
     double ar, ai, br, bi;
     bool cplx;
     int s, L16;
+    int up;               // Plan::up()
     const TabSet* tab;    // device tables of this s
 };
 void crt(const Stream& st, const CrtArgs& a);
+
+// ---- GEMMs of all planes and the CRT of a tile in one workgroup -------------------
+struct FusedArgs {
+    const int8_t *A, *B;
+    int64_t kp, plane_a, plane_b;
+    int tiles_m, tiles_n, s, nl;
+    const TabSet* tab;
+    const int32_t *D, *E;
+    double* C;
+    int64_t mb, nb, ldc;
+    double ar, br;
+};
+void fused(const Stream& st, int code, const FusedArgs& a);
 
 // ---- Ozaki Scheme I (the accuracy benchmark's comparison baseline) --------------------
 // L balanced base-128 digits of RNE(op(X)[r][p] 2^ex[r]) per element into one extended

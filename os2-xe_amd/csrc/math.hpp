@@ -219,6 +219,15 @@ OZ2_HD uint32_t pack_lo_bytes(uint32_t b0, uint32_t b1, uint32_t b2, uint32_t b3
 #endif
 }
 
+// the low halves of a and b in one word (a lowest)
+OZ2_HD uint32_t pack_lo_halves(uint32_t a, uint32_t b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_perm(b, a, 0x05040100u);
+#else
+    return (a & 0xFFFFu) | b << 16;
+#endif
+}
+
 // symmetric residue value in [-h, m-1-h] (complex split needs the value, not the byte)
 template <Limbs F, typename Tab>
 OZ2_HD int32_t sym_value(const uint32_t (&a)[4], Tab tb, int t) {
@@ -258,18 +267,36 @@ OZ2_HD double ldexp_(double v, int e) {
 // the exact one, which lies within 1/4 of q whenever |C'| <= M/4 (the scaling guarantees it),
 // so rounding it gives q (the reference's fp32 estimate gives the same q for the same reason).
 //
-// C' = sum_t r_t W_t - q M as NL little-endian words (two's complement, mod 2^(32 NL)) from its 2 NL limb
-// sums, each with q Mc16 below 2^30 in magnitude.
+// keeps the compiler from merging the operations before and after
+OZ2_HD void settle(int32_t& x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm("" : "+v"(x));
+#else
+    (void)x;
+#endif
+}
+
+// V = 2^up C' = sum_t r_t (2^up W_t) - q (2^up M) as NL little-endian words (two's complement, mod 2^(32 NL);
+// |V| < 2^(32 NL - 2)) from its 2 NL limb sums, each with q Mc16 below 2^30 in magnitude.  Per limb one
+// v_mad_i32_i24 and one add whose carry operand is the high half of its register (SDWA); without settle()
+// the compiler takes a multiplication, a shift and a three-way addition.
 template <int NL, typename Tab, typename Limb>
 OZ2_HD void crt_carry(Tab tb, uint32_t uq, Limb limb, uint32_t (&w)[NL]) {
-    const int32_t q = static_cast<int32_t>(uq >> 16);
-    int32_t carry = 0;
-    OZ2_UNROLL for (int l = 0; l < 2 * NL; ++l) {
-        const int32_t v = static_cast<int32_t>(mad_i24(q, static_cast<int32_t>(tb->Mc16[l]), limb(l))) + carry;
-        const uint32_t lo = static_cast<uint32_t>(v) & 0xFFFFu;
-        if (l & 1) w[l >> 1] |= lo << 16;
-        else w[l >> 1] = lo;
-        carry = v >> 16;
+    int32_t q = static_cast<int32_t>(uq) >> 16;
+    settle(q);
+    int32_t prev = 0;
+    OZ2_UNROLL for (int i = 0; i < NL; ++i) {
+        int32_t v[2];
+        OZ2_UNROLL for (int h = 0; h < 2; ++h) {
+            const int l = 2 * i + h;
+            int32_t x = static_cast<int32_t>(limb(l));
+            settle(x);
+            x = static_cast<int32_t>(mad_i24(q, static_cast<int32_t>(tb->Mc16[l]), static_cast<uint32_t>(x)));
+            settle(x);
+            v[h] = x + (prev >> 16);
+            prev = v[h];
+        }
+        w[i] = pack_lo_halves(static_cast<uint32_t>(v[0]), static_cast<uint32_t>(v[1]));
     }
 }
 
@@ -299,12 +326,12 @@ struct CrtAcc {
     }
 };
 
-// RNE(C') * 2^-shift.  The window is 64 bits of C' from its sign bit on, every lower bit folded into the
-// window's last one (sticky).  It stays in two's complement: the fold moves the value towards the next odd
-// number, and the rounding boundaries of a 53-bit result are even, so negative values round as their
-// magnitudes do.
+// RNE(V) * 2^-shift (shift includes up), any V.  The window is 64 bits of V from its sign bit on, every lower
+// bit folded into the window's last one (sticky).  It stays in two's complement: the fold moves the value
+// towards the next odd number, and the rounding boundaries of a 53-bit result are even, so negative values
+// round as their magnitudes do.
 template <int NL>
-OZ2_HD double crt_round(const uint32_t (&w)[NL], int shift) {
+OZ2_HD double crt_round_any(const uint32_t (&w)[NL], int shift) {
     constexpr int G = (NL + 1) / 2;
     static_assert(G <= 3, "at most 6 words");
     int64_t g[G];
@@ -329,6 +356,28 @@ OZ2_HD double crt_round(const uint32_t (&w)[NL], int shift) {
     top |= (below || rest != 0) ? 1u : 0u;
     // the window's lsb weighs 2^(base - sh); one RNE here, a second only if subnormal
     return ldexp_(static_cast<double>(static_cast<int64_t>(top)), base - sh - shift);
+}
+
+// RNE(V) * 2^-shift: the top 96 bits of V as a sum of two 48-bit doubles, a 2^48 + b, exact but for the last
+// bit of b, which folds in every lower word; one addition rounds it.  The fold is right where a unit of the
+// result is at least four of b's (the rounding boundaries are then even): |a| >= 65, that is |C'| above about
+// 2^-40 of its bound, or where nothing was folded (every V of at most 3 words, and V = 0).  For the rest, rare,
+// `any` is set and crt_round_any has the value.
+template <int NL>
+OZ2_HD double crt_round(const uint32_t (&w)[NL], int shift, bool& any) {
+    any = false;
+    if (NL == 2) {
+        const double v = __builtin_fma(static_cast<double>(static_cast<int32_t>(w[1])), 4294967296.0, static_cast<double>(w[0]));
+        return ldexp_(v, -shift);
+    }
+    constexpr int T = NL >= 3 ? NL : 3;  // (the words below exist for NL >= 3)
+    uint32_t low = 0;
+    OZ2_UNROLL for (int i = 0; i + 3 < NL; ++i) low |= w[i];
+    const double a = __builtin_fma(static_cast<double>(static_cast<int32_t>(w[T - 1])), 65536.0, static_cast<double>(w[T - 2] >> 16));
+    const uint32_t w0 = w[T - 3] | (low < 1u ? low : 1u);
+    const double b = __builtin_fma(static_cast<double>(w[T - 2] & 0xFFFFu), 4294967296.0, static_cast<double>(w0));
+    any = NL > 3 && __builtin_fabs(a) < 65.0 && low != 0;
+    return ldexp_(__builtin_fma(a, 281474976710656.0, b), 32 * (NL - 3) - shift);
 }
 
 }  // namespace math

@@ -145,6 +145,10 @@ void make_tabsets(TabSet* out) {
         TabSet& tb = out[s];
         tb.s = s;
         tb.L16 = 2 * p.NL;
+        auto scale = [&](Wide& w) {  // w 2^up
+            for (int u = p.up(); u > 0; u -= 31) w.mul(1u << std::min(u, 31));
+        };
+        auto limb = [](const Wide& w, int l) { return (w.word32(l / 2) >> (16 * (l % 2))) & 0xFFFFu; };
         for (int t = 0; t < s; ++t) {
             const uint32_t m = p.m[t];
             const uint32_t h = (m - 1) / 2;
@@ -170,21 +174,25 @@ void make_tabsets(TabSet* out) {
                     tb.Wd[row0 + i][t] = static_cast<int8_t>(d);
                 }
             };
+            Wide W = p.W[t];  // W_t 2^up; its digits and limbs mod 2^(32 NL)
+            scale(W);
             const uint32_t F = static_cast<uint32_t>((static_cast<uint64_t>(p.y[t]) * (1u << 17) + m) / (2u * m));
-            digits([&](int i) { return static_cast<int>((p.W[t].word32(i / 4) >> (8 * (i % 4))) & 0xFFu); }, 0, 4 * p.NL);
+            digits([&](int i) { return static_cast<int>((limb(W, i / 2) >> (8 * (i % 2))) & 0xFFu); }, 0, 4 * p.NL);
             digits([&](int i) { return static_cast<int>((F >> (8 * i)) & 0xFFu); }, 4 * p.NL, 3);
             tb.F16p[t / 2] |= F << (16 * (t % 2));
             for (int l = 0; l < tb.L16; ++l) {
-                const uint32_t limb = (p.W[t].word32(l / 2) >> (16 * (l % 2))) & 0xFFFFu;
-                tb.Kc[2 * l] += static_cast<int32_t>(128u * limb);
-                tb.W16p[t / 2][l] |= limb << (16 * (t % 2));
+                const uint32_t x = limb(W, l);
+                tb.Kc[2 * l] += static_cast<int32_t>(128u * x);
+                tb.W16p[t / 2][l] |= x << (16 * (t % 2));
             }
             tb.Kc[4 * p.NL] += static_cast<int32_t>(128u * F);
         }
         tb.Kc[4 * p.NL] += 0x8000;
-        uint32_t borrow = 1;  // 2^(32 NL) - M = ~M + 1
+        Wide M = p.M;
+        scale(M);
+        uint32_t borrow = 1;  // 2^(32 NL) - x = ~x + 1
         for (int l = 0; l < tb.L16; ++l) {
-            const uint32_t v = (~(p.M.word32(l / 2) >> (16 * (l % 2))) & 0xFFFFu) + borrow;
+            const uint32_t v = (~limb(M, l) & 0xFFFFu) + borrow;
             tb.Mc16[l] = v & 0xFFFFu;
             borrow = v >> 16;
         }

@@ -65,6 +65,7 @@ struct Plan {
     uint32_t y[kMaxModuli] = {};
     Wide W[kMaxModuli];
     Wide M;
+    int up() const { return 32 * NL - M.bits(); }  // the CRT works on C' 2^up (TabSet)
 };
 
 // Throws std::invalid_argument (s out of range, k < 1, s too small for k),
@@ -94,16 +95,17 @@ struct TabSet {
     uint32_t h2[kMaxModuli];                // 2 h
     uint32_t c8[kMaxModuli][4];             // bytes 2^(8 j) mod m, j = 0..15, four to a word (low first)
     uint32_t c30[kMaxModuli];               // m * ceil(2^30 / m) (GEMM residue epilogue offset; 0 for m = 256)
-    // CRT (hpp:222-236) as an int8 matrix product over the moduli: row r of the sums is
+    // CRT (hpp:222-236), of C' 2^up with up = 32 NL - bits(M): its sign bit is then the top bit of NL words
+    // whatever M is.  As an int8 matrix product over the moduli row r of the sums is
     // sum_t (r_t - 128) Wd[r][t] + Kc[r].  Rows 0 .. 4 NL - 1 are the balanced base-256 digits of
-    // W_t mod 2^(32 NL), rows 4 NL .. 4 NL + 2 those of the quotient weight F_t = round(2^16 y_t / m_t);
-    // Kc adds the 128 W_t (per 16-bit limb, in the limb's even row) and 128 F_t + 2^15 back.
+    // W_t 2^up mod 2^(32 NL), rows 4 NL .. 4 NL + 2 those of the quotient weight F_t = round(2^16 y_t / m_t);
+    // Kc adds the 128 W_t 2^up (per 16-bit limb, in the limb's even row) and 128 F_t + 2^15 back.
     alignas(16) int8_t Wd[kCrtRows][32];
     alignas(16) int32_t Kc[kCrtRows];
-    uint32_t Mc16[2 * kMaxLimbs];           // 16-bit limbs of 2^(32 NL) - M
+    uint32_t Mc16[2 * kMaxLimbs];           // 16-bit limbs of 2^(32 NL) - M 2^up
     // the same sums by 16-bit dot products, two moduli a step
     uint32_t F16p[kMaxModuli / 2];          // F_2i | F_2i+1 << 16 (0 past s)
-    uint32_t W16p[kMaxModuli / 2][2 * kMaxLimbs];  // 16-bit limbs l of W_2i | W_2i+1 << 16 (0 past s)
+    uint32_t W16p[kMaxModuli / 2][2 * kMaxLimbs];  // 16-bit limbs l of W_2i 2^up | W_2i+1 2^up << 16 (0 past s)
 };
 // tables for s = 0..24 (entries 0 and 1 unused); y_t and W_t do not depend on k
 void make_tabsets(TabSet* out /* [kMaxModuli + 1] */);

@@ -117,7 +117,7 @@ void emu_acc_residue(const int32_t* x, int64_t n, int s, uint8_t* out) {
 // CRT of residues res[i * s + t] in [0, m_t): out[i] = RNE(C') * 2^-shift[i]
 void emu_crt(const uint8_t* res, const int32_t* shift, int64_t n, int s, double* out) {
     const TabSet* tb = tables() + s;
-    const int nl = limbs_for(s);
+    const int nl = limbs_for(s), up = make_plan(s, 1).up();
     for (int64_t i = 0; i < n; ++i) {
         const uint8_t* r = res + i * s;
         switch (nl) {
@@ -130,7 +130,8 @@ void emu_crt(const uint8_t* res, const int32_t* shift, int64_t n, int s, double*
         };                                                 \
         uint32_t w[NL];                                    \
         math::crt_words<NL>(tb, row, w);                   \
-        out[i] = math::crt_round<NL>(w, shift[i]);         \
+        bool fold;                                         \
+        out[i] = math::crt_round<NL>(w, shift[i] + up, fold); \
         math::CrtAcc<NL> a;                                \
         uint32_t wd[NL];                                   \
         for (int t = 0; t < s; t += 2)                     \
@@ -138,6 +139,10 @@ void emu_crt(const uint8_t* res, const int32_t* shift, int64_t n, int s, double*
         a.words(tb, wd);                                   \
         /* both forms of the sums give the same words */   \
         if (std::memcmp(w, wd, sizeof(w)) != 0) out[i] = NAN; \
+        /* and both roundings the same value where the short one holds */ \
+        const double any = math::crt_round_any<NL>(w, shift[i] + up); \
+        if (fold) out[i] = any;                            \
+        if (std::memcmp(&any, &out[i], 8) != 0) out[i] = NAN; \
         break;                                             \
     }
             OZ2_EMU_NL(2) OZ2_EMU_NL(3) OZ2_EMU_NL(4) OZ2_EMU_NL(5) OZ2_EMU_NL(6)

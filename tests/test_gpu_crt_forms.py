@@ -31,6 +31,14 @@ def test_complex_quads(oz, s):
         complex_case(oz, "N", "C", m, n, 40, s, "phi", alpha=1 + 0.5j, beta=beta, ld_extra=pad, check_bound=False)
 
 
+@pytest.mark.parametrize("s", EDGES[2:])
+def test_far_below_the_bound(oz, s):
+    # small integers: |C'| is tiny next to M / 4, so the rounding takes its general window; results
+    # are exact
+    real_case(oz, "N", "T", 70, 9, 33, s, "ints", check_bound=False)
+    complex_case(oz, "T", "N", 37, 5, 21, s, "ints", check_bound=False)
+
+
 @pytest.mark.parametrize("s", [8, 12, 16, 18, 24])
 def test_chunks(oz, s):
     real_case(oz, "T", "N", 7, 5, 70001, s, "phi", beta=1.0, check_bound=False)
