@@ -4,6 +4,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <map>
 #include <numeric>
 #include <stdexcept>
 #include <string>
@@ -46,6 +47,7 @@ BatchPlan::BatchPlan(Engine& eng, std::vector<GemmDesc> descs, const std::vector
     struct P {
         Plan plan;
         k::Tile tile;
+        int ftile;  // tile of the fused GEMM + CRT kernel, 0: separate kernels
         int64_t kp, kch, mpad, npad, planeA, planeB, planeR;
         size_t oD, oE, oPA, oPB, oA, oB, oR;
     };
@@ -57,6 +59,7 @@ BatchPlan::BatchPlan(Engine& eng, std::vector<GemmDesc> descs, const std::vector
         off = align_up(off + bytes, 256);
         return o;
     };
+    std::map<std::pair<int, int>, double> rounds;  // of the fused launches: (tile, limbs) -> tiles / slots
     for (size_t i = 0; i < np; ++i) {
         const GemmDesc& g = d_[i];
         if (g.m == 0 || g.n == 0) continue;
@@ -72,6 +75,17 @@ BatchPlan::BatchPlan(Engine& eng, std::vector<GemmDesc> descs, const std::vector
         if (tiles.empty() || tiles[i] <= 0) q.tile = eng_.pick_tile(g.m, g.n, k_chunk_len(q.kp), planes);
         else k::tile_from_code(tiles[i], q.tile);
         tile_codes_[i] = k::tile_code(q.tile);
+        q.ftile = fused_batch_tile(q.tile, q.kp, q.kch, planes);
+        if (q.ftile)
+            rounds[{q.ftile, q.plan.NL}] += static_cast<double>(round_up(g.m, q.ftile)) * round_up(g.n, q.ftile) /
+                                            (q.ftile * q.ftile * fused_per_cu(q.ftile, planes) * eng_.compute_units());
+        work.push_back(i);
+    }
+    for (size_t i : work) {
+        const GemmDesc& g = d_[i];
+        P& q = pp[i];
+        const int planes = s_[i];
+        if (q.ftile && rounds[{q.ftile, q.plan.NL}] < kFusedRounds) q.ftile = 0;
         q.mpad = round_up(g.m, k::tile_m(q.tile));
         q.npad = round_up(g.n, k::tile_n(q.tile));
         q.planeA = q.mpad * q.kp;
@@ -83,8 +97,7 @@ BatchPlan::BatchPlan(Engine& eng, std::vector<GemmDesc> descs, const std::vector
         q.oPB = carve(k::scale_partial_elems(g.n, g.k, g.tb == Op::N) * 8);
         q.oA = carve(static_cast<size_t>(planes) * q.planeA);
         q.oB = carve(static_cast<size_t>(planes) * q.planeB);
-        q.oR = carve(static_cast<size_t>(q.kch) * planes * q.planeR);
-        work.push_back(i);
+        q.oR = carve(q.ftile ? 0 : static_cast<size_t>(q.kch) * planes * q.planeR);
     }
     const size_t data_bytes = off;
 
@@ -93,6 +106,7 @@ BatchPlan::BatchPlan(Engine& eng, std::vector<GemmDesc> descs, const std::vector
     std::vector<k::SplitArgs> pj;
     std::vector<k::GemmJob> gj;
     std::vector<k::CrtArgs> cj;
+    std::vector<k::FusedJob> fj;
     std::vector<size_t> by_cost = work;
     if (opt_.largest_first)
         std::stable_sort(by_cost.begin(), by_cost.end(), [&](size_t a, size_t b) {
@@ -107,6 +121,7 @@ BatchPlan::BatchPlan(Engine& eng, std::vector<GemmDesc> descs, const std::vector
         pj.clear();
         gj.clear();
         cj.clear();
+        fj.clear();
         for (size_t i : work) {
             const GemmDesc& g = d_[i];
             const P& q = pp[i];
@@ -135,6 +150,7 @@ BatchPlan::BatchPlan(Engine& eng, std::vector<GemmDesc> descs, const std::vector
                 a.tab = tabs + s_[i];
                 pj.push_back(a);
             }
+            if (q.ftile) continue;
             k::CrtArgs c{};
             c.R = reinterpret_cast<const uint8_t*>(base + q.oR);
             c.plane_r = q.planeR;
@@ -160,6 +176,31 @@ BatchPlan::BatchPlan(Engine& eng, std::vector<GemmDesc> descs, const std::vector
         }
         for (size_t i : by_cost) {
             const P& q = pp[i];
+            if (q.ftile) {
+                const GemmDesc& g = d_[i];
+                k::FusedArgs f{};
+                f.A = reinterpret_cast<const int8_t*>(base + q.oA);
+                f.B = reinterpret_cast<const int8_t*>(base + q.oB);
+                f.kp = q.kp;
+                f.plane_a = q.planeA;
+                f.plane_b = q.planeB;
+                f.tiles_m = static_cast<int>(q.mpad / q.ftile);
+                f.tiles_n = static_cast<int>(q.npad / q.ftile);
+                f.s = s_[i];
+                f.nl = q.plan.NL;
+                f.up = q.plan.up();
+                f.tab = tabs + s_[i];
+                f.D = reinterpret_cast<const int32_t*>(base + q.oD);
+                f.E = reinterpret_cast<const int32_t*>(base + q.oE);
+                f.C = g.C;
+                f.mb = g.m;
+                f.nb = g.n;
+                f.ldc = g.ldc;
+                f.ar = g.alpha;
+                f.br = g.beta;
+                fj.push_back({q.ftile, f});
+                continue;
+            }
             for (int64_t c = 0; c < q.kch; ++c) {
                 k::GemmArgs a{};
                 a.A = reinterpret_cast<const int8_t*>(base + q.oA);
@@ -184,14 +225,16 @@ BatchPlan::BatchPlan(Engine& eng, std::vector<GemmDesc> descs, const std::vector
         split_.clear();
         gemm_.clear();
         crt_.clear();
+        fused_.clear();
         k::prep_scale(scale_, sj);
         k::prep_split(split_, pj);
         k::prep_gemm(gemm_, gj);
         k::prep_crt(crt_, cj);
+        k::prep_fused(fused_, fj);
     };
     build(nullptr);
     size_t tables = 0;
-    for (auto* v : {&scale_, &split_, &gemm_, &crt_})
+    for (auto* v : {&scale_, &split_, &gemm_, &crt_, &fused_})
         for (const k::GroupedLaunch& g : *v)
             tables += align_up(g.items.size(), 256) + align_up(g.start.size() * 4, 256) +
                       align_up(g.owner.size() * 4, 256);
@@ -210,7 +253,7 @@ BatchPlan::BatchPlan(Engine& eng, std::vector<GemmDesc> descs, const std::vector
     // upload the tables (once; the captured graph only reads them)
     size_t toff = data_bytes;
     std::vector<std::byte> host(tables);
-    for (auto* v : {&scale_, &split_, &gemm_, &crt_})
+    for (auto* v : {&scale_, &split_, &gemm_, &crt_, &fused_})
         for (k::GroupedLaunch& g : *v) {
             std::memcpy(host.data() + (toff - data_bytes), g.items.data(), g.items.size());
             g.d_items = ws_ + toff;
@@ -259,7 +302,7 @@ BatchPlan::~BatchPlan() {
 
 int BatchPlan::launches() const {
     int n = static_cast<int>(special_.size());
-    for (auto* v : {&scale_, &split_, &crt_}) n += static_cast<int>(v->size());
+    for (auto* v : {&scale_, &split_, &crt_, &fused_}) n += static_cast<int>(v->size());
     for (const k::GroupedLaunch& g : gemm_) n += k::gemm_grouped_launches(g, opt_.persistent);
     return n;
 }
@@ -275,19 +318,13 @@ void BatchPlan::enqueue(hipStream_t st) {
         k::launch_gemm_grouped(st, gemm_[i], counters_ + k::kGemmCounters * i, eng_.compute_units(),
                                opt_.persistent);
     for (const k::GroupedLaunch& g : crt_) k::launch_crt_grouped(st, g);
+    for (const k::GroupedLaunch& g : fused_) k::launch_fused_grouped(st, g);
 }
 
 void BatchPlan::run(hipStream_t st) {
     if (exec_) hip_check(hipGraphLaunch(exec_, st), "batch graph launch");
     else enqueue(st);
     hip_check(hipGetLastError(), "batch launch");
-}
-
-void BatchPlan::run_gemm_only(hipStream_t st) {
-    for (size_t i = 0; i < gemm_.size(); ++i)
-        k::launch_gemm_grouped(st, gemm_[i], counters_ + k::kGemmCounters * i, eng_.compute_units(),
-                               opt_.persistent);
-    hip_check(hipGetLastError(), "batch gemm launch");
 }
 
 namespace {

@@ -54,7 +54,6 @@ public:
     BatchPlan& operator=(const BatchPlan&) = delete;
 
     void run(hipStream_t st);           // enqueue the whole batch on st
-    void run_gemm_only(hipStream_t st); // the grouped INT8 GEMM launches alone (autotuning)
     const std::vector<int>& moduli() const { return s_; }
     const std::vector<int>& tiles() const { return tile_codes_; }  // k::tile_code per problem (0: no GEMM)
     size_t workspace_bytes() const { return ws_size_; }
@@ -68,7 +67,7 @@ private:
     BatchOptions opt_;
     std::vector<int> s_, tile_codes_;
     std::vector<size_t> special_;  // k == 0 or alpha == 0: C = beta C
-    std::vector<k::GroupedLaunch> scale_, split_, gemm_, crt_;
+    std::vector<k::GroupedLaunch> scale_, split_, gemm_, crt_, fused_;
     std::byte* ws_ = nullptr;
     size_t ws_size_ = 0;
     uint32_t* counters_ = nullptr;

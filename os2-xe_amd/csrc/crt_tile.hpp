@@ -23,8 +23,9 @@ namespace k {
 typedef int crt_v4i __attribute__((ext_vector_type(4)));
 typedef int crt_v16i __attribute__((ext_vector_type(16)));
 
-// digits and constants of one modulus set, held by a wave for all its entries
-template <int NL>
+// digits and constants of one modulus set, held by a wave for all its entries.  SYM: the residues come as
+// signed bytes in [-128, 127] (any representative), else as bytes in [0, m).
+template <int NL, bool SYM = false>
 struct CrtTile {
     static constexpr int SC = 4 * NL;  // moduli of NL words of M: at most 4 NL
     crt_v4i a[NL > 4 ? 2 : 1][2];      // [moduli 0 .. 15, 16 .. 31][lanes 0 .. 31, 32 .. 63]
@@ -44,7 +45,7 @@ struct CrtTile {
         for (int b = 0; b < 4; ++b) {
             const crt_v4i c = *reinterpret_cast<const crt_v4i*>(&tab->Kc[8 * b + 4 * half]);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) init[4 * b + i] = c[i];
+            for (int i = 0; i < 4; ++i) init[4 * b + i] = SYM ? 0 : c[i];
         }
     }
 
@@ -60,10 +61,10 @@ struct CrtTile {
             const uint32_t hi01 = __builtin_amdgcn_perm(r[4 * g + 1], r[4 * g], 0x07030602u);
             const uint32_t lo23 = __builtin_amdgcn_perm(r[4 * g + 3], r[4 * g + 2], 0x05010400u);
             const uint32_t hi23 = __builtin_amdgcn_perm(r[4 * g + 3], r[4 * g + 2], 0x07030602u);
-            b[0][g] = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u) ^ 0x80808080u;
-            b[1][g] = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u) ^ 0x80808080u;
-            b[2][g] = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u) ^ 0x80808080u;
-            b[3][g] = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u) ^ 0x80808080u;
+            b[0][g] = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u) ^ (SYM ? 0u : 0x80808080u);
+            b[1][g] = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u) ^ (SYM ? 0u : 0x80808080u);
+            b[2][g] = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u) ^ (SYM ? 0u : 0x80808080u);
+            b[3][g] = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u) ^ (SYM ? 0u : 0x80808080u);
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -88,7 +89,7 @@ struct CrtTile {
                 }
             }
             uint32_t w[NL];
-            math::crt_words<NL>(tb, [&](int x) { return row[x]; }, w);
+            math::crt_words<NL, SYM>(tb, [&](int x) { return row[x]; }, w);
             out(e, w);
         }
     }

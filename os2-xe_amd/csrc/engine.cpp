@@ -174,13 +174,21 @@ StageTimes Engine::stage_times() {
     }
     for (size_t i = 0; i < marks_.size(); ++i) {
         const uint64_t* w = ts.data() + i * kW;
-        const uint64_t b = w[0], e = *std::max_element(w + 1, w + kW);
+        const uint64_t b = w[0], e = *std::max_element(w + 1, w + 1 + k::kStampEnds);
         const double ms = e > b ? static_cast<double>(e - b) / static_cast<double>(clock_khz_) : 0.0;
         switch (marks_[i]) {
             case Stage::Scale: t.scale_ms += ms; break;
             case Stage::Split: t.split_ms += ms; break;
             case Stage::Gemm: t.gemm_ms += ms; break;
             case Stage::Crt: t.crt_ms += ms; break;
+            case Stage::Fused: {
+                // divided as the launch's first workgroup divided its time
+                const uint64_t crt0 = w[k::kStampInner], end = w[k::kStampInner + 1];
+                const double f = end > crt0 && crt0 > b ? static_cast<double>(end - crt0) / static_cast<double>(end - b) : 0.0;
+                t.gemm_ms += ms * (1.0 - f);
+                t.crt_ms += ms * f;
+                break;
+            }
         }
     }
     return t;
@@ -334,6 +342,12 @@ void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, doubl
         StageTimer timer(*this, st);
         launch(k::Stream(on, timed ? &timer : nullptr));
     };
+    // Column blocks of a panel pair: with more than one, the B blocks are split and the CRTs run on
+    // the second stream while the GEMM of the next block runs on the caller's (a fixed workspace
+    // keeps the one-stream order: it records no events)
+    const int nblocks = fixed_ws ? 1 : overlap_blocks();
+    // GEMMs and CRT in one kernel (its tile), or 0
+    const int ftile = nblocks > 1 ? 0 : fused_tile(cs, L, mb, nb);
     // split of `rows` rows of op(X) starting at row r0 into the planes from plane row prow
     auto split_rows = [&](const k::Stream& on, bool is_b, int64_t r0, int64_t rows, int64_t prow) {
         const Op op = is_b ? tb : ta;
@@ -344,7 +358,7 @@ void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, doubl
         sp.X = sp.kcontig ? X + cw * r0 * ldx : X + cw * r0;
         sp.ldx = ldx;
         sp.rows = rows;
-        sp.rows_pad = round_up(rows, is_b ? L.TN : L.TM);
+        sp.rows_pad = round_up(rows, ftile ? ftile : is_b ? L.TN : L.TM);
         sp.k = k;
         sp.kp = kp;
         sp.ex = (is_b ? E : D) + r0;
@@ -418,16 +432,36 @@ void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, doubl
         ca.tab = tab;
         k::crt(on, ca);
     };
+    // GEMMs and CRT of rows i0 .. i0 + rows by columns j0 .. j0 + cols (the whole panel pair) in one launch
+    auto fused_block = [&](const k::Stream& on, int64_t i0, int64_t rows, int64_t j0, int64_t cols) {
+        k::FusedArgs f{};
+        f.A = Ap;
+        f.B = Bp;
+        f.kp = kp;
+        f.plane_a = L.planeA;
+        f.plane_b = L.planeB;
+        f.tiles_m = static_cast<int>((rows + ftile - 1) / ftile);
+        f.tiles_n = static_cast<int>((cols + ftile - 1) / ftile);
+        f.s = s;
+        f.nl = p.NL;
+        f.up = p.up();
+        f.tab = tab;
+        f.D = D + i0;
+        f.E = E + j0;
+        f.C = C + i0 + j0 * ldc;
+        f.mb = rows;
+        f.nb = cols;
+        f.ldc = ldc;
+        f.ar = ar;
+        f.br = br;
+        k::fused(on, ftile, f);
+    };
 
     // scale: exponents of the rows of op(A) and the columns of op(B) (hpp:974-989)
     timed_on(Stage::Scale, stream_, [&](const k::Stream& on) {
         k::scale(on, A, lda, m, k, ta != Op::N, cplx, tk, PA, D);
         k::scale(on, B, ldb, n, k, tb == Op::N, cplx, tk, PB, E);
     });
-    // Column blocks of a panel pair: with more than one, the B blocks are split and the CRTs run on
-    // the second stream while the GEMM of the next block runs on the caller's (a fixed workspace
-    // keeps the one-stream order: it records no events)
-    const int nblocks = fixed_ws ? 1 : overlap_blocks();
     bool forked = false;
     for (int64_t j0 = 0; j0 < n; j0 += nb) {
         const int64_t nbj = std::min(nb, n - j0);
@@ -438,6 +472,10 @@ void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, doubl
             const int64_t mbi = std::min(mb, m - i0);
             if (ti.pm > 1 || j0 == 0) timed_on(Stage::Split, stream_, [&](const k::Stream& on) { split_rows(on, false, i0, mbi, 0); });
             if (nblk == 1) {
+                if (ftile) {
+                    timed_on(Stage::Fused, stream_, [&](const k::Stream& on) { fused_block(on, i0, mbi, j0, nbj); });
+                    continue;
+                }
                 timed_on(Stage::Gemm, stream_, [&](const k::Stream& on) { gemm_block(on, mbi, 0, nbj); });
                 timed_on(Stage::Crt, stream_, [&](const k::Stream& on) { crt_block(on, i0, mbi, j0, 0, nbj); });
                 continue;

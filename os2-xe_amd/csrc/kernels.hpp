@@ -20,7 +20,7 @@ namespace oz2 {
 namespace k {
 
 // Source of a timed launch's stamps (stage times): kStampWords device words of its own.
-inline constexpr uint32_t kStampWords = 16;
+inline constexpr uint32_t kStampWords = 16, kStampEnds = 13, kStampInner = 14;
 struct LaunchTimer {
     virtual uint64_t* next() = 0;
 
@@ -40,8 +40,8 @@ struct Stream {
 };
 
 #if defined(__HIPCC__)
-// Begin of a kernel in ts[0], ends in the other words (ts null: not timed).  Workgroups start in order,
-// so the first one stamps the begin; the end is the latest of the last kStampWords - 1 workgroups, each
+// Begin of a kernel in ts[0], ends in the words from 1 on (ts null: not timed).  Workgroups start in order,
+// so the first one stamps the begin; the end is the latest of the last kStampEnds workgroups, each
 // with a word of its own (one word for all of 256 workgroups, by atomicMax, cost 1.5 us a launch).  The
 // clock only grows, so words left by an earlier launch do not count.
 struct Stamp {
@@ -52,7 +52,11 @@ struct Stamp {
         if (ts && b == 0 && threadIdx.x == 0) ts[0] = wall_clock64();
     }
     __device__ __forceinline__ void end() const {
-        if (ts && n - b < kStampWords && threadIdx.x == 0) ts[n - b] = wall_clock64();
+        if (ts && n - b <= kStampEnds && threadIdx.x == 0) ts[n - b] = wall_clock64();
+    }
+    // a moment inside the first workgroup (a kernel of two stages)
+    __device__ __forceinline__ void inner(int i) const {
+        if (ts && b == 0 && threadIdx.x == 0) ts[kStampInner + i] = wall_clock64();
     }
 };
 
@@ -152,18 +156,20 @@ struct CrtArgs {
 };
 void crt(const Stream& st, const CrtArgs& a);
 
-// ---- GEMMs of all planes and the CRT of a tile in one workgroup -------------------
+// ---- INT8 GEMMs of all planes and the CRT of a tile in one workgroup --------------
+// a real product of one k-chunk; tile 128 or 64 (square): the planes are padded to it
 struct FusedArgs {
-    const int8_t *A, *B;
+    const int8_t *A, *B;      // planes of op(A), op(B)
     int64_t kp, plane_a, plane_b;
-    int tiles_m, tiles_n, s, nl;
+    int tiles_m, tiles_n;
+    int s, nl, up;            // moduli, Plan::NL, Plan::up()
     const TabSet* tab;
-    const int32_t *D, *E;
-    double* C;
-    int64_t mb, nb, ldc;
+    const int32_t *D, *E;     // exponents per row, per column (offset to the panel)
+    double* C;                // offset to the panel
+    int64_t mb, nb, ldc;      // panel extent
     double ar, br;
 };
-void fused(const Stream& st, int code, const FusedArgs& a);
+void fused(const Stream& st, int tile, const FusedArgs& a);
 
 // ---- Ozaki Scheme I (the accuracy benchmark's comparison baseline) --------------------
 // L balanced base-128 digits of RNE(op(X)[r][p] 2^ex[r]) per element into one extended
@@ -209,10 +215,15 @@ struct GemmJob {
     Tile tile;
     GemmArgs args;
 };
+struct FusedJob {
+    int tile;
+    FusedArgs args;
+};
 void prep_scale(std::vector<GroupedLaunch>& out, const std::vector<ScaleJob>& jobs);
 void prep_split(std::vector<GroupedLaunch>& out, const std::vector<SplitArgs>& jobs);
 void prep_gemm(std::vector<GroupedLaunch>& out, const std::vector<GemmJob>& jobs);
 void prep_crt(std::vector<GroupedLaunch>& out, const std::vector<CrtArgs>& jobs);
+void prep_fused(std::vector<GroupedLaunch>& out, const std::vector<FusedJob>& jobs);
 bool launch_scale_split_grouped(hipStream_t st, const GroupedLaunch& g);
 // persistent (128 x 128 and 64 x 64 tiles at their blocks per CU, 256 x 128 at one per CU):
 // min(blocks, cus x that) workgroups pull tiles through counter[0 .. kGemmCounters) (reset
@@ -222,6 +233,7 @@ inline constexpr int kGemmCounters = 8;
 void launch_gemm_grouped(hipStream_t st, const GroupedLaunch& g, uint32_t* counter, int cus, bool persistent);
 int gemm_grouped_launches(const GroupedLaunch& g, bool persistent);  // kernels launch_gemm_grouped enqueues
 void launch_crt_grouped(hipStream_t st, const GroupedLaunch& g);
+void launch_fused_grouped(hipStream_t st, const GroupedLaunch& g);
 
 }  // namespace k
 }  // namespace oz2

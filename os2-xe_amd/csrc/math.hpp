@@ -301,10 +301,11 @@ OZ2_HD void crt_carry(Tab tb, uint32_t uq, Limb limb, uint32_t (&w)[NL]) {
 }
 
 // from the rows of the matrix product: limb l is x[2l] + 256 x[2l+1] (24 * 128 * 128 * 257 + 24 * 128 * 65535
-// + 24 * 255 * 65535 < 2^30); the 2^15 of q's rounding is in Kc
-template <int NL, typename Tab, typename Row>
+// + 24 * 255 * 65535 < 2^30); the 2^15 of q's rounding is in
+// Kc, which signed residues (SYM, of any representative in [-128, 127]) do without: q may then be negative
+template <int NL, bool SYM = false, typename Tab, typename Row>
 OZ2_HD void crt_words(Tab tb, Row x, uint32_t (&w)[NL]) {
-    const uint32_t uq = static_cast<uint32_t>(x(4 * NL)) + ((static_cast<uint32_t>(x(4 * NL + 1)) +
+    const uint32_t uq = (SYM ? 0x8000u : 0u) + static_cast<uint32_t>(x(4 * NL)) + ((static_cast<uint32_t>(x(4 * NL + 1)) +
                                                             (static_cast<uint32_t>(x(4 * NL + 2)) << 8)) << 8);
     crt_carry<NL>(tb, uq, [&](int l) { return static_cast<uint32_t>(x(2 * l)) + (static_cast<uint32_t>(x(2 * l + 1)) << 8); }, w);
 }

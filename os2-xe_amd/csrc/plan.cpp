@@ -164,6 +164,7 @@ void make_tabsets(TabSet* out) {
             tb.h2[t] = 2 * h;
             for (int j = 0; j < 16; ++j) tb.c8[t][j >> 2] |= static_cast<uint32_t>(pow2_mod(8 * j, m)) << (8 * (j & 3));
             tb.c30[t] = m == 256 ? 0 : m * static_cast<uint32_t>(((uint64_t{1} << 30) + m - 1) / m);
+            tb.mg[t] = m == 256 ? 0 : static_cast<uint32_t>(((uint64_t{1} << 39) + m - 1) / m);
             // balanced digits in [-128, 127]; the carry out of the last one is dropped (mod 2^(32 NL))
             auto digits = [&](auto byte, int row0, int n) {
                 int carry = 0;

@@ -95,6 +95,7 @@ struct TabSet {
     uint32_t h2[kMaxModuli];                // 2 h
     uint32_t c8[kMaxModuli][4];             // bytes 2^(8 j) mod m, j = 0..15, four to a word (low first)
     uint32_t c30[kMaxModuli];               // m * ceil(2^30 / m) (GEMM residue epilogue offset; 0 for m = 256)
+    uint32_t mg[kMaxModuli];                // ceil(2^39 / m): exact quotients of values below 2^31 (0 for m = 256)
     // CRT (hpp:222-236), of C' 2^up with up = 32 NL - bits(M): its sign bit is then the top bit of NL words
     // whatever M is.  As an int8 matrix product over the moduli row r of the sums is
     // sum_t (r_t - 128) Wd[r][t] + Kc[r].  Rows 0 .. 4 NL - 1 are the balanced base-256 digits of

@@ -81,6 +81,37 @@ double gemm_seconds(const CallShape& c, const Layout& L, int64_t rows, int64_t c
 }
 }  // namespace
 
+namespace {
+// longest k at which 128 x 128 tiles of the fused kernel are ahead of the separate ones in full rounds, us on
+// MI355X, separate / fused: 4096 x 4096 x 768 s = 8 192 / 181, x 1024 220 / 227; x 1024 s = 16 439 / 410;
+// 2048 x 2048 x 1024 s = 16 109 / 93, x 1536 139 / 129, 4096 x 4096 x 1024 s = 24 679 / 676
+int64_t fused_k(int s) { return limbs_for(s) == 2 ? 512 : limbs_for(s) == 6 ? 768 : 1024; }
+}  // namespace
+
+int fused_tile(const CallShape& c, const Layout& L, int64_t mb, int64_t nb) {
+    if (c.cplx || L.kch != 1 || c.per_plane || c.forced_tile != -1) return 0;
+    const int nl = limbs_for(c.s);
+    const double area = static_cast<double>(mb) * static_cast<double>(nb), cus = c.cus;
+    // 64 x 64 tiles, three (two) per CU, pay at short k, where the separate path is mostly traffic, also with
+    // ragged rounds; with less than 0.6 of a round (1024 x 1024 x 256 s = 16: 19.3 / 19.3 us) nothing is gained.
+    // Separate / 64 tiles: 1408 x 1408 x 256 s = 16 35 / 26, 3000 x 3000 x 256 131 / 97, x 1024 241 / 268,
+    // 2304 x 2304 s = 20 k = 128 81 / 71, k = 256 92 / 90.  Above 20 moduli the 128 tiles spill: 8192 x 8192
+    // x 128 s = 24 1261 / 891, 128 tiles 1084.
+    const bool t64 = L.kp <= (nl > 4 ? 128 : 256) && area >= 0.6 * 64 * 64 * fused_per_cu(64, c.s) * cus;
+    if (nl == 6 && t64) return 64;
+    // 128 x 128 tiles, one per CU, want their rounds full: the fused rounds are long (s planes each), the
+    // separate path's are a plane each.  3000 x 3000 x 256 s = 16 (72 %) 131 / 118, x 1024 241 / 253; s = 8
+    // x 256 72 / 80; 2816 x 2816 (95 %) x 256 s = 8 61 / 59.
+    const double rounds = std::ceil(static_cast<double>(ceil_div(mb, 128)) * static_cast<double>(ceil_div(nb, 128)) / cus);
+    if (L.kp <= fused_k(c.s) && area >= 0.8 * 128 * 128 * cus * rounds && L.TM % 128 == 0 && L.TN % 128 == 0) return 128;
+    return t64 ? 64 : 0;
+}
+
+int fused_batch_tile(k::Tile tile, int64_t kp, int64_t kch, int s) {
+    if (kch != 1 || kp > fused_k(s)) return 0;
+    return tile == k::Tile::T64 ? 64 : 128;
+}
+
 bool same_call(const CallShape& a, const CallShape& b) {
     return a.m == b.m && a.n == b.n && a.k == b.k && a.s == b.s && a.cplx == b.cplx && a.partial_a == b.partial_a &&
            a.partial_b == b.partial_b && a.cus == b.cus && a.pad_planes == b.pad_planes && a.pow2 == b.pow2 &&

@@ -73,6 +73,18 @@ k::Tile pick_tile(int64_t mb, int64_t nb, int64_t klen, int planes, int forced_c
 Layout layout(const CallShape& c, int64_t mb, int64_t nb);
 // modelled seconds of the whole call with mb x nb panels on MI355X
 double panel_cost(const CallShape& c, int64_t mb, int64_t nb);
+// Tile of the fused GEMM + CRT kernel for panels of mb x nb, 128 or 64, or 0 where the separate kernels are
+// ahead (or the product is complex or has several k-chunks); the panels' planes are laid out as L
+int fused_tile(const CallShape& c, const Layout& L, int64_t mb, int64_t nb);
+// the same for a product in a batch, whose launches the other products help to fill
+int fused_batch_tile(k::Tile tile, int64_t kp, int64_t kch, int s);
+// Products of a batch that would fill less than this many rounds of a fused launch take the separate kernels:
+// a workgroup runs long (s planes), and a launch of less than one round is all tail.  MI355X, all fused / from
+// one round on / all separate, us: 64 products of 64 .. 1024 620 / 561 / 560, 16 of 64 .. 2048 420 / 342 / 342,
+// 256 of 64 .. 512 713 / 695 / 834, 256 of 128 .. 1024 2308 / 2310 / 2682, 8 of 1024 446 / 446 / 471.
+inline constexpr double kFusedRounds = 1.0;
+// workgroups of the fused kernel that a CU holds
+constexpr int fused_per_cu(int tile, int s) { return tile == 128 ? 1 : s > 16 ? 2 : 3; }
 // cheapest panels whose workspace fits `limit`; std::runtime_error if none does
 TileInfo plan_tiling(const CallShape& c, size_t limit);
 
