@@ -173,9 +173,8 @@ __device__ __forceinline__ void fused_tile(const FusedArgs& p, uint32_t tm, uint
             ex[x] = x < TM ? p.D[min(static_cast<int64_t>(tm) * TM + x, p.mb - 1)]
                            : p.E[min(static_cast<int64_t>(tn) * TN + x - TM, p.nb - 1)];
     }
-    // The sums start at c30 + 128: u = x + c30 + 128 < 2^31 (|x| < 2^30 - 2^21), and with mg = ceil(2^39 / m)
-    // u mg >> 39 is floor(u / m) exactly (u (mg m - 2^39) < 2^31 2^8).  The residue of x + 128, xored with
-    // 0x80, is x's as a signed byte in [-128, 126], as CrtTile takes it; m = 256 has mg = 0 and c30 = 0.
+    // The sums start at c30 + 128: the residue of x + 128, xored with 0x80, is x's as a signed byte in
+    // [-128, 126], as CrtTile takes it.
     uint32_t c30 = tb->c30[0] + 128;
     for (int t = 0; t < S; ++t) {
         const uint32_t m = tb->m[t], mg = tb->mg[t];
@@ -194,7 +193,7 @@ __device__ __forceinline__ void fused_tile(const FusedArgs& p, uint32_t tm, uint
 #pragma unroll
             for (int b = 0; b < 4; ++b) {
                 const uint32_t u = static_cast<uint32_t>(acc[x / 4 / FN][x / 4 % FN][4 * (x % 4) + b]);
-                r[b] = mad_i24(static_cast<int32_t>(__umulhi(u, mg) >> 7), -static_cast<int32_t>(m), u);
+                r[b] = residue_word(u, m, mg);
             }
             w[x] = pack_lo_bytes(r[0], r[1], r[2], r[3]) ^ 0x80808080u;
         }

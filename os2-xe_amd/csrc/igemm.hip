@@ -29,6 +29,11 @@
 // 256 x 128 tiles run two per CU with NS = 3 (72 KB each): with short k loops
 // the residue epilogue of one workgroup then overlaps the MFMAs of the other.
 //
+// The large tiles are bound by power: a loop of this instruction on random registers alone runs at 3.2 Pop/s,
+// on constant ones at 4.4 (8192^3, 16 planes: 2.55).  So consecutive MFMAs share an operand: the column blocks
+// go back and forth under the row blocks (register loop 3.20 -> 3.27 Pop/s; 4096 x 4096 x 1536 s = 16 444 ->
+// 434 us, 4096^3 s = 16 940 -> 929).
+//
 // MFMA 32x32x32 i8 operand layout (checked on gfx950): lane l holds row
 // (l mod 32) of A / column (l mod 32) of B with 16 k-bytes at k = 16*(l/32);
 // accumulator v of lane l is C[8*(v/4) + 4*(l/32) + v%4][l mod 32].
@@ -75,6 +80,14 @@ __device__ __forceinline__ uint32_t plane_xcd_remap(uint32_t b, uint32_t tiles, 
     return plane * tiles + (r & 7) * (tiles >> 3) + (r >> 3);
 }
 
+__device__ __forceinline__ int plane_modulus(const GemmArgs& p, uint32_t plane) {
+    return static_cast<int>((static_cast<uint32_t>(p.plane0) + plane) % static_cast<uint32_t>(p.s));
+}
+
+// Exposed where one workgroup fills the CU, so counted in VALU instructions: 3 an entry and 3 permutes for
+// four (6 with a fold of the high half before the quotient: 8192^3 s = 16 7.00 -> 6.93 ms, 4096^3 s = 8
+// 512 -> 498 us, 777 x 1023 x 515 18.0 -> 16.8, 512^3 5.6 -> 5.2).
+//
 // Residues of one wave tile (WTM x WTN) staged through LDS: 4 residues per
 // 32-bit LDS store into a [col][row] byte tile whose 16-byte chunks are
 // XOR-permuted by column, then 16-byte global stores that write whole runs of
@@ -83,37 +96,24 @@ template <int FM, int FN>
 __device__ __forceinline__ void residue_epilogue(const GemmArgs& p, v16i (&acc)[FM][FN], uint32_t plane,
                                                  int64_t row0, int64_t col0, char* wlds, int lane) {
     constexpr int WTM = FM * 32, WTN = FN * 32, NCH = WTM / 16;
-    const int t = static_cast<int>((static_cast<uint32_t>(p.plane0) + plane) % static_cast<uint32_t>(p.s));
+    const int t = plane_modulus(p, plane);
     const auto tb = const_tab(p.tab);
-    const uint32_t m = tb->m[t];
+    const uint32_t m = tb->m[t], mg = tb->mg[t];
     const int fr = lane & 31, fc = lane >> 5;
     auto lds_at = [&](int c, int r) { return wlds + c * WTM + ((((r >> 4) ^ (c & (NCH - 1))) << 4) | (r & 15)); };
-    if (m == 256) {
 #pragma unroll
-        for (int i = 0; i < FM; ++i)
+    for (int i = 0; i < FM; ++i)
 #pragma unroll
-            for (int j = 0; j < FN; ++j)
+        for (int j = 0; j < FN; ++j) {
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const uint32_t w = pack_lo_bytes(static_cast<uint32_t>(acc[i][j][4 * q]), static_cast<uint32_t>(acc[i][j][4 * q + 1]),
-                                                     static_cast<uint32_t>(acc[i][j][4 * q + 2]), static_cast<uint32_t>(acc[i][j][4 * q + 3]));
-                    *reinterpret_cast<uint32_t*>(lds_at(j * 32 + fr, i * 32 + 8 * q + 4 * fc)) = w;
-                }
-    } else {
-        const uint32_t mu = tb->mu[t], c16 = tb->c16[t], c30 = tb->c30[t];
+            for (int q = 0; q < 4; ++q) {
+                uint32_t r[4];
 #pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-            for (int j = 0; j < FN; ++j) {
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    uint32_t r[4];
-#pragma unroll
-                    for (int b = 0; b < 4; ++b) r[b] = residue_m30(static_cast<uint32_t>(acc[i][j][4 * q + b]), m, mu, c16, c30);
-                    *reinterpret_cast<uint32_t*>(lds_at(j * 32 + fr, i * 32 + 8 * q + 4 * fc)) = pack_lo_bytes(r[0], r[1], r[2], r[3]);
-                }
+                for (int b = 0; b < 4; ++b) r[b] = residue_word(static_cast<uint32_t>(acc[i][j][4 * q + b]), m, mg);
+                *reinterpret_cast<uint32_t*>(lds_at(j * 32 + fr, i * 32 + 8 * q + 4 * fc)) = pack_lo_bytes(r[0], r[1], r[2], r[3]);
             }
-    }
+            __builtin_amdgcn_sched_barrier(0);  // one block's words at a time (256 x 256: spills otherwise)
+        }
     __syncthreads();
     uint8_t* Rb = p.R + static_cast<int64_t>(plane) * p.plane_r;
     constexpr int CPI = 64 / NCH;  // columns per pass
@@ -210,13 +210,15 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint32_t plane, uin
         offb[ks] = BM * KT + rb * 64 + (((2 * ks + fc) ^ ((rb >> 2) & 3)) << 4);
     }
 
+    // residues: the sums start at c30 (residue_word in math.hpp)
+    const int c30 = I32 ? 0 : static_cast<int>(const_tab(p.tab)->c30[plane_modulus(p, plane)]);
     v16i acc[FM][FN];
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0;
+            for (int v = 0; v < 16; ++v) acc[i][j][v] = c30;
     v4i fa0[2][FM], fb0[2][FN], fa1[2][FM], fb1[2][FN];
 
     // stage KT_ (clamped to the last one: past the end the DMA refills a
@@ -247,7 +249,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint32_t plane, uin
             _Pragma("unroll") for (int r = 0; r < NR; ++r) if (r * NMF / NR == u) OZ2_READ(NA, NB, KTR, r)       \
             __builtin_amdgcn_sched_barrier(0);                                                                   \
             {                                                                                                    \
-                const int ks = u / (FM * FN), i = (u / FN) % FM, j = u % FN;                                     \
+                const int ks = u / (FM * FN), i = (u / FN) % FM, j = i % 2 ? FN - 1 - u % FN : u % FN;\
                 acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(FA[ks][i], FB[ks][j], acc[i][j], 0, 0, 0);     \
             }                                                                                                    \
             __builtin_amdgcn_sched_barrier(0);                                                                   \

@@ -57,6 +57,9 @@ OZ2_HD uint32_t mulhi24(uint32_t a, uint32_t b) {
 #endif
 }
 
+// v_mul_hi_u32
+OZ2_HD uint32_t mulhi32(uint32_t a, uint32_t b) { return static_cast<uint32_t>((static_cast<uint64_t>(a) * b) >> 32); }
+
 // v_dot2_u32_u16: c + a.lo * b.lo + a.hi * b.hi (16-bit halves, no clamping)
 OZ2_HD uint32_t udot2(uint32_t a, uint32_t b, uint32_t c) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -235,22 +238,18 @@ OZ2_HD int32_t sym_value(const uint32_t (&a)[4], Tab tb, int t) {
     return static_cast<int32_t>(sym_residue<F>(a, tb, t));
 }
 
-// GEMM epilogue: int32 dot product x (as bits) of one k-chunk -> x mod m in [0, m),
-// m <= 255.  A chunk holds at most kMaxKChunk = 65408 k, so |x| <= 65408 * 2^14 <
-// 2^30 - 255, and with c30 = m ceil(2^30 / m) in [2^30, 2^30 + m) the value u = x + c30
-// lies in [0, 2^31) and keeps x's residue.  One v_mad_i32_i24 folds the high half:
-// y = u + (u >> 16)(c16 - 2^16) = (u >> 16) c16 + (u & 0xffff) <= (2^15 - 1) 254 + 65535
-// < 2^23, then y mod m by the exact quotient.
-OZ2_HD uint32_t residue_m30(uint32_t x, uint32_t m, uint32_t mu, uint32_t c16, uint32_t c30) {
-    const uint32_t u = x + c30;
-    const uint32_t y = mad_i24(static_cast<int32_t>(u >> 16), static_cast<int32_t>(c16) - 65536, u);
-    return mod_m23(y, m, mu);
+// GEMM epilogue: int32 dot product x of one k-chunk -> x mod m in [0, m), m <= 255.  A chunk holds at most
+// kMaxKChunk = 65408 k, so |x| <= 65408 * 2^14 <= 2^30 - 2^21, and with c30 = m ceil(2^30 / m) in
+// [2^30, 2^30 + m) the value u = x + c30 lies in [0, 2^31) and keeps x's residue; the sums start at c30, so u
+// is what the matrix cores leave.  With mg = ceil(2^39 / m), u mg / 2^39 = u/m + u e / (m 2^39), e < m < 2^8:
+// the excess stays below 1/m, so q = floor(u mg / 2^39) = floor(u/m).  q may exceed 23 bits, so only the low
+// byte of the returned word is u - q m.  m = 256 has mg = c30 = 0: the low byte of x.
+OZ2_HD uint32_t residue_word(uint32_t u, uint32_t m, uint32_t mg) {
+    return mad_i24(static_cast<int32_t>(mulhi32(u, mg) >> 7), -static_cast<int32_t>(m), u);
 }
 template <typename Tab>
 OZ2_HD uint32_t acc_residue(uint32_t x, Tab tb, int t) {
-    const uint32_t m = tb->m[t];
-    if (m == 256) return x & 0xFFu;
-    return residue_m30(x, m, tb->mu[t], tb->c16[t], tb->c30[t]);
+    return residue_word(x + tb->c30[t], tb->m[t], tb->mg[t]) & 0xFFu;
 }
 
 OZ2_HD double ldexp_(double v, int e) {

@@ -155,7 +155,6 @@ void make_tabsets(TabSet* out) {
             tb.m[t] = m;
             tb.mu[t] = static_cast<uint32_t>(((uint64_t{1} << 31) + m - 1) / m);
             tb.h[t] = h;
-            tb.c16[t] = pow2_mod(16, m);
             const int offs[3] = {62, 95, 104};
             for (int f = 0; f < 3; ++f) {
                 tb.off[f][t] = (m - pow2_mod(offs[f], m) + h) % m;

@@ -89,7 +89,6 @@ struct TabSet {
     uint32_t m[kMaxModuli];
     uint32_t mu[kMaxModuli];                // ceil(2^31 / m): exact quotients of values below 2^23 (mod_m23)
     uint32_t h[kMaxModuli];                 // (m - 1) / 2
-    uint32_t c16[kMaxModuli];               // 2^16 mod m
     uint32_t off[3][kMaxModuli];            // (m - 2^OFF mod m + h) mod m, OFF = 62, 95, 104 (limb_form 0, 1, 2)
     uint32_t offh[3][kMaxModuli];           // off - h (mod 2^32): start of the symmetric split's dot chain
     uint32_t h2[kMaxModuli];                // 2 h
