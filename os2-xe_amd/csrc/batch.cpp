@@ -139,6 +139,7 @@ BatchPlan::BatchPlan(Engine& eng, std::vector<GemmDesc> descs, const std::vector
                 a.rows_pad = which == 0 ? q.mpad : q.npad;
                 a.k = g.k;
                 a.kp = q.kp;
+                a.map = k::PlaneMap::of(q.tile, q.ftile, a.rows_pad, q.kp);
                 a.ex = which == 0 ? D : E;
                 a.P = reinterpret_cast<int8_t*>(base + (which == 0 ? q.oA : q.oB));
                 a.plane = which == 0 ? q.planeA : q.planeB;
@@ -205,7 +206,8 @@ BatchPlan::BatchPlan(Engine& eng, std::vector<GemmDesc> descs, const std::vector
                 k::GemmArgs a{};
                 a.A = reinterpret_cast<const int8_t*>(base + q.oA);
                 a.B = reinterpret_cast<const int8_t*>(base + q.oB);
-                a.kp = q.kp;
+                a.map_a = k::PlaneMap::of(q.tile, false, q.mpad, q.kp);
+                a.map_b = k::PlaneMap::of(q.tile, false, q.npad, q.kp);
                 a.plane_a = q.planeA;
                 a.plane_b = q.planeB;
                 a.plane_r = q.planeR;

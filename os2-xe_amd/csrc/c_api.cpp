@@ -480,6 +480,7 @@ int oz2_unit_split(void* stream, const double* X, int64_t ldx, int64_t rows, int
         a.kp = kp;
         a.ex = ex;
         a.P = planes;
+        a.map = oz2::k::PlaneMap::by_band(kp);
         a.plane = rows_pad * kp;
         a.group = static_cast<int64_t>(num_moduli) * a.plane;
         a.s = num_moduli;
@@ -538,7 +539,7 @@ int oz2_unit_gemm(void* stream, const int8_t* A, const int8_t* B, int64_t mpad, 
         a.A = A;
         a.B = B;
         a.R = R;
-        a.kp = kp;
+        a.map_a = a.map_b = oz2::k::PlaneMap::by_band(kp);
         a.plane_a = mpad * kp;
         a.plane_b = npad * kp;
         a.plane_r = ldr * npad;

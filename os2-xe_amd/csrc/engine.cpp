@@ -348,6 +348,7 @@ void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, doubl
     const int nblocks = fixed_ws ? 1 : overlap_blocks();
     // GEMMs and CRT in one kernel (its tile), or 0
     const int ftile = nblocks > 1 ? 0 : fused_tile(cs, L, mb, nb);
+    const k::PlaneMap map_a = k::PlaneMap::of(tile_, ftile, L.mpad, kp), map_b = k::PlaneMap::of(tile_, ftile, L.npad, kp);
     // split of `rows` rows of op(X) starting at row r0 into the planes from plane row prow
     auto split_rows = [&](const k::Stream& on, bool is_b, int64_t r0, int64_t rows, int64_t prow) {
         const Op op = is_b ? tb : ta;
@@ -362,7 +363,8 @@ void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, doubl
         sp.k = k;
         sp.kp = kp;
         sp.ex = (is_b ? E : D) + r0;
-        sp.P = (is_b ? Bp : Ap) + prow * kp;  // plane rows come in 16-row bands of kp bytes each
+        sp.map = is_b ? map_b : map_a;
+        sp.P = (is_b ? Bp : Ap) + prow / 64 * sp.map.group;
         sp.plane = is_b ? L.planeB : L.planeA;
         sp.group = static_cast<int64_t>(s) * sp.plane;
         sp.s = s;
@@ -376,8 +378,9 @@ void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, doubl
     auto gemm_block = [&](const k::Stream& on, int64_t rows, int64_t c0, int64_t cols) {
         k::GemmArgs ga{};
         ga.A = Ap;
-        ga.B = Bp + c0 * kp;
-        ga.kp = kp;
+        ga.B = Bp + c0 / 64 * map_b.group;
+        ga.map_a = map_a;
+        ga.map_b = map_b;
         ga.plane_a = L.planeA;
         ga.plane_b = L.planeB;
         ga.plane_r = L.planeR;
@@ -568,7 +571,8 @@ void Engine::ozaki1(int64_t m, int64_t n, int64_t k, const double* A, int64_t ld
         k::GemmArgs ga{};
         ga.A = Ap;
         ga.B = Bp;
-        ga.kp = kpx;
+        ga.map_a = k::PlaneMap::by_k(mpad);
+        ga.map_b = k::PlaneMap::by_k(npad);
         ga.ldr = mpad;
         ga.tiles_m = static_cast<int>(mpad / TM);
         ga.tiles_n = static_cast<int>(npad / TN);

@@ -30,8 +30,6 @@ using namespace math;
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
-typedef __attribute__((address_space(3))) void* lds_ptr;
-typedef __attribute__((address_space(1))) void* glb_ptr;
 
 namespace {
 
@@ -46,7 +44,6 @@ constexpr int vm_wait(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
 // are dealt to the waves in turn.  Fragments, MFMA operand layout and bank pattern as in igemm.hip.
 template <int TM, int TN, int GM, int GN, int NS, int NL>
 __device__ __forceinline__ void fused_tile(const FusedArgs& p, uint32_t tm, uint32_t tn, v4i* smem, const Stamp& st) {
-#if defined(__HIP_DEVICE_COMPILE__)  // buffer resources are a device type
     constexpr int NWV = GM * GN;
     constexpr int WTM = TM / GM, WTN = TN / GN;
     constexpr int FM = WTM / 32, FN = WTN / 32;
@@ -63,9 +60,9 @@ __device__ __forceinline__ void fused_tile(const FusedArgs& p, uint32_t tm, uint
     const int fr = lane & 31, fc = lane >> 5;
     const int S = p.s;
     const int nst = static_cast<int>(p.kp / KT);  // kp is a multiple of 128
-    const int64_t band = p.kp * 16;  // bytes of a 16-row band of a plane
     const auto tb = const_tab(p.tab);
     // block b of a stage: k half b % 2 of band b / 2 (bands of A, then of B); this wave's are d NWV + wave
+    const PlaneMap map = PlaneMap::by_group(p.kp);
     const int8_t* src[ND];
     int64_t step[ND];  // next plane
 #pragma unroll
@@ -74,7 +71,7 @@ __device__ __forceinline__ void fused_tile(const FusedArgs& p, uint32_t tm, uint
         const bool isa = b < TM / 8;
         const int64_t row = isa ? static_cast<int64_t>(tm) * (TM / 16) + (b >> 1)
                                 : static_cast<int64_t>(tn) * (TN / 16) + (b >> 1) - TM / 16;
-        src[d] = (isa ? p.A : p.B) + row * band + (b & 1) * 1024;
+        src[d] = (isa ? p.A : p.B) + (row >> 2) * map.group + (row & 3) * map.band + (b & 1) * map.blk;
         step[d] = isa ? p.plane_a : p.plane_b;
     }
     char* sbase = reinterpret_cast<char*>(smem);
@@ -86,21 +83,14 @@ __device__ __forceinline__ void fused_tile(const FusedArgs& p, uint32_t tm, uint
         offa[ks] = wm * WTM * KT + rowoff + ch;
         offb[ks] = (TM + wn * WTN) * KT + rowoff + ch;
     }
-    // DMA stream, plane-major: stage `left` stages before the end, at k byte dko of its plane
+    // DMA stream, plane-major: stage `left` stages before the end, at offset dko of its plane
+    const int kstep = static_cast<int>(2 * map.blk), kend = nst * kstep;
     int left = S * nst, dko = 0, dbuf = 0;
-    const int kend = nst * 2048;
-    auto rsrc = [](const int8_t* q) {
-        return __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(q), 0, 0xFFFFFFFFu, 0x00027000);
-    };
-    auto dma = [&](int d) {  // the wave's d-th block of the stage
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc(src[d]), (lds_ptr)(sbase + dbuf + (d * NWV + wave) * 1024), 16,
-                                                 lane * 16, dko, 0, 0);
-    };
+    auto dma = [&](int d) { block_to_lds(src[d], dko, lane, sbase + dbuf + (d * NWV + wave) * 1024); };  // the wave's d-th block
     // next stage; past the last one the same stage is fetched again into a buffer that is not read
     auto dma_next = [&] {
         dbuf = dbuf == (NS - 1) * STAGE ? 0 : dbuf + STAGE;
-        const int last = --left <= 0;
-        dko += last ? 0 : 2048;
+        dko += --left <= 0 ? 0 : kstep;
         const bool wrap = dko == kend;
         dko = wrap ? 0 : dko;
 #pragma unroll
@@ -271,7 +261,6 @@ __device__ __forceinline__ void fused_tile(const FusedArgs& p, uint32_t tm, uint
                 if (row + e < p.mb) cp[e] = v[e];
         }
     }
-#endif
 }
 
 // tile (tm, tn) of index w: columns of 8 tile-rows, walking tile-columns inside a group

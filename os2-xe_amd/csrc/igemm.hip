@@ -8,10 +8,10 @@
 // every entry mod m_t to a byte, the only information the CRT needs
 // (hpp:590-601), cutting the CRT's reads from 4s to s bytes per entry.
 //
-// Operand planes are stored blocked (plane_offset() in kernels.hpp): 1 KB per
+// Operand planes are stored blocked (PlaneMap in kernels.hpp): 1 KB per
 // 16 rows x 64 k, the four 16-byte k-chunks of a row XOR-permuted by
 // (row >> 2) & 3.  One stage of a macro tile is then a run of whole 1 KB
-// blocks, each fetched by one global_load_lds_dwordx4 (lane l -> bytes
+// blocks, each fetched by one 16-byte LDS-DMA load (lane l -> bytes
 // 16l..16l+15) straight into LDS in the same order, and the MFMA operand reads
 // (lane l: row l mod 32, chunk 2 ks + l / 32) are free of bank conflicts:
 // ds_read_b128 serves 16 lanes per pass from the quads {0,3,5,6} and {1,2,4,7}
@@ -49,8 +49,6 @@ using namespace math;
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
-typedef __attribute__((address_space(3))) void* lds_ptr;
-typedef __attribute__((address_space(1))) void* glb_ptr;
 
 namespace {
 
@@ -186,19 +184,17 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint32_t plane, uin
     constexpr int VM_AHEAD = (NS - 3) * ND;    // DMAs still in flight when a stage must have landed
     static_assert(WTM * WTN * 4 <= NS * STAGE, "epilogue staging must fit in the stage buffers");
 
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave >> 1, wn = wave & 1;
     const int fr = lane & 31, fc = lane >> 5;
     const int nkt = static_cast<int>(p.klen / KT);  // even: klen is a multiple of 128
-    const int64_t kblocks = p.kp / KT;              // plane blocks per 16 rows
-    // this lane's 16 bytes of each of its DMA blocks at stage 0
+    // first of the wave's DMA blocks of A and of B, at the stage that the DMA stream has reached
     const int8_t* Ag = p.A + static_cast<int64_t>(plane) * p.plane_a +
-                       ((static_cast<int64_t>(tm) * (BM / 16) + wave * LA) * kblocks + p.k0 / KT) * 1024 + lane * 16;
+                       static_cast<int64_t>(tm) * (BM / 64) * p.map_a.group + wave * LA / 4 * p.map_a.group + wave * LA % 4 * p.map_a.band + p.k0 / KT * p.map_a.blk;
     const int8_t* Bg = p.B + static_cast<int64_t>(plane) * p.plane_b +
-                       ((static_cast<int64_t>(tn) * (BN / 16) + wave * LB) * kblocks + (p.k0 + p.kb_extra) / KT) * 1024 +
-                       lane * 16;
-    const int64_t bstride = kblocks * 1024;  // next 16-row block
+                       static_cast<int64_t>(tn) * (BN / 64) * p.map_b.group + wave * LB / 4 * p.map_b.group + wave * LB % 4 * p.map_b.band + (p.k0 + p.kb_extra) / KT * p.map_b.blk;
+    const int band_a = static_cast<int>(p.map_a.band), band_b = static_cast<int>(p.map_b.band);
+    int left = nkt, dbuf = 0, rbuf = 0;  // stages that the stream has left; LDS offsets of its stage and of the read one
     char* sbase = reinterpret_cast<char*>(smem);
     // LDS byte offsets of this lane's fragments (row-major 64-byte rows; the
     // chunk permutation depends on row bits 2-3 only, so fragment i is +2 KB * i)
@@ -221,41 +217,43 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint32_t plane, uin
             for (int v = 0; v < 16; ++v) acc[i][j][v] = c30;
     v4i fa0[2][FM], fb0[2][FN], fa1[2][FM], fb1[2][FN];
 
-    // stage KT_ (clamped to the last one: past the end the DMA refills a
-    // buffer that is never read again, keeping the vmcnt arithmetic uniform)
-#define OZ2_DMA(KT_, D_)                                                                                         \
+    // past the last stage the DMA refills a buffer that is never read again with the last one, keeping the
+    // vmcnt arithmetic uniform
+    auto dma = [&](int d) {
+        if (d < LA) block_to_lds(Ag, d * band_a, lane, sbase + dbuf + (wave * LA + d) * 1024);
+        else block_to_lds(Bg, (d - LA) * band_b, lane, sbase + dbuf + BM * KT + (wave * LB + d - LA) * 1024);
+    };
+    auto dma_next = [&] {
+        dbuf = dbuf == (NS - 1) * STAGE ? 0 : dbuf + STAGE;
+        const bool more = --left > 0;
+        Ag += more ? p.map_a.blk : 0;
+        Bg += more ? p.map_b.blk : 0;
+    };
+    auto read_next = [&] { rbuf = rbuf == (NS - 1) * STAGE ? 0 : rbuf + STAGE; };
+#define OZ2_READ(NA, NB, R_)                                                                                     \
     {                                                                                                            \
-        char* st_ = sbase + ((KT_) % NS) * STAGE;                                                               \
-        const int64_t ko_ = static_cast<int64_t>(min((KT_), nkt - 1)) * 1024;                                    \
-        if ((D_) < LA)                                                                                           \
-            __builtin_amdgcn_global_load_lds((glb_ptr)(Ag + (D_) * bstride + ko_),                               \
-                                             (lds_ptr)(st_ + (wave * LA + (D_)) * 1024), 16, 0, 0);            \
-        else                                                                                                     \
-            __builtin_amdgcn_global_load_lds((glb_ptr)(Bg + ((D_) - LA) * bstride + ko_),                        \
-                                             (lds_ptr)(st_ + BM * KT + (wave * LB + (D_) - LA) * 1024), 16, 0, 0); \
-    }
-#define OZ2_READ(NA, NB, KT_, R_)                                                                                \
-    {                                                                                                            \
-        const char* s_ = sbase + ((KT_) % NS) * STAGE;                                                          \
+        const char* s_ = sbase + rbuf;                                                                           \
         const int ks_ = (R_) / (FM + FN), w_ = (R_) % (FM + FN);                                                 \
         if (w_ < FM) NA[ks_][w_] = *reinterpret_cast<const v4i*>(s_ + offa[ks_] + w_ * 2048);                   \
         else NB[ks_][w_ - FM] = *reinterpret_cast<const v4i*>(s_ + offb[ks_] + (w_ - FM) * 2048);               \
     }
-    // one stage: MFMAs on (FA, FB), reads of stage KTR into (NA, NB), DMAs of stage KTI,
+    // one stage: MFMAs on (FA, FB), reads of the next stage into (NA, NB), DMAs NS - 1 stages ahead,
     // spread evenly in a fixed order
-#define OZ2_HALF(FA, FB, NA, NB, KTR, KTI)                                                                       \
+#define OZ2_HALF(FA, FB, NA, NB)                                                                                 \
     {                                                                                                            \
         _Pragma("unroll") for (int u = 0; u < NMF; ++u) {                                                        \
-            _Pragma("unroll") for (int r = 0; r < NR; ++r) if (r * NMF / NR == u) OZ2_READ(NA, NB, KTR, r)       \
+            _Pragma("unroll") for (int r = 0; r < NR; ++r) if (r * NMF / NR == u) OZ2_READ(NA, NB, r)       \
             __builtin_amdgcn_sched_barrier(0);                                                                   \
             {                                                                                                    \
                 const int ks = u / (FM * FN), i = (u / FN) % FM, j = i % 2 ? FN - 1 - u % FN : u % FN;\
                 acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(FA[ks][i], FB[ks][j], acc[i][j], 0, 0, 0);     \
             }                                                                                                    \
             __builtin_amdgcn_sched_barrier(0);                                                                   \
-            _Pragma("unroll") for (int d = 0; d < ND; ++d) if (d * NMF / ND == u) OZ2_DMA(KTI, d)                \
+            _Pragma("unroll") for (int d = 0; d < ND; ++d) if (d * NMF / ND == u) dma(d);                \
             __builtin_amdgcn_sched_barrier(0);                                                                   \
         }                                                                                                        \
+        dma_next();                                                                                              \
+        read_next();                                                                                             \
     }
     // top of a stage: its successor landed (own DMAs, then everyone's) and the
     // fragments read during the previous stage are in registers
@@ -270,21 +268,23 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, uint32_t plane, uin
 
     // prologue: stages 0 .. NS-2 in flight, stage 0 landed and read
 #pragma unroll
-    for (int s0 = 0; s0 < NS - 1; ++s0)
+    for (int s0 = 0; s0 < NS - 1; ++s0) {
 #pragma unroll
-        for (int d = 0; d < ND; ++d) OZ2_DMA(s0, d)
+        for (int d = 0; d < ND; ++d) dma(d);
+        dma_next();
+    }
     __builtin_amdgcn_s_waitcnt(vm_wait((NS - 2) * ND));
     __builtin_amdgcn_s_barrier();
 #pragma unroll
-    for (int r = 0; r < NR; ++r) OZ2_READ(fa0, fb0, 0, r)
+    for (int r = 0; r < NR; ++r) OZ2_READ(fa0, fb0, r)
+    read_next();
 
     for (int kt = 0; kt < nkt; kt += 2) {
         OZ2_WAIT()
-        OZ2_HALF(fa0, fb0, fa1, fb1, kt + 1, kt + NS - 1)
+        OZ2_HALF(fa0, fb0, fa1, fb1)
         OZ2_WAIT()
-        OZ2_HALF(fa1, fb1, fa0, fb0, kt + 2, kt + NS)  // the last pass reads a stage that is not used
+        OZ2_HALF(fa1, fb1, fa0, fb0)  // the last pass reads a stage that is not used
     }
-#undef OZ2_DMA
 #undef OZ2_READ
 #undef OZ2_HALF
 #undef OZ2_WAIT

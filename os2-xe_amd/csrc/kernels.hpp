@@ -2,7 +2,7 @@
 //
 // Data layout in HBM (all owned by the engine's workspace):
 //   planes   int8  [group][t] then blocked: 1 KB per 16 rows x 64 k of op(A) (or op(B)^T),
-//                  blocks k-major within a 16-row band (plane_offset); rows padded with zeros to
+//                  1 KB blocks of 16 rows x 64 k (PlaneMap); rows padded with zeros to
 //                  the GEMM tile, k to kp
 //   residues uint8 [chunk][group][t][j][ldr]  GEMM results reduced mod m_t, i contiguous
 //   D, E     int32 exponents per row of op(A) / column of op(B)
@@ -68,23 +68,48 @@ void launch(const Stream& st, void (*kernel)(P...), dim3 grid, dim3 block, A&&..
 }
 #endif
 
-// Byte offset of element (row r, k p) inside one operand plane with kp columns:
-// 16-row bands of kp/64 consecutive 1 KB blocks; inside a block, 64 bytes per row
-// as four 16-byte chunks.  Byte b of chunk c holds k = block_k(c, b) of the block:
-// chunk c takes the pair (2c, 2c+1) of each group of 8 consecutive k, so the four
-// threads that fill the chunks of one row read 64 contiguous bytes of a
+// Layout of one operand plane: 1 KB blocks of 16 rows (a band) x 64 k, 64 bytes per row as four 16-byte
+// chunks.  Byte b of chunk c holds k = block_k(c, b) of the block: chunk c takes the pair (2c, 2c+1) of each
+// group of 8 consecutive k, so the four threads that fill the chunks of one row read 64 contiguous bytes of a
 // k-contiguous row per load.  The GEMM's dot products do not depend on the k order
 // inside a block, which both operands share.  The chunks of row r are permuted by
 // XOR with (r >> 2) & 3: the GEMM's DMA copies blocks verbatim to LDS, where that
 // permutation makes the MFMA operand reads free of bank conflicts.
 __host__ __device__ constexpr int block_k(int c, int b) { return 8 * (b >> 1) + 2 * c + (b & 1); }
-__host__ __device__ inline int64_t chunk_offset(int64_t r, int64_t blk, int c, int64_t kp) {
-    return (((r >> 4) * (kp >> 6) + blk) << 10) + ((r & 15) << 6) + ((c ^ static_cast<int>((r >> 2) & 3)) << 4);
+// Bytes from one group of 4 bands to the next, from band to band in it, and from block column to block column.
+// A stage of a GEMM tile reads one block column of 4 to 16 bands.
+//   by_band:  a band's blocks side by side (the documented layout of the kernel-level entry points).  With kp
+//             a multiple of 256 the blocks of a stage lie on a few of the L2's channels.
+//   by_group: the four bands of a block column side by side, 4 KB, which cover the channels evenly; a tile's
+//             operand is a few runs of memory.  For 128 x 128 and 64 x 64 tiles and the fused kernel.
+//   by_k:     all bands of a block column side by side.  For the tiles of 256 rows: the split's writes are
+//             whole runs too, where a long k makes the groups' strides powers of two.
+// MI355X, us, by_band / by_group / by_k: GEMM 1024^3 s = 14 (128 x 128) 32.0 / 25.8 / 28.9, 512 x 512 x 2048
+// s = 16 22.7 / 16.8 / 15.0, 1024 x 1024 x 1152 s = 14 (256 x 256) 25.7 / 26.0 / 25.0, 8192^3 s = 16 6900 /
+// 6680 / 6670, 4096^3 s = 8 498 / 479 / 476; split of 2048 x 65000 by 65000 x 2048 s = 24 1965 / 2032 / 1890,
+// of 8192 x 8192 both s = 16 665 / 625 / 628.
+struct PlaneMap {
+    int64_t group, band, blk;
+    static constexpr PlaneMap by_band(int64_t kp) { return {kp * 64, kp * 16, 1024}; }
+    static constexpr PlaneMap by_group(int64_t kp) { return {kp * 64, 1024, 4096}; }
+    static constexpr PlaneMap by_k(int64_t rows_pad) { return {4096, 1024, rows_pad * 64}; }
+    static constexpr PlaneMap of(Tile t, bool fused, int64_t rows_pad, int64_t kp) {
+        return !fused && (t == Tile::T256 || t == Tile::T256x128) ? by_k(rows_pad) : by_group(kp);
+    }
+};
+__host__ __device__ inline int64_t chunk_offset(int64_t r, int64_t blk, int c, const PlaneMap& map) {
+    return (r >> 6) * map.group + ((r >> 4) & 3) * map.band + blk * map.blk + ((r & 15) << 6) + ((c ^ static_cast<int>((r >> 2) & 3)) << 4);
 }
-__host__ __device__ inline int64_t plane_offset(int64_t r, int64_t p, int64_t kp) {
-    const int q = static_cast<int>(p & 63);
-    return chunk_offset(r, p >> 6, (q >> 1) & 3, kp) + (((q >> 3) << 1) | (q & 1));
+
+#if defined(__HIPCC__)
+// one plane block, at src + offset (both uniform), to LDS by DMA: lane l moves bytes 16 l .. 16 l + 15
+__device__ __forceinline__ void block_to_lds(const int8_t* src, int offset, int lane, char* lds) {
+#if defined(__HIP_DEVICE_COMPILE__)  // buffer resources are a device type
+    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(src), 0, 0xFFFFFFFFu, 0x00027000);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)lds, 16, lane * 16, offset, 0, 0);
+#endif
 }
+#endif
 
 // ---- scaling -----------------------------------------------------------------
 // Exponents of the `len` rows of op(X) over k columns.  kcontig: row r of op(X)
@@ -105,6 +130,7 @@ struct SplitArgs {
     int64_t kp;           // padded k (multiple of 128)
     const int32_t* ex;    // exponent per row (already offset)
     int8_t* P;            // planes
+    PlaneMap map;
     int64_t plane;        // bytes per plane (rows_pad * kp)
     int64_t group;        // bytes per group of s planes (complex)
     int s;
@@ -116,10 +142,10 @@ void split(const Stream& st, const SplitArgs& a);
 
 // ---- INT8 GEMM with residue epilogue ------------------------------------------
 struct GemmArgs {
-    const int8_t* A;      // planes of op(A): nplanes x (mpad x kp, blocked by plane_offset)
-    const int8_t* B;      // planes of op(B): nplanes x (npad x kp, blocked by plane_offset)
+    const int8_t* A;      // planes of op(A): nplanes x (mpad x kp, blocked as map_a says)
+    const int8_t* B;      // planes of op(B): nplanes x (npad x kp, blocked as map_b says)
     uint8_t* R;           // residues [nplanes][npad_c][ldr]
-    int64_t kp;           // row stride of planes (bytes)
+    PlaneMap map_a, map_b;
     int64_t plane_a, plane_b, plane_r;
     int64_t ldr;          // column stride of residues (= mpad)
     int64_t k0, klen;     // k range (multiples of 128)
@@ -159,7 +185,7 @@ void crt(const Stream& st, const CrtArgs& a);
 // ---- INT8 GEMMs of all planes and the CRT of a tile in one workgroup --------------
 // a real product of one k-chunk; tile 128 or 64 (square): the planes are padded to it
 struct FusedArgs {
-    const int8_t *A, *B;      // planes of op(A), op(B)
+    const int8_t *A, *B;      // planes of op(A), op(B): PlaneMap::by_group
     int64_t kp, plane_a, plane_b;
     int tiles_m, tiles_n;
     int s, nl, up;            // moduli, Plan::NL, Plan::up()
@@ -173,7 +199,7 @@ void fused(const Stream& st, int tile, const FusedArgs& a);
 
 // ---- Ozaki Scheme I (the accuracy benchmark's comparison baseline) --------------------
 // L balanced base-128 digits of RNE(op(X)[r][p] 2^ex[r]) per element into one extended
-// plane of rows_pad x (L kp) bytes (blocked as plane_offset with L kp columns): digit i
+// plane of rows_pad x (L kp) bytes (PlaneMap::by_k): digit i
 // (most significant first) at k-slot i, or L - 1 - i with rev
 struct Oz1SliceArgs {
     const double* X;

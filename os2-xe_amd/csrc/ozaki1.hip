@@ -5,7 +5,7 @@
 //
 // Digit planes: every row of op(X) (rows of A, columns of B) keeps its L balanced
 // base-128 digits side by side along k in one extended plane of L * kp columns, in
-// the GEMM's blocked layout (plane_offset): digit i of A at k-slot i, digit i of B at
+// the GEMM's blocked layout (PlaneMap): digit i of A at k-slot i, digit i of B at
 // k-slot L - 1 - i.  The anti-diagonal d = sum_{a <= d} A_a B_{d-a} is then one GEMM
 // over k-slots 0 .. d of A and L - 1 - d .. L - 1 of B.
 #include "kernels.hpp"
@@ -56,7 +56,7 @@ __global__ void __launch_bounds__(256) oz1_slice_kernel(Oz1SliceArgs a) {
         const int64_t mag = static_cast<int64_t>(scaled_mag62(bits, e));
         x[q] = (zero_row || p >= a.k) ? 0 : ((bits >> 63) ? -mag : mag);
     }
-    const int64_t kblocks = static_cast<int64_t>(L) * (a.kp >> 6);
+    const PlaneMap map = PlaneMap::by_k(a.rows_pad);
     for (int i = L - 1; i >= 0; --i) {
         uint32_t w[4];
 #pragma unroll
@@ -72,7 +72,7 @@ __global__ void __launch_bounds__(256) oz1_slice_kernel(Oz1SliceArgs a) {
             w[g] = pack_lo_bytes(b[0], b[1], b[2], b[3]);
         }
         const int64_t slot = a.rev ? L - 1 - i : i;
-        int8_t* out = a.P + chunk_offset(r, slot * (a.kp >> 6) + blk, c, kblocks << 6);
+        int8_t* out = a.P + chunk_offset(r, slot * (a.kp >> 6) + blk, c, map);
         *reinterpret_cast<uint4*>(out) = make_uint4(w[0], w[1], w[2], w[3]);
     }
 }

@@ -6,7 +6,7 @@
 // Inf/NaN) and hpp:251-303, 407-520 (x = RNE(v 2^e) taken exactly from the
 // IEEE bits, symmetric residues per modulus; complex: Re, +-Im, Re+-Im).
 //
-// Both operands are written in one blocked plane layout (plane_offset: 1 KB
+// Both operands are written in one blocked plane layout (PlaneMap: 1 KB
 // blocks of 16 rows x 64 k), so the GEMM copies A and B tiles the same way.
 // A thread's 16 k lie in one 16-byte chunk of a block (block_k order), so each
 // plane store is one aligned vector store.  Rows of op(X)
@@ -224,17 +224,19 @@ struct SplitSlot {
 
 // (row, slot) of a thread.  KCONTIG: row r is contiguous (X[p + r*ldx]); a block
 // covers 256 slots along the row(s).  !KCONTIG: rows strided (X[r + p*ldx]); a block
-// is 16 rows x 16 slots, lanes along rows, so a wave (16 rows x 4 slots) fills whole
-// 1 KB plane blocks and reads one 128-byte line per load.
-template <bool KCONTIG>
+// is one 64-k block of 4 bands (2 for half chunks), lanes along rows, so a wave (16 rows x 4 slots)
+// reads one 128-byte line per load, and the block 512 bytes of a column, and writes a run of plane blocks.
+template <bool KCONTIG, int Q>
 __device__ __forceinline__ void split_thread(int lg_tpr, uint32_t bx, uint32_t by, int64_t& r, int64_t& ck) {
     if (KCONTIG) {
         const int tpr = 1 << lg_tpr;  // threads per row in a block
         r = static_cast<int64_t>(bx) * (256 >> lg_tpr) + (threadIdx.x >> lg_tpr);
         ck = static_cast<int64_t>(by) * tpr + (threadIdx.x & (tpr - 1));
     } else {
-        r = static_cast<int64_t>(bx) * 16 + (threadIdx.x & 15);
-        ck = static_cast<int64_t>(by) * 16 + (threadIdx.x >> 4);
+        constexpr int slots = 64 / Q;
+        const int wq = threadIdx.x >> 4;  // 16 rows x one slot
+        r = static_cast<int64_t>(bx) * (256 / slots) + wq / slots * 16 + (threadIdx.x & 15);
+        ck = static_cast<int64_t>(by) * slots + wq % slots;
     }
 }
 
@@ -253,7 +255,7 @@ template <int FORM, bool KCONTIG, int Q>
 __device__ __forceinline__ void split_real_body(const SplitArgs& a, int lg_tpr, uint32_t bx, uint32_t by) {
     const auto tb = const_tab(a.tab);
     int64_t r, ck;
-    split_thread<KCONTIG>(lg_tpr, bx, by, r, ck);
+    split_thread<KCONTIG, Q>(lg_tpr, bx, by, r, ck);
     if (r >= a.rows_pad || ck >= a.kp / Q) return;
     const SplitSlot<Q> sl(ck);
     const bool rowok = r < a.rows;
@@ -289,7 +291,7 @@ __device__ __forceinline__ void split_real_body(const SplitArgs& a, int lg_tpr, 
     uint32_t limbs[Q][4];
 #pragma unroll
     for (int q = 0; q < Q; ++q) to_limbs<F>(rowzero ? 0 : bits[q], e, false, limbs[q]);
-    int8_t* out = a.P + chunk_offset(r, sl.blk, sl.c, a.kp) + sl.q0;
+    int8_t* out = a.P + chunk_offset(r, sl.blk, sl.c, a.map) + sl.q0;
     uint32_t w[4] = {0, 0, 0, 0};
     // plane 0 has m = 256 in every moduli set: its residue byte is the low byte of u
 #pragma unroll
@@ -312,7 +314,7 @@ template <int FORM, bool KCONTIG, bool CONJ, int Q>
 __device__ __forceinline__ void split_cplx_body(const SplitArgs& a, int lg_tpr, uint32_t bx, uint32_t by) {
     const auto tb = const_tab(a.tab);
     int64_t r, ck;
-    split_thread<KCONTIG>(lg_tpr, bx, by, r, ck);
+    split_thread<KCONTIG, Q>(lg_tpr, bx, by, r, ck);
     if (r >= a.rows_pad || ck >= a.kp / Q) return;
     const SplitSlot<Q> sl(ck);
     const bool rowok = r < a.rows;
@@ -349,7 +351,7 @@ __device__ __forceinline__ void split_cplx_body(const SplitArgs& a, int lg_tpr, 
         to_limbs<F>(rowzero ? 0 : br[q], e, false, lr[q]);
         to_limbs<F>(rowzero ? 0 : bi[q], e, false, li[q]);
     }
-    int8_t* out = a.P + chunk_offset(r, sl.blk, sl.c, a.kp) + sl.q0;
+    int8_t* out = a.P + chunk_offset(r, sl.blk, sl.c, a.map) + sl.q0;
     for (int t = 0; t < a.s; ++t) {
         const int32_t m = static_cast<int32_t>(tb->m[t]);
         const int32_t h = static_cast<int32_t>(tb->h[t]);
@@ -425,8 +427,9 @@ SplitItem split_item(const SplitArgs& a, uint32_t& gy) {
         it.gx = static_cast<uint32_t>((a.rows_pad + (256 / tpr) - 1) / (256 / tpr));
         gy = static_cast<uint32_t>((nck + tpr - 1) / tpr);
     } else {
-        it.gx = static_cast<uint32_t>((a.rows_pad + 15) / 16);
-        gy = static_cast<uint32_t>((nck + 15) / 16);
+        const int slots = 64 / q;
+        it.gx = static_cast<uint32_t>((a.rows_pad + 256 / slots - 1) / (256 / slots));
+        gy = static_cast<uint32_t>((nck + slots - 1) / slots);
     }
     return it;
 }
