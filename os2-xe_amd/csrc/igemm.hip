@@ -59,25 +59,6 @@ constexpr int KT = 64;   // k bytes per LDS stage = one plane block column
 constexpr int vm_wait(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
 constexpr int kLgkmWait0 = 0xC07F & ~0x0F00;  // lgkmcnt(0) only
 
-// blockIdx -> work item with the 8 XCDs of MI355X each given a contiguous
-// range (workgroups are dispatched round-robin over XCDs, so consecutive ids
-// land on different L2s; remapping keeps tiles that share A/B rows together).
-__device__ __forceinline__ uint32_t xcd_remap(uint32_t b, uint32_t n) {
-    if ((n & 7) != 0) return b;
-    return (b & 7) * (n >> 3) + (b >> 3);
-}
-
-// The same per plane: work items stay plane-major and each plane's tiles are
-// split over the XCDs in contiguous ranges, so all XCDs work on one plane at a
-// time and share its A and B planes in the last-level cache (with whole ranges
-// of planes per XCD, 8 plane pairs compete for it).
-__device__ __forceinline__ uint32_t plane_xcd_remap(uint32_t b, uint32_t tiles, uint32_t n) {
-    if ((tiles & 7) != 0) return xcd_remap(b, n);
-    const uint32_t plane = b / tiles;
-    const uint32_t r = b - plane * tiles;
-    return plane * tiles + (r & 7) * (tiles >> 3) + (r >> 3);
-}
-
 __device__ __forceinline__ int plane_modulus(const GemmArgs& p, uint32_t plane) {
     return static_cast<int>((static_cast<uint32_t>(p.plane0) + plane) % static_cast<uint32_t>(p.s));
 }
@@ -305,8 +286,7 @@ __global__ void __launch_bounds__(256, MINB) igemm_residue_kernel(GemmArgs p, ui
     __shared__ v4i smem[TileShape<BM, BN, NS>::SMEM / 16];
     const Stamp st(ts);
     uint32_t plane, tm, tn;
-    const uint32_t tiles = static_cast<uint32_t>(p.tiles_m) * static_cast<uint32_t>(p.tiles_n);
-    tile_coords(p, plane_xcd_remap(blockIdx.x, tiles, gridDim.x), plane, tm, tn);
+    tile_coords(p, xcd_window(blockIdx.x, gridDim.x, 256 * MINB), plane, tm, tn);
     gemm_tile<BM, BN, NS>(p, plane, tm, tn, smem);
     st.end();
 }
@@ -315,8 +295,7 @@ template <int BM, int BN, int MINB, int NS>
 __global__ void __launch_bounds__(256, MINB) igemm_int32_kernel(GemmArgs p) {
     __shared__ v4i smem[TileShape<BM, BN, NS>::SMEM / 16];
     uint32_t plane, tm, tn;
-    const uint32_t tiles = static_cast<uint32_t>(p.tiles_m) * static_cast<uint32_t>(p.tiles_n);
-    tile_coords(p, plane_xcd_remap(blockIdx.x, tiles, gridDim.x), plane, tm, tn);
+    tile_coords(p, xcd_window(blockIdx.x, gridDim.x, 256 * MINB), plane, tm, tn);
     gemm_tile<BM, BN, NS, true>(p, plane, tm, tn, smem);
 }
 
@@ -383,13 +362,13 @@ __global__ void __launch_bounds__(256, MINB) igemm_grouped_kernel(const GemmArgs
     }
 }
 
-// One workgroup per tile, work indices spread over the XCDs in contiguous ranges.
+// One workgroup per tile.
 template <int BM, int BN, int MINB, int NS>
 __global__ void __launch_bounds__(256, MINB) igemm_grouped_blocks_kernel(const GemmArgs* __restrict__ items,
                                                                          const uint32_t* __restrict__ start,
                                                                          const uint32_t* __restrict__ owner) {
     __shared__ v4i smem[TileShape<BM, BN, NS>::SMEM / 16];
-    const uint32_t w = xcd_remap(blockIdx.x, gridDim.x);
+    const uint32_t w = xcd_window(blockIdx.x, gridDim.x, 256 * MINB);
     const uint32_t it = owner[w];
     const GemmArgs& p = items[it];
     uint32_t plane, tm, tn;

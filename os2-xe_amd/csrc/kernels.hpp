@@ -102,6 +102,18 @@ __host__ __device__ inline int64_t chunk_offset(int64_t r, int64_t blk, int c, c
 }
 
 #if defined(__HIPCC__)
+// blockIdx -> work item.  Workgroups go round-robin over the 8 XCDs, each with an L2 of its own; of every
+// `window` items (a multiple of 8: what the chip holds at once) each XCD takes a contiguous share, so that
+// the tiles it runs together share A and B bands, of large planes and of small ones.  With each plane's tiles
+// spread over all XCDs, as large planes like it, an XCD held two tiles of 8 planes at 512 x 512 and read three
+// times the planes' bytes from memory; with tile counts that 8 does not divide left as they came, five times
+// (1537 x 771 x 3001 s = 15).  Before -> after, us: 512 x 512 x 2048 s = 16 16.4 -> 10.5, 1024 x 1024 x 2048
+// 45.2 -> 35.0, 1537 x 771 x 3001 87.4 -> 68.4 (all 128 x 128), 2048^3 135 -> 128, 8192^3 the same.
+__device__ __forceinline__ uint32_t xcd_window(uint32_t b, uint32_t n, uint32_t window) {
+    const uint32_t base = b / window * window, i = b - base, len = min(window, n - base);
+    const uint32_t x = i & 7, q = len >> 3, r = len & 7;
+    return base + x * q + min(x, r) + (i >> 3);
+}
 // one plane block, at src + offset (both uniform), to LDS by DMA: lane l moves bytes 16 l .. 16 l + 15
 __device__ __forceinline__ void block_to_lds(const int8_t* src, int offset, int lane, char* lds) {
 #if defined(__HIP_DEVICE_COMPILE__)  // buffer resources are a device type
