@@ -128,8 +128,8 @@ BatchPlan::BatchPlan(Engine& eng, std::vector<GemmDesc> descs, const std::vector
             const int tk = q.plan.tk;
             int32_t* D = reinterpret_cast<int32_t*>(base + q.oD);
             int32_t* E = reinterpret_cast<int32_t*>(base + q.oE);
-            sj.push_back({g.A, g.lda, g.m, g.k, g.ta != Op::N, false, tk, reinterpret_cast<uint64_t*>(base + q.oPA), D});
-            sj.push_back({g.B, g.ldb, g.n, g.k, g.tb == Op::N, false, tk, reinterpret_cast<uint64_t*>(base + q.oPB), E});
+            sj.push_back({g.A, g.lda, g.m, g.k, g.ta != Op::N, false, tk, reinterpret_cast<uint64_t*>(base + q.oPA), D, true});
+            sj.push_back({g.B, g.ldb, g.n, g.k, g.tb == Op::N, false, tk, reinterpret_cast<uint64_t*>(base + q.oPB), E, true});
             for (int which = 0; which < 2; ++which) {
                 k::SplitArgs a{};
                 a.kcontig = which == 0 ? g.ta != Op::N : g.tb == Op::N;
@@ -140,7 +140,13 @@ BatchPlan::BatchPlan(Engine& eng, std::vector<GemmDesc> descs, const std::vector
                 a.k = g.k;
                 a.kp = q.kp;
                 a.map = k::PlaneMap::of(q.tile, q.ftile, a.rows_pad, q.kp);
-                a.ex = which == 0 ? D : E;
+                a.ex = a.ex_out = which == 0 ? D : E;
+                if (k::scale_folds(a.rows, a.k, a.kcontig)) {
+                    a.part = sj[sj.size() - 2 + which].partial;
+                    a.part_ld = a.rows;
+                    a.nkb = k::scale_partials(a.rows, a.k, a.kcontig);
+                    a.tk = tk;
+                }
                 a.P = reinterpret_cast<int8_t*>(base + (which == 0 ? q.oA : q.oB));
                 a.plane = which == 0 ? q.planeA : q.planeB;
                 a.group = static_cast<int64_t>(s_[i]) * a.plane;

@@ -349,8 +349,9 @@ void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, doubl
     // GEMMs and CRT in one kernel (its tile), or 0
     const int ftile = nblocks > 1 ? 0 : fused_tile(cs, L, mb, nb);
     const k::PlaneMap map_a = k::PlaneMap::of(tile_, ftile, L.mpad, kp), map_b = k::PlaneMap::of(tile_, ftile, L.npad, kp);
+    const bool fold_a = k::scale_folds(m, k, ta != Op::N), fold_b = k::scale_folds(n, k, tb == Op::N);
     // split of `rows` rows of op(X) starting at row r0 into the planes from plane row prow
-    auto split_rows = [&](const k::Stream& on, bool is_b, int64_t r0, int64_t rows, int64_t prow) {
+    auto split_args = [&](bool is_b, int64_t r0, int64_t rows, int64_t prow) {
         const Op op = is_b ? tb : ta;
         const double* X = is_b ? B : A;
         const int64_t ldx = is_b ? ldb : lda;
@@ -362,7 +363,13 @@ void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, doubl
         sp.rows_pad = round_up(rows, ftile ? ftile : is_b ? L.TN : L.TM);
         sp.k = k;
         sp.kp = kp;
-        sp.ex = (is_b ? E : D) + r0;
+        sp.ex = sp.ex_out = (is_b ? E : D) + r0;
+        if (is_b ? fold_b : fold_a) {
+            sp.part = (is_b ? PB : PA) + r0;
+            sp.part_ld = is_b ? n : m;
+            sp.nkb = k::scale_partials(sp.part_ld, k, sp.kcontig);
+            sp.tk = tk;
+        }
         sp.map = is_b ? map_b : map_a;
         sp.P = (is_b ? Bp : Ap) + prow / 64 * sp.map.group;
         sp.plane = is_b ? L.planeB : L.planeA;
@@ -372,7 +379,7 @@ void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, doubl
         sp.conj = cplx && op == Op::C;
         sp.form = form;
         sp.tab = tab;
-        k::split(on, sp);
+        return sp;
     };
     // INT8 GEMMs of `rows` rows of the A panel by columns c0 .. c0 + cols of the B panel
     auto gemm_block = [&](const k::Stream& on, int64_t rows, int64_t c0, int64_t cols) {
@@ -462,18 +469,20 @@ void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, doubl
 
     // scale: exponents of the rows of op(A) and the columns of op(B) (hpp:974-989)
     timed_on(Stage::Scale, stream_, [&](const k::Stream& on) {
-        k::scale(on, A, lda, m, k, ta != Op::N, cplx, tk, PA, D);
-        k::scale(on, B, ldb, n, k, tb == Op::N, cplx, tk, PB, E);
+        k::scale(on, {A, lda, m, k, ta != Op::N, cplx, tk, PA, D, fold_a}, {B, ldb, n, k, tb == Op::N, cplx, tk, PB, E, fold_b});
     });
     bool forked = false;
     for (int64_t j0 = 0; j0 < n; j0 += nb) {
         const int64_t nbj = std::min(nb, n - j0);
         const int64_t wb = nblocks > 1 ? round_up((nbj + nblocks - 1) / nblocks, L.TN) : nbj;
         const int64_t nblk = (nbj + wb - 1) / wb;
-        if (nblk == 1) timed_on(Stage::Split, stream_, [&](const k::Stream& on) { split_rows(on, true, j0, nbj, 0); });
         for (int64_t i0 = 0; i0 < m; i0 += mb) {
             const int64_t mbi = std::min(mb, m - i0);
-            if (ti.pm > 1 || j0 == 0) timed_on(Stage::Split, stream_, [&](const k::Stream& on) { split_rows(on, false, i0, mbi, 0); });
+            const bool split_a = ti.pm > 1 || j0 == 0, split_b = nblk == 1 && i0 == 0;
+            if (split_a || split_b) timed_on(Stage::Split, stream_, [&](const k::Stream& on) {
+                if (split_a && split_b) k::split(on, split_args(false, i0, mbi, 0), split_args(true, j0, nbj, 0));
+                else k::split(on, split_a ? split_args(false, i0, mbi, 0) : split_args(true, j0, nbj, 0));
+            });
             if (nblk == 1) {
                 if (ftile) {
                     timed_on(Stage::Fused, stream_, [&](const k::Stream& on) { fused_block(on, i0, mbi, j0, nbj); });
@@ -491,7 +500,7 @@ void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, doubl
             if (i0 == 0)  // the B panel's blocks, once per panel column, ahead of the CRTs
                 for (int64_t c = 0; c < nblk; ++c) {
                     const int64_t c0 = c * wb, cols = std::min(wb, nbj - c0);
-                    timed_on(Stage::Split, aux_, [&](const k::Stream& on) { split_rows(on, true, j0 + c0, cols, c0); });
+                    timed_on(Stage::Split, aux_, [&](const k::Stream& on) { k::split(on, split_args(true, j0 + c0, cols, c0)); });
                     split_done[c] = sync_event();
                     hip_check(hipEventRecord(split_done[c], aux_), "event record");
                 }
@@ -561,8 +570,8 @@ void Engine::ozaki1(int64_t m, int64_t n, int64_t k, const double* A, int64_t ld
     double* Th = reinterpret_cast<double*>(ws_ + oH);
     double* Tl = reinterpret_cast<double*>(ws_ + oL);
 
-    k::scale(stream_, A, lda, m, k, false, false, tk, reinterpret_cast<uint64_t*>(ws_ + oPA), D);
-    k::scale(stream_, B, ldb, n, k, true, false, tk, reinterpret_cast<uint64_t*>(ws_ + oPB), E);
+    k::scale(stream_, {A, lda, m, k, false, false, tk, reinterpret_cast<uint64_t*>(ws_ + oPA), D},
+             {B, ldb, n, k, true, false, tk, reinterpret_cast<uint64_t*>(ws_ + oPB), E});
     k::oz1_slices(stream_, k::Oz1SliceArgs{A, lda, m, mpad, k, kp, D, Ap, false, false}, L);
     k::oz1_slices(stream_, k::Oz1SliceArgs{B, ldb, n, npad, k, kp, E, Bp, true, true}, L);
     for (int d = 0; d < L; ++d) {

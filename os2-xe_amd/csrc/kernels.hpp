@@ -127,10 +127,20 @@ __device__ __forceinline__ void block_to_lds(const int8_t* src, int offset, int 
 // Exponents of the `len` rows of op(X) over k columns.  kcontig: row r of op(X)
 // is contiguous (X[p + r*ldx]); otherwise rows are strided (X[r + p*ldx]).
 // Complex data (interleaved re, im) scales by the max over both parts.
-// `partial` needs partial_elems(len, k) u64 entries when !kcontig.
+// `partial` needs scale_partial_elems(len, k) u64 entries when !kcontig.
+struct ScaleJob {
+    const double* X;
+    int64_t ldx, len, k;
+    bool kcontig, cplx;
+    int tk;
+    uint64_t* partial;    // [scale_partials][len] maxima (strided rows only)
+    int32_t* ex;
+    bool fold = false;    // where scale_folds() the exponents are left to the split (SplitArgs::part)
+};
 size_t scale_partial_elems(int64_t len, int64_t k, bool kcontig);
-void scale(const Stream& st, const double* X, int64_t ldx, int64_t len, int64_t k, bool kcontig, bool cplx, int tk,
-           uint64_t* partial, int32_t* ex);
+int scale_partials(int64_t len, int64_t k, bool kcontig);
+bool scale_folds(int64_t len, int64_t k, bool kcontig);
+void scale(const Stream& st, const ScaleJob& a, const ScaleJob& b);  // both operands of a product
 
 // ---- split -------------------------------------------------------------------
 struct SplitArgs {
@@ -140,7 +150,11 @@ struct SplitArgs {
     int64_t rows_pad;     // rows written (>= rows, multiple of 32)
     int64_t k;            // valid k
     int64_t kp;           // padded k (multiple of 128)
-    const int32_t* ex;    // exponent per row (already offset)
+    const int32_t* ex;    // exponent per row (already offset); unused with part
+    const uint64_t* part; // strided rows: the scale kernel's partial maxima (already offset), or null
+    int64_t part_ld;      // from one k-block's maxima to the next
+    int nkb, tk;          // with part
+    int32_t* ex_out;      // with part: the exponents are written here
     int8_t* P;            // planes
     PlaneMap map;
     int64_t plane;        // bytes per plane (rows_pad * kp)
@@ -151,6 +165,7 @@ struct SplitArgs {
     const TabSet* tab;    // device tables of this s
 };
 void split(const Stream& st, const SplitArgs& a);
+void split(const Stream& st, const SplitArgs& a, const SplitArgs& b);  // both operands of a product (one form)
 
 // ---- INT8 GEMM with residue epilogue ------------------------------------------
 struct GemmArgs {
@@ -241,14 +256,6 @@ void scale_c(hipStream_t st, double* C, int64_t ldc, int64_t m, int64_t n, doubl
 // ---- grouped launches over many problems (batched GEMMs) -------------------------
 // prep_* append launches (one per kernel variant the jobs need) whose blocks
 // run exactly the single-problem kernels' blocks; launch order = vector order.
-struct ScaleJob {
-    const double* X;
-    int64_t ldx, len, k;
-    bool kcontig, cplx;
-    int tk;
-    uint64_t* partial;    // scale_partial_elems(len, k, kcontig) entries (strided rows only)
-    int32_t* ex;
-};
 struct GemmJob {
     Tile tile;
     GemmArgs args;

@@ -98,24 +98,12 @@ OZ2_HD int32_t exponent_from_maxbits(uint64_t b, int tk) {
     return tk - frexp_exp_bits(b);
 }
 
-// Exact RNE(|v| * 2^e) for |v * 2^e| < 2^101 as a 128-bit magnitude (hpp:251-289),
-// in straight-line code: with sh < 0 the 53-bit mantissa moves right by
-// min(-sh, 63) and rounds to nearest even (all in lo); with sh >= 0 it moves
-// left by sh <= 100 across the two words.  Shift counts stay below 64.
-OZ2_HD void scaled_mag(uint64_t bits, int e, uint64_t& hi, uint64_t& lo) {
-    const int bexp = static_cast<int>((bits >> 52) & 0x7FF);
-    const uint64_t mant = (bits & 0xFFFFFFFFFFFFFull) | (bexp ? 0x10000000000000ull : 0);
-    const int sh = (bexp ? bexp : 1) - 1075 + e;
-    const int ls = sh > 0 ? sh : 0;
-    const int rs = sh < 0 ? (-sh < 63 ? -sh : 63) : 0;
-    const uint64_t q = mant >> rs;
-    const uint64_t rem = mant & ((1ull << rs) - 1);
-    const uint64_t half = rs ? (1ull << (rs - 1)) : ~0ull;
-    const uint64_t down = q + (rem + (q & 1) > half ? 1 : 0);
-    const uint64_t l0 = mant << (ls & 63);                       // ls < 64: low word
-    const uint64_t h0 = (mant >> 1) >> ((63 - ls) & 63);         // ls < 64: bits shifted out of it
-    lo = sh < 0 ? down : (ls < 64 ? l0 : 0);
-    hi = sh < 0 ? 0 : (ls < 64 ? h0 : l0);                       // ls >= 64: mant << (ls - 64)
+OZ2_HD double ldexp_(double v, int e) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_ldexp(v, e);
+#else
+    return std::ldexp(v, e);
+#endif
 }
 
 // RNE(|v| * 2^e) for |v * 2^e| < 2^62 (narrow values) in straight-line code: the
@@ -134,41 +122,31 @@ OZ2_HD uint64_t scaled_mag62(uint64_t bits, int e) {
     return q + (rem + (q & 1) > half ? 1 : 0);
 }
 
-// Octet forms of the offset-binary value u = 2^OFF + x (x = +-RNE(|v| 2^e), |x| <= 2^tk),
-// kept as little-endian 32-bit words; the residue chain takes one v_dot4 per word:
-//   Octets8  OFF = 62  (tk <= 62): the 8 bytes of u <= 2^63 in a[0..1];
-//   Octets12 OFF = 95  (tk <= 94): the 12 bytes of u < 2^96 in a[0..2] (every plan: tk <= 91);
-//   Octets14 OFF = 104 (tk <= 100): the 14 bytes of u <= 2^105 in a[0..3].
+// Words of x = RNE(v 2^e) in base 2^31, x = sum_w (a[w] - 2^31) 2^(31 w): the residue chain takes one v_dot4 a word
+//   Octets8  two words, |x| <= 2^61;   Octets12  three, |x| <= 2^92 (every plan has tk <= 91);
+//   Octets14 four, |x| <= 2^100.
 enum class Limbs { Octets8, Octets12, Octets14 };
 template <Limbs F>
 inline constexpr int kLimbWords = F == Limbs::Octets8 ? 2 : F == Limbs::Octets12 ? 3 : 4;
 
+// Adding 1.5 2^52 + 2^31 units of 2^(31 w) leaves word w, rounded to nearest, in the low half of the sum's bits;
+// subtracting that is exact, and the remainder of at most half a unit goes to the next word.  So the top word is
+// at most 2^30 from 2^31 and the others too, none wraps, and the last sum is the rounding to nearest even, ties
+// included (the words above are even).  Subnormal v scale exactly; what vanishes below 2^-1074 rounds to 0.
+// 8 instructions an element for three words; with shifts and masks of the mantissa in 64-bit halves it was about
+// 60, and 35 for two words.  With sym_float, split on MI355X, us: 2048 x 200000 by 200000 x 2048 s = 24 5380 ->
+// 5215, 256 products of 64 .. 4096 with 17 to 24 moduli 1882 -> 1712, 1024^3 s = 14 14.7 -> 11.9, 1537 x 771 x
+// 3001 s = 15 36.6 -> 31.5, complex 4096^2 twice s = 16 510 -> 454, complex 777 x 1023 x 515 39 -> 23.
 // zero: the element is outside the matrix or its row is non-finite, giving x = 0.
 template <Limbs F>
 OZ2_HD void to_limbs(uint64_t bits, int e, bool zero, uint32_t (&a)[4]) {
-    const bool neg = (bits >> 63) != 0 && !zero;
-    if (F != Limbs::Octets8) {  // mag <= 2^100; the high word of u is 2^(OFF - 64) +- hi
-        constexpr int kTop = F == Limbs::Octets12 ? 31 : 40;
-        uint64_t hi = 0, lo = 0;
-        if (!zero) scaled_mag(bits, e, hi, lo);
-        uint64_t uh, ul;
-        if (neg) {
-            ul = 0 - lo;
-            uh = (1ull << kTop) - hi - (lo != 0 ? 1 : 0);
-        } else {
-            ul = lo;
-            uh = (1ull << kTop) + hi;
-        }
-        a[0] = static_cast<uint32_t>(ul);
-        a[1] = static_cast<uint32_t>(ul >> 32);
-        a[2] = static_cast<uint32_t>(uh);
-        a[3] = static_cast<uint32_t>(uh >> 32);
-    } else {  // mag <= 2^62
-        const uint64_t lo = zero ? 0 : scaled_mag62(bits, e);
-        const uint64_t ul = neg ? (1ull << 62) - lo : (1ull << 62) + lo;
-        a[0] = static_cast<uint32_t>(ul);
-        a[1] = static_cast<uint32_t>(ul >> 32);
-        a[2] = a[3] = 0;
+    double y = ldexp_(__builtin_bit_cast(double, zero ? uint64_t{0} : bits), e);
+    OZ2_UNROLL
+    for (int w = kLimbWords<F> - 1; w >= 0; --w) {
+        const double c = (6755399441055744.0 + 2147483648.0) * (w > 2 ? 0x1p93 : w > 1 ? 0x1p62 : w > 0 ? 0x1p31 : 1.0);
+        const double t = y + c;
+        a[w] = static_cast<uint32_t>(__builtin_bit_cast(uint64_t, t));
+        y -= t - c;
     }
 }
 
@@ -189,26 +167,63 @@ OZ2_HD uint32_t sym_m23(uint32_t w, uint32_t m, uint32_t mu, uint32_t h2) {
     return mad_i24(static_cast<int32_t>(q), -static_cast<int32_t>(m), w);
 }
 
-// Symmetric residue r - h of x for modulus index t >= 1 (m <= 255), r = (x + h) mod m,
-// as a 32-bit value whose low byte is the int8 plane entry, from the octets of
-// u = 2^OFF + x: v = (h - 2^OFF mod m) + sum_j byte_j(u) (2^(8 j) mod m) <= 16 * 255 * 254
-// + 254 < 2^20, one v_dot4 per word.  The chain starts at off - h (mod 2^32), so it
-// yields w = v - h for sym_m23.
+OZ2_HD float as_float(uint32_t x) { return __builtin_bit_cast(float, x); }
+// Low byte: v - m round(v / m), the symmetric residue of v, for F = v + B (B = TabSet::fb) as the bits of a float
+// in [2^23, 2^24): F is 2^23 ulps up, so a chain of integer additions that starts at the bits of B's float leaves
+// the float itself.  One fma with 1.5 2^23 rounds F / m to the integer in its low bits.  B is a multiple of m;
+// F 2^-24 / m is up to half the distance of a quotient from its tie, so whether rounding 1/m to a float moves a
+// quotient over one depends on m: for the moduli in use none of the chains' values does (all checked in the tests)
+// except with m = 255, which takes sym_m23.  The high byte of the fma's bits does not enter, 2^22 m and 2^23 are
+// multiples of 256.
+OZ2_HD uint32_t sym_float(uint32_t F, uint32_t m, float rm) {
+    const uint32_t q = __builtin_bit_cast(uint32_t, __builtin_fmaf(as_float(F), rm, 12582912.0f));
+    return mad_i24(static_cast<int32_t>(q), -static_cast<int32_t>(m), F);
+}
+
+// Chain of x's words for modulus index t from `start`: start + sum over the octets of (2^(31 w + 8 j) mod m)
 template <Limbs F, typename Tab>
-OZ2_HD uint32_t sym_residue(const uint32_t (&a)[4], Tab tb, int t) {
-    constexpr int f = static_cast<int>(F);
-    uint32_t w = udot4(a[0], tb->c8[t][0], tb->offh[f][t]);
+OZ2_HD uint32_t octet_chain(const uint32_t (&a)[4], Tab tb, int t, uint32_t start) {
+    uint32_t w = udot4(a[0], tb->c8[t][0], start);
     w = udot4(a[1], tb->c8[t][1], w);
     if (kLimbWords<F> > 2) w = udot4(a[2], tb->c8[t][2], w);
     if (kLimbWords<F> > 3) w = udot4(a[3], tb->c8[t][3], w);
-    return sym_m23(w, tb->m[t], tb->mu[t], tb->h2[t]);
+    return w;
 }
 
-// int8 byte of the symmetric residue of x for modulus index t (m = 256 only at t = 0)
+// Symmetric residues (low byte) of x, of y and of x + y for modulus index t >= 1 (m <= 255).
+//   EXACT, t = 1 (m = 255 in the sets of up to six moduli) and four words: w = v - h by sym_m23 with v = x + h (mod m), v < 2^20;
+//   else sym_float: one instruction less, also for the sum.
+template <Limbs F>
+inline constexpr bool kFloatResidues = F != Limbs::Octets14;
+template <Limbs F, bool EXACT, typename Tab>
+OZ2_HD uint32_t sym_residue(const uint32_t (&a)[4], Tab tb, int t) {
+    constexpr int f = static_cast<int>(F);
+    if (EXACT) return sym_m23(octet_chain<F>(a, tb, t, tb->offh[f][t]), tb->m[t], tb->mu[t], tb->h2[t]);
+    return sym_float(octet_chain<F>(a, tb, t, tb->fstart[f][t]), tb->m[t], tb->rm[t]);
+}
+template <Limbs F, bool EXACT, typename Tab>
+OZ2_HD void sym_residues(const uint32_t (&a)[4], const uint32_t (&b)[4], Tab tb, int t, uint32_t (&out)[3]) {
+    constexpr int f = static_cast<int>(F);
+    const uint32_t m = tb->m[t];
+    if (EXACT) {
+        const uint32_t mu = tb->mu[t], h2 = tb->h2[t];
+        out[0] = sym_m23(octet_chain<F>(a, tb, t, tb->offh[f][t]), m, mu, h2);
+        out[1] = sym_m23(octet_chain<F>(b, tb, t, tb->offh[f][t]), m, mu, h2);
+        out[2] = sym_m23(out[0] + out[1] + m, m, mu, h2);  // both in [-h, h]: v = the sum + m + h > 0
+        return;
+    }
+    const uint32_t x = octet_chain<F>(a, tb, t, tb->fstart[f][t]), y = octet_chain<F>(b, tb, t, tb->fstart[f][t]);
+    const float rm = tb->rm[t];
+    out[0] = sym_float(x, m, rm);
+    out[1] = sym_float(y, m, rm);
+    out[2] = sym_float(x + y - tb->fb[t], m, rm);
+}
+
+// int8 byte of the symmetric residue of x for modulus index t (m = 256 only at t = 0, m = 255 only at t = 1)
 template <Limbs F, typename Tab>
 OZ2_HD uint32_t sym_byte(const uint32_t (&a)[4], Tab tb, int t) {
-    if (t == 0) return a[0] & 0xFFu;  // m = 256: x mod 256 = u mod 256
-    return sym_residue<F>(a, tb, t) & 0xFFu;
+    if (t == 0) return a[0] & 0xFFu;  // m = 256: the words' units are multiples of it
+    return (t == 1 || !kFloatResidues<F> ? sym_residue<F, true>(a, tb, t) : sym_residue<F, false>(a, tb, t)) & 0xFFu;
 }
 
 // the low bytes of b0..b3 packed into one word (b0 lowest): two v_perm_b32 (each
@@ -231,13 +246,6 @@ OZ2_HD uint32_t pack_lo_halves(uint32_t a, uint32_t b) {
 #endif
 }
 
-// symmetric residue value in [-h, m-1-h] (complex split needs the value, not the byte)
-template <Limbs F, typename Tab>
-OZ2_HD int32_t sym_value(const uint32_t (&a)[4], Tab tb, int t) {
-    if (t == 0) return static_cast<int32_t>((a[0] + 127u) & 0xFFu) - 127;
-    return static_cast<int32_t>(sym_residue<F>(a, tb, t));
-}
-
 // GEMM epilogue: int32 dot product x of one k-chunk -> x mod m in [0, m), m <= 255.  A chunk holds at most
 // kMaxKChunk = 65408 k, so |x| <= 65408 * 2^14 <= 2^30 - 2^21, and with c30 = m ceil(2^30 / m) in
 // [2^30, 2^30 + m) the value u = x + c30 lies in [0, 2^31) and keeps x's residue; the sums start at c30, so u
@@ -250,14 +258,6 @@ OZ2_HD uint32_t residue_word(uint32_t u, uint32_t m, uint32_t mg) {
 template <typename Tab>
 OZ2_HD uint32_t acc_residue(uint32_t x, Tab tb, int t) {
     return residue_word(x + tb->c30[t], tb->m[t], tb->mg[t]) & 0xFFu;
-}
-
-OZ2_HD double ldexp_(double v, int e) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    return __builtin_amdgcn_ldexp(v, e);
-#else
-    return std::ldexp(v, e);
-#endif
 }
 
 // Exact reconstruction of one entry from its limb and quotient sums (as rows of the

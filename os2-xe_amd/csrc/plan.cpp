@@ -155,13 +155,18 @@ void make_tabsets(TabSet* out) {
             tb.m[t] = m;
             tb.mu[t] = static_cast<uint32_t>(((uint64_t{1} << 31) + m - 1) / m);
             tb.h[t] = h;
-            const int offs[3] = {62, 95, 104};
+            tb.rm[t] = 1.0f / static_cast<float>(m);
+            tb.fb[t] = 0x4B000000u + (m * (((1u << 23) + m - 1) / m) - (1u << 23));
+            uint32_t K = pow2_mod(31, m) + pow2_mod(62, m);  // two words
             for (int f = 0; f < 3; ++f) {
-                tb.off[f][t] = (m - pow2_mod(offs[f], m) + h) % m;
-                tb.offh[f][t] = tb.off[f][t] - h;
+                const uint32_t minus = (m - K % m) % m;
+                tb.offh[f][t] = (minus + h) % m - h;
+                tb.fstart[f][t] = tb.fb[t] + minus;
+                K += pow2_mod(31 * (f + 3), m);
             }
             tb.h2[t] = 2 * h;
-            for (int j = 0; j < 16; ++j) tb.c8[t][j >> 2] |= static_cast<uint32_t>(pow2_mod(8 * j, m)) << (8 * (j & 3));
+            for (int j = 0; j < 16; ++j)
+                tb.c8[t][j >> 2] |= static_cast<uint32_t>(pow2_mod(31 * (j >> 2) + 8 * (j & 3), m)) << (8 * (j & 3));
             tb.c30[t] = m == 256 ? 0 : m * static_cast<uint32_t>(((uint64_t{1} << 30) + m - 1) / m);
             tb.mg[t] = m == 256 ? 0 : static_cast<uint32_t>(((uint64_t{1} << 39) + m - 1) / m);
             // balanced digits in [-128, 127]; the carry out of the last one is dropped (mod 2^(32 NL))

@@ -15,9 +15,9 @@ inline constexpr int kMaxModuli = 24;
 inline constexpr int kMinModuli = 2;
 inline constexpr int kMaxLimbs = 6;           // 32-bit words of M for s = 24
 inline constexpr int kMaxScaleBits = 100;     // tk cap (hpp:29)
-inline constexpr int kNarrowScaleBits = 62;   // tk <= 62: |x| < 2^63 (hpp:30)
-inline constexpr int kWideScaleBits = 94;     // tk <= 94: 2^95 + x fits 96 bits (every plan has tk <= 91)
-// octet form of the split for a scaling width tk: 0 (8 octets), 1 (12), 2 (14)
+inline constexpr int kNarrowScaleBits = 61;   // tk <= 61: two words of base 2^31 (to_limbs in math.hpp; hpp:30)
+inline constexpr int kWideScaleBits = 92;     // tk <= 92: three (every plan has tk <= 91)
+// form of the split for a scaling width tk: 0 (two words), 1 (three), 2 (four)
 constexpr int limb_form(int tk) { return tk <= kNarrowScaleBits ? 0 : tk <= kWideScaleBits ? 1 : 2; }
 inline constexpr int32_t kNonFinite = INT32_MIN;
 // k-chunks of the INT8 GEMM.  The reference splits k at 131071 (hpp:32), the
@@ -89,10 +89,15 @@ struct TabSet {
     uint32_t m[kMaxModuli];
     uint32_t mu[kMaxModuli];                // ceil(2^31 / m): exact quotients of values below 2^23 (mod_m23)
     uint32_t h[kMaxModuli];                 // (m - 1) / 2
-    uint32_t off[3][kMaxModuli];            // (m - 2^OFF mod m + h) mod m, OFF = 62, 95, 104 (limb_form 0, 1, 2)
-    uint32_t offh[3][kMaxModuli];           // off - h (mod 2^32): start of the symmetric split's dot chain
+    uint32_t offh[3][kMaxModuli];           // (h - K mod m) mod m - h (mod 2^32), K = the words' offsets 2^31 2^(31 w) of
+                                            // limb_form 0, 1, 2: start of the dot chain that ends at sym_m23
     uint32_t h2[kMaxModuli];                // 2 h
-    uint32_t c8[kMaxModuli][4];             // bytes 2^(8 j) mod m, j = 0..15, four to a word (low first)
+    uint32_t c8[kMaxModuli][4];             // [word w] bytes 2^(31 w + 8 j) mod m, j = 0..3 (low first)
+    // the chain that ends at sym_float (m <= 253): float 1 / m, bits of the float B = m ceil(2^23 / m), and the
+    // chain's start, those bits + (-K mod m)
+    float rm[kMaxModuli];
+    uint32_t fb[kMaxModuli];
+    uint32_t fstart[3][kMaxModuli];
     uint32_t c30[kMaxModuli];               // m * ceil(2^30 / m) (GEMM residue epilogue offset; 0 for m = 256)
     uint32_t mg[kMaxModuli];                // ceil(2^39 / m): exact quotients of values below 2^31 (0 for m = 256)
     // CRT (hpp:222-236), of C' 2^up with up = 32 NL - bits(M): its sign bit is then the top bit of NL words

@@ -14,6 +14,7 @@
 // with lanes along rows, so no separate transpose pass is needed.
 #include <algorithm>
 #include <stdexcept>
+#include <type_traits>
 
 #include "grouped.hpp"
 #include "kernels.hpp"
@@ -35,19 +36,23 @@ __device__ __forceinline__ uint64_t absbits(const double* p) {
     return __double_as_longlong(*p) & 0x7FFFFFFFFFFFFFFFll;
 }
 
-// One wave per row of op(X), row contiguous in memory: n doubles from base.
-struct ScaleKcItem {
+// Maximum of every row of op(X).  Rows strided in memory over several k-blocks leave a partial maximum each.
+struct ScaleItem {
     const double* X;
-    int64_t ldx, len, ndbl;
-    int cplx, tk;
+    int64_t ldx, len, k;
+    int64_t kper;         // strided rows: k of a block
+    int kcontig, cplx, tk, nkb;
+    uint64_t* partial;    // strided rows with nkb > 1
     int32_t* ex;
-    uint32_t gx;
+    uint32_t gx;          // blocks along the rows
+    uint32_t blocks;
 };
-__device__ __forceinline__ void scale_kcontig_body(const ScaleKcItem& it, uint32_t bx) {
+// One wave per row of op(X), row contiguous in memory: n doubles from base.
+__device__ __forceinline__ void scale_kcontig_body(const ScaleItem& it, uint32_t bx) {
     const int lane = threadIdx.x & 63;
     const int64_t r = static_cast<int64_t>(bx) * 4 + (threadIdx.x >> 6);
     if (r >= it.len) return;
-    const int64_t ndbl = it.ndbl;
+    const int64_t ndbl = it.cplx ? 2 * it.k : it.k;
     const double* row = it.X + (it.cplx ? 2 : 1) * r * it.ldx;
     uint64_t mx = 0;
     if ((reinterpret_cast<uintptr_t>(row) & 15) == 0) {
@@ -88,15 +93,9 @@ __device__ __forceinline__ void scale_kcontig_body(const ScaleKcItem& it, uint32
     if (lane == 0) it.ex[r] = exponent_from_maxbits(mx, it.tk);
 }
 
-// Rows strided in memory: block = 64 rows x 4 k-lanes over a k range; partial max per (k block, row).
-struct ScaleKsItem {
-    const double* X;
-    int64_t ldx, len, k, kper;
-    int cplx;
-    uint64_t* partial;
-    uint32_t gx;
-};
-__device__ __forceinline__ void scale_kstrided_body(const ScaleKsItem& it, uint32_t bx, uint32_t by) {
+// Rows strided in memory: block = 64 rows x 4 k-lanes over a k range; partial max per (k block, row), the
+// exponent itself with one k block.
+__device__ __forceinline__ void scale_kstrided_body(const ScaleItem& it, uint32_t bx, uint32_t by) {
     __shared__ uint64_t red[4][64];
     const int rl = threadIdx.x & 63, kl = threadIdx.x >> 6;
     const int64_t r = static_cast<int64_t>(bx) * 64 + rl;
@@ -140,18 +139,17 @@ __device__ __forceinline__ void scale_kstrided_body(const ScaleKsItem& it, uint3
     __syncthreads();
     if (kl == 0 && r < it.len) {
         mx = max(max(red[0][rl], red[1][rl]), max(red[2][rl], red[3][rl]));
-        it.partial[static_cast<int64_t>(by) * it.len + r] = mx;
+        if (it.nkb == 1) it.ex[r] = exponent_from_maxbits(mx, it.tk);
+        else it.partial[static_cast<int64_t>(by) * it.len + r] = mx;
     }
 }
 
-struct ScaleFinItem {
-    const uint64_t* partial;
-    int64_t len;
-    int nkb, tk;
-    int32_t* ex;
-    uint32_t gx;
-};
-__device__ __forceinline__ void scale_finalize_body(const ScaleFinItem& it, uint32_t bx) {
+__device__ __forceinline__ void scale_body(const ScaleItem& it, uint32_t l) {
+    if (it.kcontig) scale_kcontig_body(it, l);
+    else scale_kstrided_body(it, l % it.gx, l / it.gx);
+}
+
+__device__ __forceinline__ void scale_finalize_body(const ScaleItem& it, uint32_t bx) {
     const int64_t r = static_cast<int64_t>(bx) * 256 + threadIdx.x;
     if (r >= it.len) return;
     uint64_t mx = 0;
@@ -166,23 +164,34 @@ __device__ __forceinline__ void scale_finalize_body(const ScaleFinItem& it, uint
     it.ex[r] = exponent_from_maxbits(mx, it.tk);
 }
 
-__global__ void __launch_bounds__(256) scale_kcontig_kernel(ScaleKcItem it, uint64_t* ts) {
+// Both operands of a product in one launch: the first a.blocks blocks are a's.  A launch of its own for each
+// costs 3 us where the operands are small, and leaves the chip half empty.  MI355X, scale and split of both, us,
+// launches of their own / together (exponents from partials in the split included): 64^3 s = 16 23.5 / 9.4,
+// 1024^3 s = 14 32 / 22, 4096 x 256 by 256 x 4096 s = 16 40 / 21.
+__global__ void __launch_bounds__(256) scale_kernel(ScaleItem a, ScaleItem b, uint64_t* ts) {
     const Stamp st(ts);
-    scale_kcontig_body(it, blockIdx.x);
+    const bool second = blockIdx.x >= a.blocks;
+    const ScaleItem it = second ? b : a;
+    scale_body(it, second ? blockIdx.x - a.blocks : blockIdx.x);
     st.end();
 }
-__global__ void __launch_bounds__(256) scale_kstrided_kernel(ScaleKsItem it, uint64_t* ts) {
+// ex of the rows of a and of b from their partials; na blocks are a's
+__global__ void __launch_bounds__(256) scale_finalize_kernel(ScaleItem a, ScaleItem b, uint32_t na, uint64_t* ts) {
     const Stamp st(ts);
-    scale_kstrided_body(it, blockIdx.x, blockIdx.y);
-    st.end();
-}
-__global__ void __launch_bounds__(256) scale_finalize_kernel(ScaleFinItem it, uint64_t* ts) {
-    const Stamp st(ts);
-    scale_finalize_body(it, blockIdx.x);
+    const bool second = blockIdx.x >= na;
+    const ScaleItem it = second ? b : a;
+    scale_finalize_body(it, second ? blockIdx.x - na : blockIdx.x);
     st.end();
 }
 
 constexpr int64_t kScaleRowsPerBlock = 64;
+// Up to this many partial maxima a row the split reads them itself (512 bytes a block each, beside its 32 KB
+// of operand), instead of a launch that reduces them: 2.2 to 4.3 us at k = 257 to 4096, where calls take 50 to
+// 200.  With more of them the launch's 5 to 20 us are a thousandth of the call.
+constexpr int kScaleFold = 16;
+// Blocks of a launch up to which the split deals a block's moduli to several (a quarter of the CUs: four times as
+// many still run at once).  64^3 s = 16, 2 blocks: 7.8 us an operand before, 5.2 for both.
+constexpr uint32_t kSplitFewBlocks = 64;
 
 int64_t scale_kblocks(int64_t len, int64_t k) {
     const int64_t rb = (len + kScaleRowsPerBlock - 1) / kScaleRowsPerBlock;
@@ -191,16 +200,30 @@ int64_t scale_kblocks(int64_t len, int64_t k) {
     return std::min<int64_t>(kb, 65535);
 }
 
+ScaleItem scale_item(const ScaleJob& j) {
+    ScaleItem it{j.X, j.ldx, j.len, j.k, j.k, j.kcontig ? 1 : 0, j.cplx ? 1 : 0, j.tk, 1, j.partial, j.ex, 0, 0};
+    if (j.len <= 0) return it;
+    if (j.kcontig) {
+        it.blocks = it.gx = static_cast<uint32_t>((j.len + 3) / 4);
+    } else {
+        it.nkb = static_cast<int>(scale_kblocks(j.len, j.k));
+        it.kper = (j.k + it.nkb - 1) / it.nkb;
+        it.gx = static_cast<uint32_t>((j.len + kScaleRowsPerBlock - 1) / kScaleRowsPerBlock);
+        it.blocks = it.gx * static_cast<uint32_t>(it.nkb);
+    }
+    return it;
+}
+// blocks of the launch that finalizes the item's exponents: none where the scale kernel wrote them or the split does
+uint32_t finalize_blocks(const ScaleJob& j, const ScaleItem& it) {
+    return it.blocks && it.nkb > 1 && !(j.fold && scale_folds(j.len, j.k, j.kcontig)) ? static_cast<uint32_t>((j.len + 255) / 256) : 0;
+}
+
 // ---------------------------------------------------------------------------
 // split
 // ---------------------------------------------------------------------------
 
-// Bit pattern of op(X)[r][p] for a row that exists (r < rows) and p < k.
-template <bool KCONTIG, bool CPLX>
-__device__ __forceinline__ uint64_t load_bits(const double* __restrict__ X, int64_t ldx, int64_t r, int64_t p, int part) {
-    const int64_t i = KCONTIG ? r * ldx + p : r + p * ldx;
-    return static_cast<uint64_t>(__double_as_longlong(CPLX ? X[2 * i + part] : X[i]));
-}
+__device__ __forceinline__ uint64_t bits_of(const double* p) { return static_cast<uint64_t>(__double_as_longlong(*p)); }
+__device__ __forceinline__ uint64_t word64(uint32_t lo, uint32_t hi) { return static_cast<uint64_t>(lo) | (static_cast<uint64_t>(hi) << 32); }
 
 // Thread slot of a split: Q bytes (Q = 16: a whole 16-byte chunk, Q = 8: half of one) of
 // one row of the planes.  ck counts the slots along the row.
@@ -222,23 +245,66 @@ struct SplitSlot {
     __device__ __forceinline__ int64_t k_of(int q) const { return kb + 8 * ((q0 + q) >> 1) + ((q0 + q) & 1); }
 };
 
-// (row, slot) of a thread.  KCONTIG: row r is contiguous (X[p + r*ldx]); a block
-// covers 256 slots along the row(s).  !KCONTIG: rows strided (X[r + p*ldx]); a block
-// is one 64-k block of 4 bands (2 for half chunks), lanes along rows, so a wave (16 rows x 4 slots)
-// reads one 128-byte line per load, and the block 512 bytes of a column, and writes a run of plane blocks.
-template <bool KCONTIG, int Q>
-__device__ __forceinline__ void split_thread(int lg_tpr, uint32_t bx, uint32_t by, int64_t& r, int64_t& ck) {
-    if (KCONTIG) {
-        const int tpr = 1 << lg_tpr;  // threads per row in a block
-        r = static_cast<int64_t>(bx) * (256 >> lg_tpr) + (threadIdx.x >> lg_tpr);
-        ck = static_cast<int64_t>(by) * tpr + (threadIdx.x & (tpr - 1));
-    } else {
+// A split of one operand.  Rows contiguous in memory (X[p + r*ldx]): a block covers 256 slots, 1 << lg of
+// each row.  Rows strided (X[r + p*ldx]): a block is one 64-k block of 4 bands (2 for half chunks), lanes along
+// rows, so a wave (16 rows x 4 slots) reads one 128-byte line per load, and the block 512 bytes of a column,
+// and writes a run of plane blocks.
+struct SplitItem {
+    SplitArgs a;
+    int lg;
+    int tper;         // moduli of a block (all of them, or a part where the blocks are few)
+    uint32_t gx, gy;  // blocks along the rows, along k
+    uint32_t blocks;  // gx gy, times the parts of the moduli
+};
+
+// What a thread of a split works on.
+template <int Q>
+struct SplitThread {
+    int64_t r, ck;    // row, slot
+    int t0, t1;       // moduli
+    bool ok;          // inside the planes
+    int32_t ex;       // exponent of the row (INT32_MIN outside the matrix)
+
+    __device__ __forceinline__ SplitThread(const SplitItem& it, uint32_t l) {
+        const SplitArgs& a = it.a;
+        t0 = 0;
+        t1 = a.s;
+        if (it.tper < a.s) {
+            const uint32_t per = it.gx * it.gy, g = __builtin_amdgcn_readfirstlane(l / per);
+            l -= g * per;
+            t0 = static_cast<int>(g) * it.tper;
+            t1 = min(a.s, t0 + it.tper);
+        }
+        const uint32_t by = __builtin_amdgcn_readfirstlane(l / it.gx), bx = l - by * it.gx;
         constexpr int slots = 64 / Q;
-        const int wq = threadIdx.x >> 4;  // 16 rows x one slot
-        r = static_cast<int64_t>(bx) * (256 / slots) + wq / slots * 16 + (threadIdx.x & 15);
-        ck = static_cast<int64_t>(by) * slots + wq % slots;
+        const int wq = threadIdx.x >> 4;  // strided rows: 16 rows x one slot
+        if (a.kcontig) {
+            r = static_cast<int64_t>(bx) * (256 >> it.lg) + (threadIdx.x >> it.lg);
+            ck = (static_cast<int64_t>(by) << it.lg) + (threadIdx.x & ((1 << it.lg) - 1));
+        } else {
+            r = static_cast<int64_t>(bx) * (256 / slots) + wq / slots * 16 + (threadIdx.x & 15);
+            ck = static_cast<int64_t>(by) * slots + wq % slots;
+        }
+        ok = r < a.rows_pad && ck < a.kp / Q;
+        const bool in = ok && r < a.rows;
+        ex = INT32_MIN;
+        if (a.part) {
+            // the row's maximum from the scale kernel's partials: the four lanes of a wave that hold the row
+            // (16 apart) take every fourth
+            uint64_t mx = 0;
+            if (in)
+                for (int b = (threadIdx.x >> 4) & 3; b < a.nkb; b += 4) mx = max(mx, a.part[static_cast<int64_t>(b) * a.part_ld + r]);
+            mx = max(mx, shfl_xor_u64(mx, 16));
+            mx = max(mx, shfl_xor_u64(mx, 32));
+            if (in) {
+                ex = exponent_from_maxbits(mx, a.tk);
+                if (ck == 0 && t0 == 0) a.ex_out[r] = ex;
+            }
+        } else if (in) {
+            ex = a.ex[r];
+        }
     }
-}
+};
 
 // Q bytes packed little-endian from 32-bit words: one Q-byte store
 template <int Q>
@@ -251,161 +317,161 @@ __device__ __forceinline__ void store_bytes(int8_t* p, const uint32_t (&w)[4]) {
 // Q-byte store per plane.  All loads are issued before any arithmetic and stay
 // inside the matrix: padding rows read row 0 and k past the end reads k - 1, and
 // those values are then zeroed.
-template <int FORM, bool KCONTIG, int Q>
-__device__ __forceinline__ void split_real_body(const SplitArgs& a, int lg_tpr, uint32_t bx, uint32_t by) {
+template <int FORM, int Q>
+__device__ __forceinline__ void split_real_body(const SplitItem& it, uint32_t l) {
+    const SplitArgs& a = it.a;
     const auto tb = const_tab(a.tab);
-    int64_t r, ck;
-    split_thread<KCONTIG, Q>(lg_tpr, bx, by, r, ck);
-    if (r >= a.rows_pad || ck >= a.kp / Q) return;
-    const SplitSlot<Q> sl(ck);
-    const bool rowok = r < a.rows;
-    const int32_t ex = rowok ? a.ex[r] : 0;
-    const bool rowzero = !rowok || ex == INT32_MIN;
-    const int e = rowzero ? 0 : ex;
-    const int64_t rl = rowok ? r : 0;
+    const SplitThread<Q> th(it, l);
+    if (!th.ok) return;
+    const SplitSlot<Q> sl(th.ck);
+    const bool rowzero = th.ex == INT32_MIN;
+    const int e = rowzero ? 0 : th.ex;
+    const int64_t rl = th.r < a.rows ? th.r : 0;
 
     uint64_t bits[Q];
     const bool full = sl.blk * 64 + 64 <= a.k;
-    const double* rowp = a.X + rl * a.ldx;
-    if (KCONTIG && full && (reinterpret_cast<uintptr_t>(rowp + sl.kb) & 15) == 0) {
+    if (full && a.kcontig) {
+        const double* rowp = a.X + rl * a.ldx + sl.kb;
+        if ((reinterpret_cast<uintptr_t>(rowp) & 15) == 0) {
 #pragma unroll
-        for (int i = 0; i < Q / 2; ++i) {
-            const uint4 v = *reinterpret_cast<const uint4*>(rowp + sl.k_of(2 * i));
-            bits[2 * i] = static_cast<uint64_t>(v.x) | (static_cast<uint64_t>(v.y) << 32);
-            bits[2 * i + 1] = static_cast<uint64_t>(v.z) | (static_cast<uint64_t>(v.w) << 32);
+            for (int i = 0; i < Q / 2; ++i) {
+                const uint4 v = *reinterpret_cast<const uint4*>(rowp + sl.k_of(2 * i) - sl.kb);
+                bits[2 * i] = word64(v.x, v.y);
+                bits[2 * i + 1] = word64(v.z, v.w);
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < Q; ++q) bits[q] = bits_of(rowp + (sl.k_of(q) - sl.kb));
         }
     } else if (full) {
 #pragma unroll
-        for (int q = 0; q < Q; ++q) bits[q] = load_bits<KCONTIG, false>(a.X, a.ldx, rl, sl.k_of(q), 0);
+        for (int q = 0; q < Q; ++q) bits[q] = bits_of(a.X + rl + sl.k_of(q) * a.ldx);
     } else {
+        const int64_t sr = a.kcontig ? a.ldx : 1, sp = a.kcontig ? 1 : a.ldx;
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
             const int64_t p = sl.k_of(q);
-            bits[q] = load_bits<KCONTIG, false>(a.X, a.ldx, rl, p < a.k ? p : a.k - 1, 0);
+            bits[q] = bits_of(a.X + rl * sr + (p < a.k ? p : a.k - 1) * sp);
             bits[q] = p < a.k ? bits[q] : 0;
         }
     }
 
-    // the 8, 12 or 14 bytes of the offset value (limb_form of tk)
+    // two to four words (limb_form of tk)
     constexpr Limbs F = static_cast<Limbs>(FORM);
     uint32_t limbs[Q][4];
 #pragma unroll
     for (int q = 0; q < Q; ++q) to_limbs<F>(rowzero ? 0 : bits[q], e, false, limbs[q]);
-    int8_t* out = a.P + chunk_offset(r, sl.blk, sl.c, a.map) + sl.q0;
+    int8_t* out = a.P + chunk_offset(th.r, sl.blk, sl.c, a.map) + sl.q0;
     uint32_t w[4] = {0, 0, 0, 0};
-    // plane 0 has m = 256 in every moduli set: its residue byte is the low byte of u
-#pragma unroll
-    for (int g = 0; g < Q / 4; ++g)
-        w[g] = pack_lo_bytes(limbs[4 * g][0], limbs[4 * g + 1][0], limbs[4 * g + 2][0], limbs[4 * g + 3][0]);
-    store_bytes<Q>(out, w);
-    for (int t = 1; t < a.s; ++t) {
+    // plane 0 has m = 256 in every moduli set (the low byte), plane 1 m = 255 (sym_residue)
+    if (th.t0 == 0) {
 #pragma unroll
         for (int g = 0; g < Q / 4; ++g)
-            w[g] = pack_lo_bytes(sym_residue<F>(limbs[4 * g], tb, t), sym_residue<F>(limbs[4 * g + 1], tb, t),
-                                 sym_residue<F>(limbs[4 * g + 2], tb, t), sym_residue<F>(limbs[4 * g + 3], tb, t));
-        store_bytes<Q>(out + t * a.plane, w);
+            w[g] = pack_lo_bytes(limbs[4 * g][0], limbs[4 * g + 1][0], limbs[4 * g + 2][0], limbs[4 * g + 3][0]);
+        store_bytes<Q>(out, w);
     }
+    auto plane = [&](int t, auto exact) {
+        constexpr bool E = decltype(exact)::value;
+#pragma unroll
+        for (int g = 0; g < Q / 4; ++g)
+            w[g] = pack_lo_bytes(sym_residue<F, E>(limbs[4 * g], tb, t), sym_residue<F, E>(limbs[4 * g + 1], tb, t),
+                                 sym_residue<F, E>(limbs[4 * g + 2], tb, t), sym_residue<F, E>(limbs[4 * g + 3], tb, t));
+        store_bytes<Q>(out + t * a.plane, w);
+    };
+    if (th.t0 <= 1 && th.t1 > 1) plane(1, std::true_type{});
+    for (int t = max(th.t0, 2); t < th.t1; ++t) plane(t, std::bool_constant<!kFloatResidues<F>>{});
 }
 
-// Complex split: three plane groups Re, Im (negated for conj), Re+Im, each
+// Complex split: three plane groups Re, Im (negated for conj: the sign of the bits), Re+Im, each
 // reduced to the symmetric range [-h, m-1-h]; slots, k order and loads as in the
 // real split, one Q-byte store per plane of each group.
-template <int FORM, bool KCONTIG, bool CONJ, int Q>
-__device__ __forceinline__ void split_cplx_body(const SplitArgs& a, int lg_tpr, uint32_t bx, uint32_t by) {
+template <int FORM, int Q>
+__device__ __forceinline__ void split_cplx_body(const SplitItem& it, uint32_t l) {
+    const SplitArgs& a = it.a;
     const auto tb = const_tab(a.tab);
-    int64_t r, ck;
-    split_thread<KCONTIG, Q>(lg_tpr, bx, by, r, ck);
-    if (r >= a.rows_pad || ck >= a.kp / Q) return;
-    const SplitSlot<Q> sl(ck);
-    const bool rowok = r < a.rows;
-    const int32_t ex = rowok ? a.ex[r] : 0;
-    const bool rowzero = !rowok || ex == INT32_MIN;
-    const int e = rowzero ? 0 : ex;
-    const int64_t rl = rowok ? r : 0;
+    const SplitThread<Q> th(it, l);
+    if (!th.ok) return;
+    const SplitSlot<Q> sl(th.ck);
+    const bool rowzero = th.ex == INT32_MIN;
+    const int e = rowzero ? 0 : th.ex;
+    const int64_t rl = th.r < a.rows ? th.r : 0;
 
     uint64_t br[Q], bi[Q];
     const bool full = sl.blk * 64 + 64 <= a.k;
-    const double* rowp = a.X + 2 * rl * a.ldx;
-    if (KCONTIG && full && (reinterpret_cast<uintptr_t>(rowp + 2 * sl.kb) & 15) == 0) {
+    const double* rowp = a.X + 2 * rl * a.ldx + 2 * sl.kb;
+    if (a.kcontig && full && (reinterpret_cast<uintptr_t>(rowp) & 15) == 0) {
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
-            const uint4 v = *reinterpret_cast<const uint4*>(rowp + 2 * sl.k_of(q));
-            br[q] = static_cast<uint64_t>(v.x) | (static_cast<uint64_t>(v.y) << 32);
-            bi[q] = static_cast<uint64_t>(v.z) | (static_cast<uint64_t>(v.w) << 32);
+            const uint4 v = *reinterpret_cast<const uint4*>(rowp + 2 * (sl.k_of(q) - sl.kb));
+            br[q] = word64(v.x, v.y);
+            bi[q] = word64(v.z, v.w);
         }
     } else {
+        const int64_t sr = a.kcontig ? a.ldx : 1, sp = a.kcontig ? 1 : a.ldx;
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
             const int64_t p = sl.k_of(q);
-            const int64_t pc = p < a.k ? p : a.k - 1;
-            br[q] = load_bits<KCONTIG, true>(a.X, a.ldx, rl, pc, 0);
-            bi[q] = load_bits<KCONTIG, true>(a.X, a.ldx, rl, pc, 1);
+            const double* x = a.X + 2 * (rl * sr + (p < a.k ? p : a.k - 1) * sp);
+            br[q] = bits_of(x);
+            bi[q] = bits_of(x + 1);
             br[q] = p < a.k ? br[q] : 0;
             bi[q] = p < a.k ? bi[q] : 0;
         }
     }
+    const uint64_t flip = a.conj ? 1ull << 63 : 0;
     constexpr Limbs F = static_cast<Limbs>(FORM);
     uint32_t lr[Q][4], li[Q][4];
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
         to_limbs<F>(rowzero ? 0 : br[q], e, false, lr[q]);
-        to_limbs<F>(rowzero ? 0 : bi[q], e, false, li[q]);
+        to_limbs<F>(rowzero ? 0 : bi[q] ^ flip, e, false, li[q]);
     }
-    int8_t* out = a.P + chunk_offset(r, sl.blk, sl.c, a.map) + sl.q0;
-    for (int t = 0; t < a.s; ++t) {
-        const int32_t m = static_cast<int32_t>(tb->m[t]);
-        const int32_t h = static_cast<int32_t>(tb->h[t]);
+    int8_t* out = a.P + chunk_offset(th.r, sl.blk, sl.c, a.map) + sl.q0;
+    // plane t of the three groups; residues(x, y, r) of an element
+    auto plane = [&](int t, const auto& residues) {
         uint32_t w0[4] = {0, 0, 0, 0}, w1[4] = {0, 0, 0, 0}, w2[4] = {0, 0, 0, 0};
 #pragma unroll
         for (int g = 0; g < Q / 4; ++g) {
-            uint32_t b0[4], b1[4], b2[4];
+            uint32_t r[4][3];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int32_t s0 = sym_value<F>(lr[4 * g + q], tb, t);
-                int32_t s1 = sym_value<F>(li[4 * g + q], tb, t);
-                if (CONJ) s1 = -s1;
-                int32_t ss = s0 + s1;
-                ss = ss > m - 1 - h ? ss - m : ss;
-                ss = ss < -h ? ss + m : ss;
-                b0[q] = static_cast<uint32_t>(s0);
-                b1[q] = static_cast<uint32_t>(s1);
-                b2[q] = static_cast<uint32_t>(ss);
-            }
-            w0[g] = pack_lo_bytes(b0[0], b0[1], b0[2], b0[3]);
-            w1[g] = pack_lo_bytes(b1[0], b1[1], b1[2], b1[3]);
-            w2[g] = pack_lo_bytes(b2[0], b2[1], b2[2], b2[3]);
+            for (int q = 0; q < 4; ++q) residues(lr[4 * g + q], li[4 * g + q], r[q]);
+            w0[g] = pack_lo_bytes(r[0][0], r[1][0], r[2][0], r[3][0]);
+            w1[g] = pack_lo_bytes(r[0][1], r[1][1], r[2][1], r[3][1]);
+            w2[g] = pack_lo_bytes(r[0][2], r[1][2], r[2][2], r[3][2]);
         }
         store_bytes<Q>(out + t * a.plane, w0);
         store_bytes<Q>(out + a.group + t * a.plane, w1);
         store_bytes<Q>(out + 2 * a.group + t * a.plane, w2);
-    }
+    };
+    typedef const uint32_t (&words)[4];
+    typedef uint32_t (&bytes)[3];
+    if (th.t0 == 0)  // m = 256: low bytes
+        plane(0, [](words x, words y, bytes r) {
+            r[0] = x[0];
+            r[1] = y[0];
+            r[2] = x[0] + y[0];
+        });
+    if (th.t0 <= 1 && th.t1 > 1) plane(1, [&](words x, words y, bytes r) { sym_residues<F, true>(x, y, tb, 1, r); });
+    for (int t = max(th.t0, 2); t < th.t1; ++t)
+        plane(t, [&](words x, words y, bytes r) { sym_residues<F, !kFloatResidues<F>>(x, y, tb, t, r); });
 }
 
-// split variants: bits 0-1 limb form (0, 1, 2), bit 2 kcontig, 3 complex, 4 conj
-struct SplitItem {
-    SplitArgs a;
-    int lg;
-    uint32_t gx;
-};
 // bytes per thread slot: half chunks for wide complex values (their 2 x 4 octet words
 // per element would not fit 16 elements in registers), whole chunks otherwise
 constexpr int split_q(int form, bool cplx) { return form != 0 && cplx ? 8 : 16; }
-template <int V>
-__device__ __forceinline__ void split_body(const SplitItem& it, uint32_t bx, uint32_t by) {
-    constexpr int FM = V & 3;
-    constexpr bool KC = (V >> 2) & 1, CX = (V >> 3) & 1, CJ = (V >> 4) & 1;
-    if constexpr (CX) split_cplx_body<FM, KC, CJ, split_q(FM, true)>(it.a, it.lg, bx, by);
-    else split_real_body<FM, KC, split_q(FM, false)>(it.a, it.lg, bx, by);
+template <int FORM, bool CPLX>
+__device__ __forceinline__ void split_body(const SplitItem& it, uint32_t l) {
+    if constexpr (CPLX) split_cplx_body<FORM, split_q(FORM, true)>(it, l);
+    else split_real_body<FORM, split_q(FORM, false)>(it, l);
 }
-template <int V>
-__global__ void __launch_bounds__(256) split_kernel(SplitItem it, uint64_t* ts) {
+// one operand, or both of a product (scale_kernel)
+template <int FORM, bool CPLX>
+__global__ void __launch_bounds__(256) split_kernel(SplitItem a, SplitItem b, uint64_t* ts) {
     const Stamp st(ts);
-    split_body<V>(it, blockIdx.x, blockIdx.y);
+    const bool second = blockIdx.x >= a.blocks;
+    const SplitItem it = second ? b : a;
+    split_body<FORM, CPLX>(it, second ? blockIdx.x - a.blocks : blockIdx.x);
     st.end();
-}
-
-int split_variant(const SplitArgs& a) {
-    return a.form | (a.kcontig ? 4 : 0) | (a.cplx ? 8 : 0) | (a.cplx && a.conj ? 16 : 0);
 }
 
 // grid of one split: KCONTIG: rows x slot groups (tpr threads per row); strided: 16 rows x 16 slots.
@@ -414,10 +480,11 @@ int split_variant(const SplitArgs& a) {
 // a plane is written by one wave.  With a whole row per workgroup (256 slots) the two
 // rows sharing a line came from different workgroups, usually on different XCDs, and
 // the L2s wrote half lines: 0.79 against 0.69 ms for both operands at 8192^3 s = 16.
-SplitItem split_item(const SplitArgs& a, uint32_t& gy) {
+SplitItem split_item(const SplitArgs& a) {
     const int q = split_q(a.form, a.cplx);
     const int64_t nck = a.kp / q;
-    SplitItem it{a, 0, 0};
+    SplitItem it{a, 0, a.s, 0, 0, 0};
+    if (a.rows_pad <= 0) return it;
     if (a.kcontig) {
         int tpr = 1;
         while (tpr < 64 / q && tpr < nck) {
@@ -425,41 +492,45 @@ SplitItem split_item(const SplitArgs& a, uint32_t& gy) {
             ++it.lg;
         }
         it.gx = static_cast<uint32_t>((a.rows_pad + (256 / tpr) - 1) / (256 / tpr));
-        gy = static_cast<uint32_t>((nck + tpr - 1) / tpr);
+        it.gy = static_cast<uint32_t>((nck + tpr - 1) / tpr);
     } else {
         const int slots = 64 / q;
         it.gx = static_cast<uint32_t>((a.rows_pad + 256 / slots - 1) / (256 / slots));
-        gy = static_cast<uint32_t>((nck + slots - 1) / slots);
+        it.gy = static_cast<uint32_t>((nck + slots - 1) / slots);
     }
+    it.blocks = it.gx * it.gy;
     return it;
 }
+// Few blocks leave the chip idle while each goes through all its moduli: they are then dealt to up to four
+// times as many, which read the operand again (from the caches).
+void split_parts(SplitItem& it, uint32_t launch_blocks) {
+    if (it.blocks == 0 || launch_blocks > kSplitFewBlocks) return;
+    it.tper = (it.a.s + 3) / 4;
+    it.blocks *= static_cast<uint32_t>((it.a.s + it.tper - 1) / it.tper);
+}
 
-template <int V>
-void launch_split_v(const Stream& st, const SplitItem& it, uint32_t gy) {
-    launch(st, split_kernel<V>, dim3(it.gx, gy), dim3(256), it);
+template <int FORM, bool CPLX>
+void launch_split(const Stream& st, const SplitItem& a, const SplitItem& b) {
+    launch(st, split_kernel<FORM, CPLX>, dim3(a.blocks + b.blocks), dim3(256), a, b);
 }
 
 // ---- grouped forms: block b of the launch runs block (b - start[p]) of item p
-enum GroupKind { kScaleKc = 0, kScaleKs = 1, kScaleFin = 2, kSplitBase = 16 };
+enum GroupKind { kScale = 0, kScaleFin = 1, kSplitBase = 16 };
 
-template <typename Item, int K>
-__global__ void __launch_bounds__(256) grouped_scale_kernel(const Item* __restrict__ items,
+template <bool FIN>
+__global__ void __launch_bounds__(256) grouped_scale_kernel(const ScaleItem* __restrict__ items,
                                                             const uint32_t* __restrict__ start, uint32_t n) {
     const uint32_t p = owner_of(start, n, blockIdx.x);
-    const Item& it = items[p];
     const uint32_t l = blockIdx.x - start[p];
-    if constexpr (K == kScaleKc) scale_kcontig_body(it, l);
-    else if constexpr (K == kScaleKs) scale_kstrided_body(it, l % it.gx, l / it.gx);
-    else scale_finalize_body(it, l);
+    if constexpr (FIN) scale_finalize_body(items[p], l);
+    else scale_body(items[p], l);
 }
 
-template <int V>
+template <int FORM>
 __global__ void __launch_bounds__(256) grouped_split_kernel(const SplitItem* __restrict__ items,
                                                             const uint32_t* __restrict__ start, uint32_t n) {
     const uint32_t p = owner_of(start, n, blockIdx.x);
-    const SplitItem& it = items[p];
-    const uint32_t l = blockIdx.x - start[p];
-    split_body<V>(it, l % it.gx, l / it.gx);
+    split_body<FORM, false>(items[p], blockIdx.x - start[p]);
 }
 
 }  // namespace
@@ -469,71 +540,67 @@ size_t scale_partial_elems(int64_t len, int64_t k, bool kcontig) {
     return static_cast<size_t>(scale_kblocks(len, k)) * static_cast<size_t>(len);
 }
 
-void scale(const Stream& st, const double* X, int64_t ldx, int64_t len, int64_t k, bool kcontig, bool cplx, int tk,
-           uint64_t* partial, int32_t* ex) {
-    if (len <= 0) return;
-    if (kcontig) {
-        const ScaleKcItem it{X, ldx, len, cplx ? 2 * k : k, cplx ? 1 : 0, tk, ex, static_cast<uint32_t>((len + 3) / 4)};
-        launch(st, scale_kcontig_kernel, dim3(it.gx), dim3(256), it);
-    } else {
-        const int64_t nkb = scale_kblocks(len, k);
-        const int64_t kper = (k + nkb - 1) / nkb;
-        const ScaleKsItem it{X, ldx, len, k, kper, cplx ? 1 : 0, partial,
-                             static_cast<uint32_t>((len + kScaleRowsPerBlock - 1) / kScaleRowsPerBlock)};
-        launch(st, scale_kstrided_kernel, dim3(it.gx, static_cast<unsigned>(nkb)), dim3(256), it);
-        const ScaleFinItem fin{partial, len, static_cast<int>(nkb), tk, ex, static_cast<uint32_t>((len + 255) / 256)};
-        launch(st, scale_finalize_kernel, dim3(fin.gx), dim3(256), fin);
-    }
+int scale_partials(int64_t len, int64_t k, bool kcontig) {
+    return kcontig || len <= 0 ? 1 : static_cast<int>(scale_kblocks(len, k));
 }
 
-void split(const Stream& st, const SplitArgs& a) {
-    uint32_t gy = 0;
-    const SplitItem it = split_item(a, gy);
-    switch (split_variant(a)) {
-#define OZ2_V(V) case V: launch_split_v<V>(st, it, gy); break;
-#define OZ2_F(F) OZ2_V(F) OZ2_V(F + 4) OZ2_V(F + 8) OZ2_V(F + 12) OZ2_V(F + 24) OZ2_V(F + 28)
-        OZ2_F(0) OZ2_F(1) OZ2_F(2)
-#undef OZ2_F
-#undef OZ2_V
+bool scale_folds(int64_t len, int64_t k, bool kcontig) {
+    const int n = scale_partials(len, k, kcontig);
+    return n > 1 && n <= kScaleFold;
+}
+
+void scale(const Stream& st, const ScaleJob& ja, const ScaleJob& jb) {
+    const ScaleItem a = scale_item(ja), b = scale_item(jb);
+    if (a.blocks + b.blocks == 0) return;
+    launch(st, scale_kernel, dim3(a.blocks + b.blocks), dim3(256), a, b);
+    const uint32_t fa = finalize_blocks(ja, a), fb = finalize_blocks(jb, b);
+    if (fa + fb) launch(st, scale_finalize_kernel, dim3(fa + fb), dim3(256), a, b, fa);
+}
+
+void split(const Stream& st, const SplitArgs& x, const SplitArgs& y) {
+    SplitItem a = split_item(x), b = split_item(y);
+    const uint32_t n = a.blocks + b.blocks;
+    if (n == 0) return;
+    split_parts(a, n);
+    split_parts(b, n);
+    switch (x.form * 2 + (x.cplx ? 1 : 0)) {
+        case 0: launch_split<0, false>(st, a, b); break;
+        case 1: launch_split<0, true>(st, a, b); break;
+        case 2: launch_split<1, false>(st, a, b); break;
+        case 3: launch_split<1, true>(st, a, b); break;
+        case 4: launch_split<2, false>(st, a, b); break;
+        case 5: launch_split<2, true>(st, a, b); break;
         default: throw std::logic_error("oz2: no split kernel for this variant");
     }
 }
 
+void split(const Stream& st, const SplitArgs& a) {
+    SplitArgs none = a;
+    none.rows_pad = 0;
+    split(st, a, none);
+}
+
 void prep_scale(std::vector<GroupedLaunch>& out, const std::vector<ScaleJob>& jobs) {
-    GroupedLaunch kc, ks, fin;
-    kc.kind = kScaleKc;
-    ks.kind = kScaleKs;
+    GroupedLaunch all, fin;
+    all.kind = kScale;
     fin.kind = kScaleFin;
     for (const ScaleJob& j : jobs) {
-        if (j.len <= 0) continue;
-        if (j.kcontig) {
-            const ScaleKcItem it{j.X, j.ldx, j.len, j.cplx ? 2 * j.k : j.k, j.cplx ? 1 : 0, j.tk, j.ex,
-                                 static_cast<uint32_t>((j.len + 3) / 4)};
-            kc.add(it, it.gx);
-        } else {
-            const int64_t nkb = scale_kblocks(j.len, j.k);
-            const int64_t kper = (j.k + nkb - 1) / nkb;
-            const ScaleKsItem it{j.X, j.ldx, j.len, j.k, kper, j.cplx ? 1 : 0, j.partial,
-                                 static_cast<uint32_t>((j.len + kScaleRowsPerBlock - 1) / kScaleRowsPerBlock)};
-            ks.add(it, it.gx * static_cast<uint32_t>(nkb));
-            const ScaleFinItem f{j.partial, j.len, static_cast<int>(nkb), j.tk, j.ex,
-                                 static_cast<uint32_t>((j.len + 255) / 256)};
-            fin.add(f, f.gx);
-        }
+        const ScaleItem it = scale_item(j);
+        if (it.blocks == 0) continue;
+        all.add(it, it.blocks);
+        if (const uint32_t f = finalize_blocks(j, it)) fin.add(it, f);
     }
-    for (GroupedLaunch* g : {&kc, &ks, &fin})
+    for (GroupedLaunch* g : {&all, &fin})
         if (g->n) out.push_back(std::move(*g));
 }
 
 void prep_split(std::vector<GroupedLaunch>& out, const std::vector<SplitArgs>& jobs) {
-    GroupedLaunch by[32];
+    GroupedLaunch by[3];
     for (const SplitArgs& a : jobs) {
-        if (a.rows_pad <= 0) continue;
-        uint32_t gy = 0;
-        const SplitItem it = split_item(a, gy);
-        const int v = split_variant(a);
-        by[v].kind = kSplitBase + v;
-        by[v].add(it, it.gx * gy);
+        const SplitItem it = split_item(a);
+        if (it.blocks == 0) continue;
+        by[a.form].kind = kSplitBase + a.form;
+        by[a.form].add(it, it.blocks);
     }
     for (GroupedLaunch& g : by)
         if (g.n) out.push_back(std::move(g));
@@ -543,26 +610,23 @@ bool launch_scale_split_grouped(hipStream_t st, const GroupedLaunch& g) {
     if (g.n == 0) return true;
     const dim3 grid(g.blocks), block(256);
     switch (g.kind) {
-        case kScaleKc:
-            hipLaunchKernelGGL((grouped_scale_kernel<ScaleKcItem, kScaleKc>), grid, block, 0, st,
-                               static_cast<const ScaleKcItem*>(g.d_items), g.d_start, g.n);
-            return true;
-        case kScaleKs:
-            hipLaunchKernelGGL((grouped_scale_kernel<ScaleKsItem, kScaleKs>), grid, block, 0, st,
-                               static_cast<const ScaleKsItem*>(g.d_items), g.d_start, g.n);
+        case kScale:
+            hipLaunchKernelGGL((grouped_scale_kernel<false>), grid, block, 0, st, static_cast<const ScaleItem*>(g.d_items),
+                               g.d_start, g.n);
             return true;
         case kScaleFin:
-            hipLaunchKernelGGL((grouped_scale_kernel<ScaleFinItem, kScaleFin>), grid, block, 0, st,
-                               static_cast<const ScaleFinItem*>(g.d_items), g.d_start, g.n);
+            hipLaunchKernelGGL((grouped_scale_kernel<true>), grid, block, 0, st, static_cast<const ScaleItem*>(g.d_items),
+                               g.d_start, g.n);
             return true;
-#define OZ2_V(V)                                                                                  \
-    case kSplitBase + V:                                                                          \
-        hipLaunchKernelGGL((grouped_split_kernel<V>), grid, block, 0, st,                         \
-                           static_cast<const SplitItem*>(g.d_items), g.d_start, g.n);             \
-        return true;
         // the batch takes real products only, whose plans all have tk <= 91 (forms 0 and 1)
-        OZ2_V(0) OZ2_V(1) OZ2_V(4) OZ2_V(5)
-#undef OZ2_V
+        case kSplitBase:
+            hipLaunchKernelGGL((grouped_split_kernel<0>), grid, block, 0, st, static_cast<const SplitItem*>(g.d_items),
+                               g.d_start, g.n);
+            return true;
+        case kSplitBase + 1:
+            hipLaunchKernelGGL((grouped_split_kernel<1>), grid, block, 0, st, static_cast<const SplitItem*>(g.d_items),
+                               g.d_start, g.n);
+            return true;
         default: return false;
     }
 }

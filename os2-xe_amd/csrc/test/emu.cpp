@@ -45,18 +45,12 @@ void split_cplx_form(const double* re, const double* im, const int32_t* e, int64
         const bool zero = e[i] == INT32_MIN;
         const int ee = zero ? 0 : e[i];
         math::to_limbs<F>(br, ee, zero, ar);
-        math::to_limbs<F>(bi, ee, zero, ai);
+        math::to_limbs<F>(conj ? bi ^ (uint64_t{1} << 63) : bi, ee, zero, ai);
         for (int t = 0; t < s; ++t) {
-            const int32_t m = static_cast<int32_t>(tb->m[t]), h = static_cast<int32_t>(tb->h[t]);
-            const int32_t s0 = math::sym_value<F>(ar, tb, t);
-            int32_t s1 = math::sym_value<F>(ai, tb, t);
-            if (conj) s1 = -s1;
-            int32_t ss = s0 + s1;
-            ss = ss > m - 1 - h ? ss - m : ss;
-            ss = ss < -h ? ss + m : ss;
-            planes[(0 * s + t) * n + i] = static_cast<int8_t>(s0);
-            planes[(1 * s + t) * n + i] = static_cast<int8_t>(s1);
-            planes[(2 * s + t) * n + i] = static_cast<int8_t>(ss);
+            uint32_t r[3] = {ar[0], ai[0], ar[0] + ai[0]};
+            if (t == 1 || (t && !math::kFloatResidues<F>)) math::sym_residues<F, true>(ar, ai, tb, t, r);
+            else if (t) math::sym_residues<F, false>(ar, ai, tb, t, r);
+            for (int g = 0; g < 3; ++g) planes[(g * s + t) * n + i] = static_cast<int8_t>(r[g]);
         }
     }
 }
@@ -95,7 +89,8 @@ int64_t emu_mod_m23_mismatches(int s, int t) {
 }
 
 // symmetric split reduction of modulus t of s over every dot-chain value v < 2^20 + 2^8
-// (w = v - h as the chain leaves it): entries that differ from (v mod m) - h
+// (w = v - h as the chain leaves it): entries that differ from (v mod m) - h; and sym_float over every value of
+// a chain of three words and of the sum of two, where it is used
 int64_t emu_sym_m23_mismatches(int s, int t) {
     const TabSet* tb = tables() + s;
     const uint32_t m = tb->m[t], h = tb->h[t];
@@ -103,6 +98,14 @@ int64_t emu_sym_m23_mismatches(int s, int t) {
     for (uint32_t v = 0; v < (1u << 20) + 256; ++v) {
         const int32_t got = static_cast<int32_t>(math::sym_m23(v - h, m, tb->mu[t], tb->h2[t]));
         bad += got != static_cast<int32_t>(v % m) - static_cast<int32_t>(h);
+    }
+    if (t < 2) return bad;
+    uint32_t most = m;
+    for (int w = 0; w < 3; ++w)
+        for (int j = 0; j < 32; j += 8) most += 255 * ((tb->c8[t][w] >> j) & 0xFFu);
+    for (uint32_t v = 0; v <= 2 * most; ++v) {
+        const int8_t got = static_cast<int8_t>(math::sym_float(tb->fb[t] + v, m, tb->rm[t]));
+        bad += got != static_cast<int32_t>((v + h) % m) - static_cast<int32_t>(h);
     }
     return bad;
 }

@@ -1,0 +1,37 @@
+"""Scale and split of both operands in one launch, bit for bit against the oracle, at the sizes where its forms
+change: one partial maximum a row or several, read by the split or reduced by a launch; moduli of a block dealt to
+several blocks; rows strided or contiguous on either side, odd sizes and leading dimensions."""
+import pytest
+
+import oz2
+from gpu_cases import complex_case, real_case
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def oz():
+    h = oz2.Ozaki2()
+    yield h
+    h.close()
+
+
+# k: one partial up to 256, two at 257, sixteen up to 4096, then the reducing launch
+@pytest.mark.parametrize("k", [1, 256, 257, 515, 4096, 4097])
+@pytest.mark.parametrize("ta,tb", [("N", "T"), ("N", "N"), ("T", "N"), ("T", "T")])
+def test_partials(oz, ta, tb, k):
+    real_case(oz, ta, tb, 67, 33, k, 16, "wide", -1.0, 1.0, lda_extra=1, ldc_extra=1, check_bound=False)
+    real_case(oz, ta, tb, 65, 129, k, 21, "u11", check_bound=False)
+
+
+# 64 blocks of the two splits and fewer go to parts of the moduli: rows / 64 times k / 64, both operands padded
+@pytest.mark.parametrize("m,n,k", [(1, 1, 1), (64, 64, 64), (512, 512, 256), (512, 576, 256), (640, 512, 256), (1000, 24, 500)])
+@pytest.mark.parametrize("s", [2, 3, 9, 24])
+def test_parts(oz, m, n, k, s):
+    real_case(oz, "N", "N", m, n, k, max(s, 4) if k > 64 else s, "uniform", check_bound=False)
+
+
+@pytest.mark.parametrize("ta,tb", [("N", "C"), ("C", "N"), ("T", "C"), ("N", "N")])
+@pytest.mark.parametrize("k,s", [(130, 16), (300, 24), (1200, 9)])
+def test_complex(oz, ta, tb, k, s):
+    complex_case(oz, ta, tb, 70, 130, k, s, "uniform", 1.5 - 0.5j, 0.5j, ld_extra=1, check_bound=False)
