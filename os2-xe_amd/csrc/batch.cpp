@@ -136,10 +136,10 @@ BatchPlan::BatchPlan(Engine& eng, std::vector<GemmDesc> descs, const std::vector
                 a.X = which == 0 ? g.A : g.B;
                 a.ldx = which == 0 ? g.lda : g.ldb;
                 a.rows = which == 0 ? g.m : g.n;
-                a.rows_pad = which == 0 ? q.mpad : q.npad;
+                a.rows_pad = round_up(a.rows, q.ftile ? q.ftile : which == 0 ? k::tile_pad_m(q.tile) : k::tile_pad_n(q.tile));
                 a.k = g.k;
                 a.kp = q.kp;
-                a.map = k::PlaneMap::of(q.tile, q.ftile, a.rows_pad, q.kp);
+                a.map = k::PlaneMap::of(q.tile, q.ftile, which == 0 ? q.mpad : q.npad, q.kp);
                 a.ex = a.ex_out = which == 0 ? D : E;
                 if (k::scale_folds(a.rows, a.k, a.kcontig)) {
                     a.part = sj[sj.size() - 2 + which].partial;
@@ -223,6 +223,8 @@ BatchPlan::BatchPlan(Engine& eng, std::vector<GemmDesc> descs, const std::vector
                 a.R = reinterpret_cast<uint8_t*>(base + q.oR) + c * s_[i] * q.planeR;
                 a.tiles_m = static_cast<int>(q.mpad / k::tile_m(q.tile));
                 a.tiles_n = static_cast<int>(q.npad / k::tile_n(q.tile));
+                a.rows = round_up(d_[i].m, k::tile_pad_m(q.tile));
+                a.cols = round_up(d_[i].n, k::tile_pad_n(q.tile));
                 a.nplanes = s_[i];
                 a.s = s_[i];
                 a.tab = tabs + s_[i];

@@ -548,6 +548,8 @@ int oz2_unit_gemm(void* stream, const int8_t* A, const int8_t* B, int64_t mpad, 
         a.klen = kp;
         a.tiles_m = static_cast<int>(mpad / TM);
         a.tiles_n = static_cast<int>(npad / TN);
+        a.rows = mpad;
+        a.cols = npad;
         a.nplanes = num_moduli;
         a.plane0 = 0;
         a.s = num_moduli;

@@ -360,7 +360,7 @@ void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, doubl
         sp.X = sp.kcontig ? X + cw * r0 * ldx : X + cw * r0;
         sp.ldx = ldx;
         sp.rows = rows;
-        sp.rows_pad = round_up(rows, ftile ? ftile : is_b ? L.TN : L.TM);
+        sp.rows_pad = round_up(rows, ftile ? ftile : is_b ? k::tile_pad_n(tile_) : k::tile_pad_m(tile_));
         sp.k = k;
         sp.kp = kp;
         sp.ex = sp.ex_out = (is_b ? E : D) + r0;
@@ -394,6 +394,8 @@ void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, doubl
         ga.ldr = L.mpad;
         ga.tiles_m = static_cast<int>((rows + L.TM - 1) / L.TM);
         ga.tiles_n = static_cast<int>((cols + L.TN - 1) / L.TN);
+        ga.rows = round_up(rows, k::tile_pad_m(tile_));
+        ga.cols = round_up(cols, k::tile_pad_n(tile_));
         ga.nplanes = L.planes;
         ga.s = s;
         ga.tab = tab;
@@ -585,6 +587,8 @@ void Engine::ozaki1(int64_t m, int64_t n, int64_t k, const double* A, int64_t ld
         ga.ldr = mpad;
         ga.tiles_m = static_cast<int>(mpad / TM);
         ga.tiles_n = static_cast<int>(npad / TN);
+        ga.rows = mpad;
+        ga.cols = npad;
         ga.nplanes = 1;
         ga.s = kMinModuli;
         ga.tab = dtabs_ + kMinModuli;

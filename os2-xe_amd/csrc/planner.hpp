@@ -30,6 +30,10 @@ namespace k {
 enum class Tile { T256 = 0, T128 = 1, T64 = 2, T256x128 = 3 };
 constexpr int tile_m(Tile t) { return t == Tile::T256 || t == Tile::T256x128 ? 256 : t == Tile::T128 ? 128 : 64; }
 constexpr int tile_n(Tile t) { return t == Tile::T256 ? 256 : t == Tile::T64 ? 64 : 128; }
+// Tiles of 128 x 128 and 256 x 128 take a half tile at an edge where it holds all that is left (gemm_edge in
+// igemm.hip): operands are padded to these multiples.
+constexpr int tile_pad_m(Tile t) { return t == Tile::T128 || t == Tile::T256x128 ? tile_m(t) / 2 : tile_m(t); }
+constexpr int tile_pad_n(Tile t) { return t == Tile::T128 || t == Tile::T256x128 ? tile_n(t) / 2 : tile_n(t); }
 constexpr int tile_code(Tile t) { return t == Tile::T256x128 ? 256128 : tile_m(t); }
 // workgroups per CU (LDS: 128 / 64 / 32 / 72 KB per workgroup)
 constexpr int tile_blocks_per_cu(Tile t) { return t == Tile::T256 ? 1 : t == Tile::T64 ? 4 : 2; }
