@@ -45,6 +45,38 @@ constexpr TileRate kTileRate[4] = {
 constexpr double kStreamRate = 4.7e12;
 constexpr double kLaunchSec = 6e-6;
 
+// Seconds of the INT8 GEMM tiles on MI355X: a tile with a k loop of `len` takes a + b len where c + 1 of its kind
+// share the CU (fitted to 512^2 .. 4096^2, s = 16, k = 128 .. 8192, within 8 %).
+struct TileTime {
+    double a[4], b[4];
+};
+constexpr TileTime kTileTime[4] = {
+    {{6.0e-6}, {12.2e-9}},                                                    // T256
+    {{2.2e-6, 3.0e-6}, {4.1e-9, 7.4e-9}},                                     // T128
+    {{2.3e-6, 2.3e-6, 2.4e-6, 2.5e-6}, {3.0e-9, 3.8e-9, 4.8e-9, 5.9e-9}},     // T64
+    {{3.0e-6, 3.6e-6}, {7.9e-9, 14.2e-9}},                                    // T256x128
+};
+// share of a tile's time that a half tile at the edge takes
+constexpr double kHalfTile = 0.62;
+
+// tiles along an extent, the last one a half tile where that holds what is left
+double edge_tiles(int64_t x, int64_t t, int64_t pad) {
+    const int64_t full = x / t, left = x - full * t;
+    return static_cast<double>(full) + (left == 0 ? 0.0 : left <= t / 2 && pad < t ? kHalfTile : 1.0);
+}
+
+// GEMM of rows x cols in tiles t: rounds that fill every CU, then what is left over, fewer to a CU
+double tile_seconds(k::Tile t, int64_t rows, int64_t cols, int planes, int64_t len, int cus) {
+    const TileTime& R = kTileTime[static_cast<int>(t)];
+    const int per = k::tile_blocks_per_cu(t);
+    auto time = [&](int c) { return R.a[c - 1] + R.b[c - 1] * static_cast<double>(len); };
+    const double per_cu = edge_tiles(rows, k::tile_m(t), k::tile_pad_m(t)) * edge_tiles(cols, k::tile_n(t), k::tile_pad_n(t)) *
+                          planes / cus;
+    const double full = std::floor(per_cu / per);
+    const int left = static_cast<int>(std::ceil(per_cu - full * per));
+    return full * time(per) + (left ? time(left) : 0.0);
+}
+
 // distinct balanced panel extents of x: x itself, then round_up(ceil(x / p), 64)
 // for p = 2, 3, ... down to 64 (each value once, largest first)
 template <class F>
@@ -65,17 +97,17 @@ void for_each_panel(int64_t x, F&& f) {
 }
 
 // GEMM seconds of one launch over r x c of the panel grid (tile t, k loops of klen)
-double gemm_seconds(const CallShape& c, const Layout& L, int64_t rows, int64_t cols) {
-    const TileRate& R = kTileRate[static_cast<int>(L.tile)];
-    const double tiles = static_cast<double>(ceil_div(rows, L.TM)) * static_cast<double>(ceil_div(cols, L.TN)) *
-                         L.planes;
-    const double slots = static_cast<double>(c.cus) * k::tile_blocks_per_cu(L.tile);
+double gemm_seconds(const CallShape& c, const Layout& L, k::Tile tile, int64_t rows, int64_t cols) {
+    const TileRate& R = kTileRate[static_cast<int>(tile)];
+    const int64_t TM = k::tile_m(tile), TN = k::tile_n(tile);
+    const double tiles = static_cast<double>(ceil_div(rows, TM)) * static_cast<double>(ceil_div(cols, TN)) * L.planes;
+    const double slots = static_cast<double>(c.cus) * k::tile_blocks_per_cu(tile);
     const double waves = std::ceil(tiles / slots);
     double t = 0;
     for (int64_t k0 = 0; k0 < L.kp; k0 += L.klen) {
         const double len = static_cast<double>(std::min(L.klen, L.kp - k0));
         // one wave of `slots` tiles takes 2 TM TN (len + k0) slots / peak
-        t += waves * 2.0 * L.TM * L.TN * (len + R.k0) * slots / R.peak;
+        t += waves * 2.0 * TM * TN * (len + R.k0) * slots / R.peak;
     }
     return t;
 }
@@ -134,6 +166,28 @@ k::Tile pick_tile(int64_t mb, int64_t nb, int64_t klen, int planes, int forced_c
     return blocks(128, 128) >= 256 ? k::Tile::T128 : k::Tile::T64;
 }
 
+k::Tile call_tile(int64_t mb, int64_t nb, int64_t klen, int planes, int forced_code, int cus) {
+    k::Tile forced;
+    if (k::tile_from_code(forced_code, forced)) return forced;
+    // never pad a small tile up to a bigger macro tile
+    if (std::min(mb, nb) <= 64) return k::Tile::T64;
+    // The fastest by tile_seconds.  GEMM, us, pick_tile's / this one: 1024^3 s = 14 20.2 (128 x 128) / 17.0
+    // (256 x 128), 2048^3 s = 10 89.0 / 82.6, 2048 x 300 x 4096 s = 16 55.4 / 53.5; of 20 sizes from 100^3 to 4096^2
+    // one was slower (130 x 8000 x 1000 35.6 / 37.8, the call the same).  In a batch the neighbours fill the chip,
+    // and its tiles lose (64 products of 64 .. 1024: 513 / 597).
+    k::Tile best = k::Tile::T64;
+    double least = std::numeric_limits<double>::infinity();
+    for (k::Tile t : {k::Tile::T256, k::Tile::T256x128, k::Tile::T128, k::Tile::T64}) {
+        if ((t == k::Tile::T256 && std::min(mb, nb) <= 128) || (t == k::Tile::T256x128 && mb <= 128)) continue;
+        const double s = tile_seconds(t, mb, nb, planes, klen, cus);
+        if (s < least) {
+            least = s;
+            best = t;
+        }
+    }
+    return best;
+}
+
 Layout layout(const CallShape& c, int64_t mb, int64_t nb) {
     Layout L;
     L.g = c.cplx ? 3 : 1;
@@ -141,7 +195,10 @@ Layout layout(const CallShape& c, int64_t mb, int64_t nb) {
     L.kp = round_up(c.k, kKStep);
     L.klen = k_chunk_len(L.kp);
     L.kch = k_chunks(L.kp);
-    L.tile = pick_tile(mb, nb, L.klen, L.planes, c.forced_tile);
+    // (panels of a call that does not fit keep the simpler rule, whose cost the search over them can rely on to
+    // fall with larger panels)
+    L.tile = mb == c.m && nb == c.n ? call_tile(mb, nb, L.klen, L.planes, c.forced_tile, c.cus)
+                                    : pick_tile(mb, nb, L.klen, L.planes, c.forced_tile);
     L.TM = k::tile_m(L.tile);
     L.TN = k::tile_n(L.tile);
     L.mpad = round_up(mb, L.TM);
@@ -171,11 +228,13 @@ double panel_cost(const CallShape& c, int64_t mb, int64_t nb) {
     const int64_t pm = ceil_div(c.m, mb), pn = ceil_div(c.n, nb);
     const int64_t mlast = c.m - (pm - 1) * mb, nlast = c.n - (pn - 1) * nb;
     // GEMM launches: (pm - 1) x (pn - 1) full panel pairs, the ragged last row and column
+    // (priced with the tiles of a panel, the whole call too, so that the panel counts compare)
     double gemm = 0;
-    gemm += static_cast<double>((pm - 1) * (pn - 1)) * gemm_seconds(c, L, mb, nb);
-    gemm += static_cast<double>(pn - 1) * gemm_seconds(c, L, mlast, nb);
-    gemm += static_cast<double>(pm - 1) * gemm_seconds(c, L, mb, nlast);
-    gemm += gemm_seconds(c, L, mlast, nlast);
+    const k::Tile tile = pick_tile(mb, nb, L.klen, L.planes, c.forced_tile);
+    gemm += static_cast<double>((pm - 1) * (pn - 1)) * gemm_seconds(c, L, tile, mb, nb);
+    gemm += static_cast<double>(pn - 1) * gemm_seconds(c, L, tile, mlast, nb);
+    gemm += static_cast<double>(pm - 1) * gemm_seconds(c, L, tile, mb, nlast);
+    gemm += gemm_seconds(c, L, tile, mlast, nlast);
     // bandwidth-bound bytes: each split reads its operand and writes the padded planes;
     // op(A) is split once when it is one row panel, else once per panel pair; the CRT
     // reads every residue byte and reads and writes C

@@ -72,7 +72,9 @@ struct Layout {
     size_t oD = 0, oE = 0, oPA = 0, oPB = 0, oA = 0, oB = 0, oR = 0, total = 0;
 };
 
-// GEMM macro tile for a panel of mb x nb with k loops of klen; forced_code from Tuning::gemm_tile
+// GEMM macro tile for a panel of mb x nb with k loops of klen; forced_code from Tuning::gemm_tile.  call_tile: the
+// panel has the chip to itself; pick_tile: one of a batch.
+k::Tile call_tile(int64_t mb, int64_t nb, int64_t klen, int planes, int forced_code, int cus);
 k::Tile pick_tile(int64_t mb, int64_t nb, int64_t klen, int planes, int forced_code);
 Layout layout(const CallShape& c, int64_t mb, int64_t nb);
 // modelled seconds of the whole call with mb x nb panels on MI355X
