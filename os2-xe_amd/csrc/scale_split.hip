@@ -257,6 +257,8 @@ struct SplitItem {
     uint32_t blocks;  // gx gy, times the parts of the moduli
 };
 
+constexpr uint32_t kStrip = 16;
+
 // What a thread of a split works on.
 template <int Q>
 struct SplitThread {
@@ -275,7 +277,19 @@ struct SplitThread {
             t0 = static_cast<int>(g) * it.tper;
             t1 = min(a.s, t0 + it.tper);
         }
-        const uint32_t by = __builtin_amdgcn_readfirstlane(l / it.gx), bx = l - by * it.gx;
+        // rows first; contiguous rows in strips of kStrip blocks along k, so that what runs together reads runs of
+        // 8 KB of a row, not 512 bytes at a stride that a power of two puts on few channels (MI355X, calls, us,
+        // rows first / strips: 4096^3 s = 8 654 / 640, complex 4096^3 3410 / 3363, k = 200000 20863 / 20810)
+        uint32_t bx, by;
+        if (a.kcontig) {
+            const uint32_t strip = __builtin_amdgcn_readfirstlane(l / (it.gx * kStrip)), in = l - strip * it.gx * kStrip;
+            const uint32_t n = min(kStrip, it.gy - strip * kStrip);
+            bx = __builtin_amdgcn_readfirstlane(in / n);
+            by = strip * kStrip + in - bx * n;
+        } else {
+            by = __builtin_amdgcn_readfirstlane(l / it.gx);
+            bx = l - by * it.gx;
+        }
         constexpr int slots = 64 / Q;
         const int wq = threadIdx.x >> 4;  // strided rows: 16 rows x one slot
         if (a.kcontig) {
