@@ -136,7 +136,7 @@ BatchPlan::BatchPlan(Engine& eng, std::vector<GemmDesc> descs, const std::vector
                 a.X = which == 0 ? g.A : g.B;
                 a.ldx = which == 0 ? g.lda : g.ldb;
                 a.rows = which == 0 ? g.m : g.n;
-                a.rows_pad = round_up(a.rows, q.ftile ? q.ftile : which == 0 ? k::tile_pad_m(q.tile) : k::tile_pad_n(q.tile));
+                a.rows_pad = round_up(a.rows, q.ftile ? 64 : which == 0 ? k::tile_pad_m(q.tile) : k::tile_pad_n(q.tile));
                 a.k = g.k;
                 a.kp = q.kp;
                 a.map = k::PlaneMap::of(q.tile, q.ftile, which == 0 ? q.mpad : q.npad, q.kp);

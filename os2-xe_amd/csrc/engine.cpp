@@ -360,7 +360,7 @@ void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, doubl
         sp.X = sp.kcontig ? X + cw * r0 * ldx : X + cw * r0;
         sp.ldx = ldx;
         sp.rows = rows;
-        sp.rows_pad = round_up(rows, ftile ? ftile : is_b ? k::tile_pad_n(tile_) : k::tile_pad_m(tile_));
+        sp.rows_pad = round_up(rows, ftile ? 64 : is_b ? k::tile_pad_n(tile_) : k::tile_pad_m(tile_));
         sp.k = k;
         sp.kp = kp;
         sp.ex = sp.ex_out = (is_b ? E : D) + r0;

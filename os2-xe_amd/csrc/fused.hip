@@ -271,6 +271,17 @@ __device__ __forceinline__ void tile_coords(const FusedArgs& p, uint32_t w, uint
     tn = in / gs;
 }
 
+// The tile, or where half of it holds the rows or the columns left (128 x 128), that half.  256 products of
+// 64 .. 4096 in 128 x 128 tiles: 11.53 -> 11.38 ms.
+template <int T, int GM, int GN, int NS, int NL>
+__device__ __forceinline__ void fused_edge(const FusedArgs& p, uint32_t tm, uint32_t tn, v4i* smem, const Stamp& st) {
+    if constexpr (T == 128) {
+        if (p.mb - static_cast<int64_t>(tm) * T <= T / 2) return fused_tile<T / 2, T, 2, 4, NS, NL>(p, 2 * tm, tn, smem, st);
+        if (p.nb - static_cast<int64_t>(tn) * T <= T / 2) return fused_tile<T, T / 2, 4, 2, NS, NL>(p, tm, 2 * tn, smem, st);
+    }
+    fused_tile<T, T, GM, GN, NS, NL>(p, tm, tn, smem, st);
+}
+
 template <int T, int NL>
 struct Shape;
 template <int NL>
@@ -296,7 +307,7 @@ __global__ void __launch_bounds__(THREADS, MINB) fused_kernel(FusedArgs p, uint6
     const uint32_t x = blockIdx.x & 7, q = gridDim.x >> 3, r = gridDim.x & 7;
     uint32_t tm, tn;
     tile_coords(p, x * q + min(x, r) + (blockIdx.x >> 3), tm, tn);
-    fused_tile<T, T, S::GM, S::GN, S::NS, NL>(p, tm, tn, smem, st);
+    fused_edge<T, S::GM, S::GN, S::NS, NL>(p, tm, tn, smem, st);
     st.inner(1);
     st.end();
 }
@@ -316,7 +327,7 @@ __global__ void __launch_bounds__(THREADS, MINB) fused_grouped_kernel(const Fuse
     uint32_t tm, tn;
     tile_coords(p, w - start[it], tm, tn);
     const Stamp none(nullptr);
-    fused_tile<T, T, S::GM, S::GN, S::NS, NL>(p, tm, tn, smem, none);
+    fused_edge<T, S::GM, S::GN, S::NS, NL>(p, tm, tn, smem, none);
 }
 
 }  // namespace

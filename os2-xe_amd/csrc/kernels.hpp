@@ -211,7 +211,7 @@ struct CrtArgs {
 void crt(const Stream& st, const CrtArgs& a);
 
 // ---- INT8 GEMMs of all planes and the CRT of a tile in one workgroup --------------
-// a real product of one k-chunk; tile 128 or 64 (square): the planes are padded to it
+// a real product of one k-chunk; tile 128 or 64 (square): the planes hold rows up to a multiple of 64
 struct FusedArgs {
     const int8_t *A, *B;      // planes of op(A), op(B): PlaneMap::by_group
     int64_t kp, plane_a, plane_b;

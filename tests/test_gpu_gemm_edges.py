@@ -64,3 +64,11 @@ def test_edges_of_batches(oz, tile, persistent):
 
     for x, y in zip(run(tile), run(64)):
         assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("s", [8, 12, 16, 20, 24])
+def test_edges_of_fused_tiles(oz, s):
+    for m, n in ((1985, 2048), (2048, 1985), (1921, 1921), (1984, 1983)):
+        A, B, C = rnd(m * 200, 1), rnd(200 * n, 2), torch.zeros(m * n, dtype=torch.float64, device="cuda")
+        oz.gemm("N", "N", m, n, 200, 1.0, A, m, B, 200, 0.0, C, m, s)
+        assert torch.equal(C.view(torch.int64), forced(oz, 64, m, n, 200, s, A, B)), (m, n)
