@@ -33,17 +33,6 @@ void Wide::mul(uint32_t f) {
     if (c) throw std::overflow_error("oz2: integer overflow in plan arithmetic");
 }
 
-uint64_t Wide::divmod(uint64_t d) {
-    // schoolbook division by one 64-bit digit: the running remainder stays below d
-    unsigned __int128 r = 0;
-    for (int i = N - 1; i >= 0; --i) {
-        const unsigned __int128 cur = (r << 64) | v[i];
-        v[i] = static_cast<uint64_t>(cur / d);
-        r = cur % d;
-    }
-    return static_cast<uint64_t>(r);
-}
-
 int Wide::bits() const {
     for (int i = N - 1; i >= 0; --i)
         if (v[i]) return 64 * i + 64 - __builtin_clzll(v[i]);
@@ -110,23 +99,32 @@ Plan make_plan(int s, int64_t k) {
 }
 
 int scale_bits(int s, int64_t k) {
-    // M per s, built once
+    // bit length and the 64 bits from the top one of M per s, built once
     static const struct Products {
-        Wide M[kMaxModuli + 1];
+        int bits[kMaxModuli + 1];
+        uint64_t top[kMaxModuli + 1];
         Products() {
             for (int t = kMinModuli; t <= kMaxModuli; ++t) {
-                M[t] = Wide::of(1);
-                for (int u = 0; u < t; ++u) M[t].mul(moduli(t)[u]);
+                Wide M = Wide::of(1);
+                for (int u = 0; u < t; ++u) M.mul(moduli(t)[u]);
+                bits[t] = M.bits();
+                top[t] = 0;
+                for (int i = 0; i < 64 && i < bits[t]; ++i) {
+                    const int at = bits[t] - 1 - i;
+                    top[t] |= (M.v[at / 64] >> (at % 64) & 1) << (63 - i);
+                }
             }
         }
     } prod;
     // Since k 2^(2t+2) is an integer, k 2^(2t+2) <= M  <=>  2^(2t+2) <= floor(M / k)  <=>
-    // 2t + 2 <= bits(floor(M / k)) - 1, so tk = (bits(floor(M / k)) - 3) / 2 rounded down,
-    // exactly, from one division; floor(M / k) < 16 admits no t >= 1
-    Wide q = prod.M[s];
-    q.divmod(static_cast<uint64_t>(k));
-    if (q.bits() < 5) return 0;
-    return std::min((q.bits() - 3) / 2, kMaxScaleBits);
+    // 2t + 2 <= bits(floor(M / k)) - 1, so tk = (bits(floor(M / k)) - 3) / 2 rounded down;
+    // floor(M / k) < 16 admits no t >= 1.  floor(M / k) has d = bits(M) - bits(k) bits, one more if M >= k 2^d:
+    // k 2^d has as many bits as M and zeros below its first 64, so the top 64 bits decide.  No division: a
+    // selection asks for this some 40 times a problem (64 products: 60 us with the 320-bit division, the GPU idle).
+    const int kb = 64 - __builtin_clzll(static_cast<uint64_t>(k));
+    const int q = prod.bits[s] - kb + (prod.top[s] >= static_cast<uint64_t>(k) << (64 - kb) ? 1 : 0);
+    if (q < 5) return 0;
+    return std::min((q - 3) / 2, kMaxScaleBits);
 }
 
 // ---- tables -------------------------------------------------------------------

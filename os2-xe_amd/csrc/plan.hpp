@@ -51,7 +51,6 @@ struct Wide {
     uint64_t v[N] = {};
     static Wide of(uint64_t x) { Wide w; w.v[0] = x; return w; }
     void mul(uint32_t f);                 // *this *= f; throws std::overflow_error
-    uint64_t divmod(uint64_t d);          // *this /= d (d > 0), returns the remainder
     int bits() const;                     // bit length (0 for zero)
     uint32_t word32(int i) const { return static_cast<uint32_t>(v[i / 2] >> (32 * (i % 2))); }
 };

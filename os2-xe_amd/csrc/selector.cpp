@@ -141,7 +141,10 @@ std::vector<int> Selector::choose(hipStream_t st, const std::vector<SelProblem>&
             const int si = t + kMinModuli;
             if (scale_bits(si, k) < 1) continue;  // s must admit this k
             largest = si;
-            if (!pick && pr[i * kSelOutputs + t] >= tau_) pick = si;
+            if (pr[i * kSelOutputs + t] >= tau_) {
+                pick = si;
+                break;
+            }
         }
         if (largest) {
             s[i] = pick ? pick : largest;
