@@ -181,12 +181,14 @@ StageTimes Engine::stage_times() {
             case Stage::Split: t.split_ms += ms; break;
             case Stage::Gemm: t.gemm_ms += ms; break;
             case Stage::Crt: t.crt_ms += ms; break;
-            case Stage::Fused: {
+            case Stage::Fused:
+            case Stage::ScaleSplit: {
                 // divided as the launch's first workgroup divided its time
-                const uint64_t crt0 = w[k::kStampInner], end = w[k::kStampInner + 1];
-                const double f = end > crt0 && crt0 > b ? static_cast<double>(end - crt0) / static_cast<double>(end - b) : 0.0;
-                t.gemm_ms += ms * (1.0 - f);
-                t.crt_ms += ms * f;
+                const uint64_t second = w[k::kStampInner], end = w[k::kStampInner + 1];
+                const double f = end > second && second > b ? static_cast<double>(end - second) / static_cast<double>(end - b) : 0.0;
+                const bool fused = marks_[i] == Stage::Fused;
+                (fused ? t.gemm_ms : t.scale_ms) += ms * (1.0 - f);
+                (fused ? t.crt_ms : t.split_ms) += ms * f;
                 break;
             }
         }
@@ -368,8 +370,8 @@ void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, doubl
             sp.part = (is_b ? PB : PA) + r0;
             sp.part_ld = is_b ? n : m;
             sp.nkb = k::scale_partials(sp.part_ld, k, sp.kcontig);
-            sp.tk = tk;
         }
+        sp.tk = tk;
         sp.map = is_b ? map_b : map_a;
         sp.P = (is_b ? Bp : Ap) + prow / 64 * sp.map.group;
         sp.plane = is_b ? L.planeB : L.planeA;
@@ -470,7 +472,13 @@ void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, doubl
     };
 
     // scale: exponents of the rows of op(A) and the columns of op(B) (hpp:974-989)
-    timed_on(Stage::Scale, stream_, [&](const k::Stream& on) {
+    const bool scales = k::split_scales(kp, cplx, form);  // with the split
+    auto split_on = [&](const k::Stream& on, const k::SplitArgs& x, const k::SplitArgs& y) {
+        if (scales) k::scale_split(on, x, y);
+        else k::split(on, x, y);
+    };
+    const Stage split_stage = scales ? Stage::ScaleSplit : Stage::Split;
+    if (!scales) timed_on(Stage::Scale, stream_, [&](const k::Stream& on) {
         k::scale(on, {A, lda, m, k, ta != Op::N, cplx, tk, PA, D, fold_a}, {B, ldb, n, k, tb == Op::N, cplx, tk, PB, E, fold_b});
     });
     bool forked = false;
@@ -481,9 +489,8 @@ void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, doubl
         for (int64_t i0 = 0; i0 < m; i0 += mb) {
             const int64_t mbi = std::min(mb, m - i0);
             const bool split_a = ti.pm > 1 || j0 == 0, split_b = nblk == 1 && i0 == 0;
-            if (split_a || split_b) timed_on(Stage::Split, stream_, [&](const k::Stream& on) {
-                if (split_a && split_b) k::split(on, split_args(false, i0, mbi, 0), split_args(true, j0, nbj, 0));
-                else k::split(on, split_a ? split_args(false, i0, mbi, 0) : split_args(true, j0, nbj, 0));
+            if (split_a || split_b) timed_on(split_stage, stream_, [&](const k::Stream& on) {
+                split_on(on, split_args(false, i0, split_a ? mbi : 0, 0), split_args(true, j0, split_b ? nbj : 0, 0));
             });
             if (nblk == 1) {
                 if (ftile) {
@@ -502,7 +509,7 @@ void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, doubl
             if (i0 == 0)  // the B panel's blocks, once per panel column, ahead of the CRTs
                 for (int64_t c = 0; c < nblk; ++c) {
                     const int64_t c0 = c * wb, cols = std::min(wb, nbj - c0);
-                    timed_on(Stage::Split, aux_, [&](const k::Stream& on) { k::split(on, split_args(true, j0 + c0, cols, c0)); });
+                    timed_on(split_stage, aux_, [&](const k::Stream& on) { split_on(on, split_args(false, i0, 0, 0), split_args(true, j0 + c0, cols, c0)); });
                     split_done[c] = sync_event();
                     hip_check(hipEventRecord(split_done[c], aux_), "event record");
                 }

@@ -88,7 +88,7 @@ public:
     int compute_units() const { return cus_; }
 
 private:
-    enum class Stage { Scale, Split, Gemm, Crt, Fused };  // Fused: GEMM and CRT in one launch
+    enum class Stage { Scale, Split, Gemm, Crt, Fused, ScaleSplit };  // Fused: GEMM and CRT in one launch
     // hands every launch of one stage its own stamps
     struct StageTimer final : k::LaunchTimer {
         Engine& e;

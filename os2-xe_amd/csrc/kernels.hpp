@@ -153,8 +153,8 @@ struct SplitArgs {
     const int32_t* ex;    // exponent per row (already offset); unused with part
     const uint64_t* part; // strided rows: the scale kernel's partial maxima (already offset), or null
     int64_t part_ld;      // from one k-block's maxima to the next
-    int nkb, tk;          // with part
-    int32_t* ex_out;      // with part: the exponents are written here
+    int nkb, tk;          // with part (tk: scale_split too)
+    int32_t* ex_out;      // with part, and in scale_split: the exponents are written here
     int8_t* P;            // planes
     PlaneMap map;
     int64_t plane;        // bytes per plane (rows_pad * kp)
@@ -166,6 +166,10 @@ struct SplitArgs {
 };
 void split(const Stream& st, const SplitArgs& a);
 void split(const Stream& st, const SplitArgs& a, const SplitArgs& b);  // both operands of a product (one form)
+// where split_scales(): the split of both operands (or of one: rows_pad 0) with their exponents, no scale() before;
+// rows_pad a multiple of 64, tk and ex_out set
+bool split_scales(int64_t kp, bool cplx, int form);
+void scale_split(const Stream& st, const SplitArgs& a, const SplitArgs& b);
 
 // ---- INT8 GEMM with residue epilogue ------------------------------------------
 struct GemmArgs {

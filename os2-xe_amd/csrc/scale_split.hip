@@ -259,8 +259,8 @@ struct SplitItem {
 
 constexpr uint32_t kStrip = 16;
 
-// What a thread of a split works on.
-template <int Q>
+// What a thread of a split works on.  SCALE: the block holds all k of its 64 rows, 256 threads for each 64-k block.
+template <int Q, bool SCALE = false>
 struct SplitThread {
     int64_t r, ck;    // row, slot
     int t0, t1;       // moduli
@@ -281,7 +281,10 @@ struct SplitThread {
         // 8 KB of a row, not 512 bytes at a stride that a power of two puts on few channels (MI355X, calls, us,
         // rows first / strips: 4096^3 s = 8 654 / 640, complex 4096^3 3410 / 3363, k = 200000 20863 / 20810)
         uint32_t bx, by;
-        if (a.kcontig) {
+        if (SCALE) {
+            by = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+            bx = l;
+        } else if (a.kcontig) {
             const uint32_t strip = __builtin_amdgcn_readfirstlane(l / (it.gx * kStrip)), in = l - strip * it.gx * kStrip;
             const uint32_t n = min(kStrip, it.gy - strip * kStrip);
             bx = __builtin_amdgcn_readfirstlane(in / n);
@@ -291,17 +294,18 @@ struct SplitThread {
             bx = l - by * it.gx;
         }
         constexpr int slots = 64 / Q;
-        const int wq = threadIdx.x >> 4;  // strided rows: 16 rows x one slot
+        const int tid = SCALE ? threadIdx.x & 255 : threadIdx.x, wq = tid >> 4;  // strided rows: 16 rows x one slot
         if (a.kcontig) {
-            r = static_cast<int64_t>(bx) * (256 >> it.lg) + (threadIdx.x >> it.lg);
-            ck = (static_cast<int64_t>(by) << it.lg) + (threadIdx.x & ((1 << it.lg) - 1));
+            r = static_cast<int64_t>(bx) * (256 >> it.lg) + (tid >> it.lg);
+            ck = (static_cast<int64_t>(by) << it.lg) + (tid & ((1 << it.lg) - 1));
         } else {
-            r = static_cast<int64_t>(bx) * (256 / slots) + wq / slots * 16 + (threadIdx.x & 15);
+            r = static_cast<int64_t>(bx) * (256 / slots) + wq / slots * 16 + (tid & 15);
             ck = static_cast<int64_t>(by) * slots + wq % slots;
         }
         ok = r < a.rows_pad && ck < a.kp / Q;
         const bool in = ok && r < a.rows;
         ex = INT32_MIN;
+        if (SCALE) return;
         if (a.part) {
             // the row's maximum from the scale kernel's partials: the four lanes of a wave that hold the row
             // (16 apart) take every fourth
@@ -331,15 +335,13 @@ __device__ __forceinline__ void store_bytes(int8_t* p, const uint32_t (&w)[4]) {
 // Q-byte store per plane.  All loads are issued before any arithmetic and stay
 // inside the matrix: padding rows read row 0 and k past the end reads k - 1, and
 // those values are then zeroed.
-template <int FORM, int Q>
-__device__ __forceinline__ void split_real_body(const SplitItem& it, uint32_t l) {
+template <int FORM, int Q, bool SCALE = false>
+__device__ __forceinline__ void split_real_body(const SplitItem& it, uint32_t l, const Stamp* st = nullptr) {
     const SplitArgs& a = it.a;
     const auto tb = const_tab(a.tab);
-    const SplitThread<Q> th(it, l);
-    if (!th.ok) return;
+    SplitThread<Q, SCALE> th(it, l);
+    if (!SCALE && !th.ok) return;
     const SplitSlot<Q> sl(th.ck);
-    const bool rowzero = th.ex == INT32_MIN;
-    const int e = rowzero ? 0 : th.ex;
     const int64_t rl = th.r < a.rows ? th.r : 0;
 
     uint64_t bits[Q];
@@ -369,6 +371,29 @@ __device__ __forceinline__ void split_real_body(const SplitItem& it, uint32_t l)
             bits[q] = p < a.k ? bits[q] : 0;
         }
     }
+
+    if constexpr (SCALE) {
+        // the rows' maxima: the four threads that share a row in a 64-k block, then the k blocks
+        static_assert(Q == 16, "four threads a row");
+        __shared__ uint64_t red[4][64];
+        uint64_t mx = 0;
+#pragma unroll
+        for (int q = 0; q < Q; ++q) mx = max(mx, bits[q] & 0x7FFFFFFFFFFFFFFFull);
+        mx = max(mx, shfl_xor_u64(mx, a.kcontig ? 1 : 16));
+        mx = max(mx, shfl_xor_u64(mx, a.kcontig ? 2 : 32));
+        const int row = static_cast<int>(th.r & 63);
+        if ((th.ck & 3) == 0) red[threadIdx.x >> 8][row] = mx;
+        __syncthreads();
+        mx = 0;
+        for (int b = 0; b < static_cast<int>(blockDim.x >> 8); ++b) mx = max(mx, red[b][row]);
+        if (th.r < a.rows) {
+            th.ex = exponent_from_maxbits(mx, a.tk);
+            if (th.ck == 0 && th.t0 == 0) a.ex_out[th.r] = th.ex;
+        }
+        st->inner(0);
+    }
+    const bool rowzero = th.ex == INT32_MIN;
+    const int e = rowzero ? 0 : th.ex;
 
     // two to four words (limb_form of tk)
     constexpr Limbs F = static_cast<Limbs>(FORM);
@@ -488,6 +513,19 @@ __global__ void __launch_bounds__(256) split_kernel(SplitItem a, SplitItem b, ui
     st.end();
 }
 
+// Scale and split of both operands where a block can hold all k of its rows (kp <= 256): one pass over the
+// operands and one launch.  MI355X, calls, us, scale and split / this: 64^3 s = 16 22 / 17, 4096 x 4096 x 256
+// s = 16 201.6 / 197.5.
+template <int FORM>
+__global__ void __launch_bounds__(1024) scale_split_kernel(SplitItem a, SplitItem b, uint64_t* ts) {
+    const Stamp st(ts);
+    const bool second = blockIdx.x >= a.blocks;
+    const SplitItem it = second ? b : a;
+    split_real_body<FORM, 16, true>(it, second ? blockIdx.x - a.blocks : blockIdx.x, &st);
+    st.inner(1);
+    st.end();
+}
+
 // grid of one split: KCONTIG: rows x slot groups (tpr threads per row); strided: 16 rows x 16 slots.
 // KCONTIG takes at most one 64-k block per row (tpr <= 64 / Q), so a wave fills whole
 // 1 KB plane blocks (16 rows x 64 k; 8 rows for 8-byte slots) and every 128-byte line of
@@ -586,6 +624,26 @@ void split(const Stream& st, const SplitArgs& x, const SplitArgs& y) {
         case 5: launch_split<2, true>(st, a, b); break;
         default: throw std::logic_error("oz2: no split kernel for this variant");
     }
+}
+
+bool split_scales(int64_t kp, bool cplx, int form) { return !cplx && form < 2 && kp <= 256; }
+
+void scale_split(const Stream& st, const SplitArgs& x, const SplitArgs& y) {
+    SplitItem a = split_item(x), b = split_item(y);
+    a.blocks = a.gx;
+    b.blocks = b.gx;
+    a.gy = b.gy = 1;
+    const uint32_t n = a.blocks + b.blocks;
+    if (n == 0) return;
+    // a workgroup fills half a CU or more, so the moduli are dealt out until every CU has one
+    const int parts = static_cast<int>(std::clamp<uint32_t>(256 / n, 1, 4));
+    for (SplitItem* i : {&a, &b}) {
+        i->tper = (i->a.s + parts - 1) / parts;
+        i->blocks *= static_cast<uint32_t>((i->a.s + i->tper - 1) / i->tper);
+    }
+    const dim3 grid(a.blocks + b.blocks), block(static_cast<unsigned>(4 * x.kp));
+    if (x.form == 0) launch(st, scale_split_kernel<0>, grid, block, a, b);
+    else launch(st, scale_split_kernel<1>, grid, block, a, b);
 }
 
 void split(const Stream& st, const SplitArgs& a) {
