@@ -189,9 +189,11 @@ constexpr int64_t kScaleRowsPerBlock = 64;
 // of operand), instead of a launch that reduces them: 2.2 to 4.3 us at k = 257 to 4096, where calls take 50 to
 // 200.  With more of them the launch's 5 to 20 us are a thousandth of the call.
 constexpr int kScaleFold = 16;
-// Blocks of a launch up to which the split deals a block's moduli to several (a quarter of the CUs: four times as
-// many still run at once).  64^3 s = 16, 2 blocks: 7.8 us an operand before, 5.2 for both.
-constexpr uint32_t kSplitFewBlocks = 64;
+// Blocks that a split of few blocks deals its moduli to: one a CU, four for complex data, whose blocks take three
+// groups of planes.  64^3 s = 16, 2 blocks: 7.8 us an operand undealt, 5.2 for both.  Calls, us, 256 / 512 / 1024 /
+// 2048: complex 777 x 1023 x 515 (300 blocks) 94.6 / 94.5 / 91.5 / 92.3, 1024^3 s = 14 (512) 47.2 / 47.0 / 48.2 /
+// 50.4, 1500 x 900 x 2000 in panels (256) 132.4 / 132.3 / 134.1 / 134.5.
+constexpr uint32_t kSplitBlocks = 256, kSplitBlocksCplx = 1024;
 
 int64_t scale_kblocks(int64_t len, int64_t k) {
     const int64_t rb = (len + kScaleRowsPerBlock - 1) / kScaleRowsPerBlock;
@@ -553,11 +555,12 @@ SplitItem split_item(const SplitArgs& a) {
     it.blocks = it.gx * it.gy;
     return it;
 }
-// Few blocks leave the chip idle while each goes through all its moduli: they are then dealt to up to four
+// Few blocks leave the chip idle while each goes through all its moduli: these are then dealt to up to four
 // times as many, which read the operand again (from the caches).
 void split_parts(SplitItem& it, uint32_t launch_blocks) {
-    if (it.blocks == 0 || launch_blocks > kSplitFewBlocks) return;
-    it.tper = (it.a.s + 3) / 4;
+    const int parts = static_cast<int>(std::min<uint32_t>((it.a.cplx ? kSplitBlocksCplx : kSplitBlocks) / std::max(launch_blocks, 1u), 4));
+    if (it.blocks == 0 || parts < 2) return;
+    it.tper = (it.a.s + parts - 1) / parts;
     it.blocks *= static_cast<uint32_t>((it.a.s + it.tper - 1) / it.tper);
 }
 
