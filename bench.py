@@ -8,8 +8,8 @@ product against a double-double reference.
 
 Also reported:
   roofline      the dominant kernel (the INT8 MFMA GEMM, one launch of s planes
-                per call) against the INT8 dense peak, its time measured with
-                HIP events on the library's stream over the timed region;
+                per call) against the INT8 dense peak, its time measured by
+                the clock stamps of its workgroups over the timed region;
   cpu_baseline  the oracle's CPU restatement of plain Ozaki-II (OpenMP, all
                 host cores) on a bounded sample of the same workload;
   sweep         the other op(A)/op(B) and s values of the same configuration.
@@ -34,8 +34,8 @@ HBM_PEAK_GBS = 8000.0    # MI355X HBM3E, 8 TB/s
 # A bench run cannot count its own traffic (the counters need rocprofv3 around the process), so the
 # line quotes these with their source; the GEMM's fetch (its L2 misses) differs by a few % between boxes.
 MEASURED_GEMM_TRAFFIC = {
-    ("dgemm", 8192, 8192, 8192, 16): (1.4405e10, "profiles/dgemm8192_s16_hbm_traffic.txt (one MI355X, 2026-12-03)"),
-    ("zgemm", 4096, 4096, 4096, 16): (5.6388e9, "profiles/zgemm4096_s16_hbm_traffic.txt (one MI355X, 2026-12-03)"),
+    ("dgemm", 8192, 8192, 8192, 16): (1.5146e10, "profiles/dgemm8192_s16_hbm_traffic.txt (one MI355X, 2026-12-05)"),
+    ("zgemm", 4096, 4096, 4096, 16): (5.6596e9, "profiles/zgemm4096_s16_hbm_traffic.txt (one MI355X, 2026-12-05)"),
 }
 
 
