@@ -11,7 +11,7 @@
 //   residues), 4 stages of 128 k (128 KB of LDS).  64 x 64 tiles: 4 waves of 32 x 32, 3 workgroups per CU
 //   (2 above 16 moduli), 3 stages.
 //
-// Bound: VALU (reduction 6 instructions an entry and plane, CRT 85 to 100 an entry) and the latency of the
+// Bound: VALU (reduction 4 instructions an entry and plane, CRT 85 to 100 an entry) and the latency of the
 // short k loops; the matrix cores are busy 27 % of the time at k = 256, 42 % at k = 1024.  Measured on
 // MI355X, separate -> fused, us (GEMM + CRT): 4096 x 4096 s = 16 k = 128 214 -> 126, k = 256 244 -> 160,
 // k = 512 308 -> 229, k = 1024 439 -> 410; s = 20 k = 256 314 -> 201; s = 8 k = 256 131 -> 116;

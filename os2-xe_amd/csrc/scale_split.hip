@@ -528,8 +528,8 @@ __global__ void __launch_bounds__(1024) scale_split_kernel(SplitItem a, SplitIte
     st.end();
 }
 
-// grid of one split: KCONTIG: rows x slot groups (tpr threads per row); strided: 16 rows x 16 slots.
-// KCONTIG takes at most one 64-k block per row (tpr <= 64 / Q), so a wave fills whole
+// grid of one split: contiguous rows: rows x slot groups (tpr threads per row); strided: 64 rows x 4 slots (32 x 8 for half chunks).
+// Contiguous rows take at most one 64-k block each (tpr <= 64 / Q), so a wave fills whole
 // 1 KB plane blocks (16 rows x 64 k; 8 rows for 8-byte slots) and every 128-byte line of
 // a plane is written by one wave.  With a whole row per workgroup (256 slots) the two
 // rows sharing a line came from different workgroups, usually on different XCDs, and
