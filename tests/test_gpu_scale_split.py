@@ -66,3 +66,35 @@ def test_special_rows_of_short_k(oz, ta, tb, k):
     assert torch.equal(torch.isnan(x), torch.isnan(y)) and torch.isnan(x).any()
     # the two take other widths tk (k enters it), so values agree to the accuracy of 24 moduli only
     assert torch.allclose(x.nan_to_num(0.0), y.nan_to_num(0.0), rtol=1e-13, atol=1e-13)
+
+
+@pytest.mark.parametrize("k", [200, 515])
+@pytest.mark.parametrize("ta,tb", [("N", "T"), ("T", "N")])
+def test_column_blocks_and_panels(oz, ta, tb, k):
+    # exponents written by splits on two streams and panel by panel, against one stream and one panel
+    import torch
+
+    g = torch.Generator(device="cuda").manual_seed(9)
+    m, n, s = 700, 900, 16
+    A = torch.randn(m * k, dtype=torch.float64, device="cuda", generator=g)
+    B = torch.randn(k * n, dtype=torch.float64, device="cuda", generator=g)
+
+    def run():
+        C = torch.zeros(m * n, dtype=torch.float64, device="cuda")
+        oz.gemm(ta, tb, m, n, k, 1.0, A, m if ta == "N" else k, B, k if tb == "N" else n, 0.0, C, m, s)
+        torch.cuda.synchronize()
+        return C.view(torch.int64)
+
+    want = run()
+    whole = oz.workspace_query(ta, tb, m, n, k, s)
+    try:
+        oz.set_tuning(overlap_blocks=3)
+        assert torch.equal(run(), want)
+        oz.set_workspace_limit(whole // 3)
+        assert torch.equal(run(), want)
+        oz.set_tuning()
+        assert torch.equal(run(), want)
+        assert oz.last_tiling().pm * oz.last_tiling().pn > 1
+    finally:
+        oz.set_tuning()
+        oz.set_workspace_limit(0)
