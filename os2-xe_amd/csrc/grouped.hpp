@@ -41,6 +41,19 @@ struct GroupedLaunch {
     }
 };
 
+// blocks of `threads` threads that one launch can hold (fewer than 2^32 threads in x)
+constexpr uint32_t max_blocks(uint32_t threads) { return 0xFFFFFFFFu / threads; }
+
+// adds an item of 256-thread blocks to the last launch of `out`, or to a new one of `kind` where that has no room left
+template <typename T>
+void add_item(std::vector<GroupedLaunch>& out, int kind, const T& item, uint32_t nblocks) {
+    if (out.empty() || nblocks > max_blocks(256) - out.back().blocks) {
+        out.emplace_back();
+        out.back().kind = kind;
+    }
+    out.back().add(item, nblocks);
+}
+
 #if defined(__HIPCC__)
 // item owning block b: the largest p with start[p] <= b (start[0] = 0)
 __device__ __forceinline__ uint32_t owner_of(const uint32_t* __restrict__ start, uint32_t n, uint32_t b) {

@@ -564,9 +564,21 @@ void split_parts(SplitItem& it, uint32_t launch_blocks) {
     it.blocks *= static_cast<uint32_t>((it.a.s + it.tper - 1) / it.tper);
 }
 
+// both operands of a product in one launch, or in one each where a launch cannot hold the blocks of both: operands
+// of 2^26 contiguous rows and more together (m = 67108856, n = 8), each of which one can hold
+template <typename Item>
+void launch_pair(const Stream& st, void (*kernel)(Item, Item, uint64_t*), uint32_t threads, const Item& a, const Item& b) {
+    if (b.blocks <= max_blocks(threads) - std::min(a.blocks, max_blocks(threads))) {
+        launch(st, kernel, dim3(a.blocks + b.blocks), dim3(threads), a, b);
+    } else {
+        launch(st, kernel, dim3(a.blocks), dim3(threads), a, b);
+        launch(st, kernel, dim3(b.blocks), dim3(threads), b, a);
+    }
+}
+
 template <int FORM, bool CPLX>
 void launch_split(const Stream& st, const SplitItem& a, const SplitItem& b) {
-    launch(st, split_kernel<FORM, CPLX>, dim3(a.blocks + b.blocks), dim3(256), a, b);
+    launch_pair(st, split_kernel<FORM, CPLX>, 256, a, b);
 }
 
 // ---- grouped forms: block b of the launch runs block (b - start[p]) of item p
@@ -607,7 +619,7 @@ bool scale_folds(int64_t len, int64_t k, bool kcontig) {
 void scale(const Stream& st, const ScaleJob& ja, const ScaleJob& jb) {
     const ScaleItem a = scale_item(ja), b = scale_item(jb);
     if (a.blocks + b.blocks == 0) return;
-    launch(st, scale_kernel, dim3(a.blocks + b.blocks), dim3(256), a, b);
+    launch_pair(st, scale_kernel, 256, a, b);
     const uint32_t fa = finalize_blocks(ja, a), fb = finalize_blocks(jb, b);
     if (fa + fb) launch(st, scale_finalize_kernel, dim3(fa + fb), dim3(256), a, b, fa);
 }
@@ -644,9 +656,9 @@ void scale_split(const Stream& st, const SplitArgs& x, const SplitArgs& y) {
         i->tper = (i->a.s + parts - 1) / parts;
         i->blocks *= static_cast<uint32_t>((i->a.s + i->tper - 1) / i->tper);
     }
-    const dim3 grid(a.blocks + b.blocks), block(static_cast<unsigned>(4 * x.kp));
-    if (x.form == 0) launch(st, scale_split_kernel<0>, grid, block, a, b);
-    else launch(st, scale_split_kernel<1>, grid, block, a, b);
+    const uint32_t threads = static_cast<uint32_t>(4 * x.kp);
+    if (x.form == 0) launch_pair(st, scale_split_kernel<0>, threads, a, b);
+    else launch_pair(st, scale_split_kernel<1>, threads, a, b);
 }
 
 void split(const Stream& st, const SplitArgs& a) {
@@ -656,29 +668,26 @@ void split(const Stream& st, const SplitArgs& a) {
 }
 
 void prep_scale(std::vector<GroupedLaunch>& out, const std::vector<ScaleJob>& jobs) {
-    GroupedLaunch all, fin;
-    all.kind = kScale;
-    fin.kind = kScaleFin;
+    std::vector<GroupedLaunch> all, fin;
     for (const ScaleJob& j : jobs) {
         const ScaleItem it = scale_item(j);
         if (it.blocks == 0) continue;
-        all.add(it, it.blocks);
-        if (const uint32_t f = finalize_blocks(j, it)) fin.add(it, f);
+        add_item(all, kScale, it, it.blocks);
+        if (const uint32_t f = finalize_blocks(j, it)) add_item(fin, kScaleFin, it, f);
     }
-    for (GroupedLaunch* g : {&all, &fin})
-        if (g->n) out.push_back(std::move(*g));
+    for (auto* v : {&all, &fin})
+        for (GroupedLaunch& g : *v) out.push_back(std::move(g));
 }
 
 void prep_split(std::vector<GroupedLaunch>& out, const std::vector<SplitArgs>& jobs) {
-    GroupedLaunch by[3];
+    std::vector<GroupedLaunch> by[3];
     for (const SplitArgs& a : jobs) {
         const SplitItem it = split_item(a);
         if (it.blocks == 0) continue;
-        by[a.form].kind = kSplitBase + a.form;
-        by[a.form].add(it, it.blocks);
+        add_item(by[a.form], kSplitBase + a.form, it, it.blocks);
     }
-    for (GroupedLaunch& g : by)
-        if (g.n) out.push_back(std::move(g));
+    for (auto& v : by)
+        for (GroupedLaunch& g : v) out.push_back(std::move(g));
 }
 
 bool launch_scale_split_grouped(hipStream_t st, const GroupedLaunch& g) {
