@@ -20,7 +20,7 @@ namespace oz2 {
 namespace k {
 
 // Source of a timed launch's stamps (stage times): kStampWords device words of its own.
-inline constexpr uint32_t kStampWords = 16, kStampEnds = 13, kStampInner = 14;
+inline constexpr uint32_t kStampWords = 16, kStampEnds = 8, kStampInner = 9;
 struct LaunchTimer {
     virtual uint64_t* next() = 0;
 
@@ -40,19 +40,22 @@ struct Stream {
 };
 
 #if defined(__HIPCC__)
-// Begin of a kernel in ts[0], ends in the words from 1 on (ts null: not timed).  Workgroups start in order,
-// so the first one stamps the begin; the end is the latest of the last kStampEnds workgroups, each
-// with a word of its own (one word for all of 256 workgroups, by atomicMax, cost 1.5 us a launch).  The
-// clock only grows, so words left by an earlier launch do not count.
+// Begin of a kernel in ts[0], ends in the next kStampEnds words, one an XCD (ts null: not timed).  Workgroups start in
+// order, so the first one stamps the begin.  Any can be the last to end (64 x 64 x 200000, T,T: 16 blocks of op(A)'s
+// rows outlast the 782 of op(B) behind them: 208 us of scaling, 81 by the last workgroups alone), so all store the
+// time at which their first wave ends into their XCD's word.  The stores of an XCD meet in its L2, and the last one
+// stands, which gives the end to within the flight of a store.  That costs nothing that shows, us:
+// 64^3 s = 16 14.0 / 14.0, 1024^3 s = 14 46.4 / 46.4 (atomicMax of all workgroups: 1 us more with a line an XCD, 7 to 15
+// with one for all).  The clock only grows, so words left by an earlier launch do not count.
 struct Stamp {
     uint64_t* ts;
-    uint32_t b, n;
-    __device__ __forceinline__ explicit Stamp(uint64_t* t)
-        : ts(t), b(blockIdx.y * gridDim.x + blockIdx.x), n(gridDim.x * gridDim.y) {
+    uint32_t b;
+    __device__ __forceinline__ explicit Stamp(uint64_t* t) : ts(t), b(blockIdx.y * gridDim.x + blockIdx.x) {
         if (ts && b == 0 && threadIdx.x == 0) ts[0] = wall_clock64();
     }
     __device__ __forceinline__ void end() const {
-        if (ts && n - b <= kStampEnds && threadIdx.x == 0) ts[n - b] = wall_clock64();
+        constexpr int kXccId = 20 | 3 << 11;  // hardware register 20, four bits from bit 0
+        if (ts && threadIdx.x == 0) ts[1 + (__builtin_amdgcn_s_getreg(kXccId) & (kStampEnds - 1))] = wall_clock64();
     }
     // a moment inside the first workgroup (a kernel of two stages)
     __device__ __forceinline__ void inner(int i) const {
