@@ -157,20 +157,20 @@ void Engine::order_after(hipStream_t to, hipStream_t from) {
 StageTimes Engine::stage_times() {
     StageTimes t;
     if (!profiling_ || marks_.empty()) return t;
-    // (a stream under capture cannot be waited for)
-    if (capturing() || hipStreamSynchronize(stream_) != hipSuccess) {
-        (void)hipGetLastError();
-        return t;
-    }
+    if (capturing()) return t;  // (a stream under capture cannot be waited for)
     constexpr size_t kW = k::kStampWords;
     std::vector<uint64_t> ts(marks_.size() * kW);
+    // copied on the call's own stream: a plain hipMemcpy waits for every blocking stream of the process
+    bool ok = true;
     for (const StampBlock& b : stamps_) {
         if (b.first >= marks_.size()) break;
         const size_t n = std::min(b.slots, marks_.size() - b.first);
-        if (hipMemcpy(ts.data() + b.first * kW, b.p, n * kW * sizeof(uint64_t), hipMemcpyDeviceToHost) != hipSuccess) {
-            (void)hipGetLastError();
-            return t;
-        }
+        ok = ok && hipMemcpyAsync(ts.data() + b.first * kW, b.p, n * kW * sizeof(uint64_t), hipMemcpyDeviceToHost, stream_) == hipSuccess;
+    }
+    ok = hipStreamSynchronize(stream_) == hipSuccess && ok;
+    if (!ok) {
+        (void)hipGetLastError();
+        return t;
     }
     for (size_t i = 0; i < marks_.size(); ++i) {
         const uint64_t* w = ts.data() + i * kW;

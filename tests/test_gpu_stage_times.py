@@ -1,4 +1,6 @@
 """Stage times against events around the call, and what asking for them waits for."""
+import ctypes
+
 import pytest
 import torch
 
@@ -31,3 +33,24 @@ def test_sum_of_uneven_launches(ta, tb):
             runs.append((begin.elapsed_time(end), st.total_ms(), st.as_dict()))
     call, stages, parts = min(runs)
     assert 0.95 * call <= stages <= call, (call, stages, parts)
+
+
+def test_waits_for_the_calls_stream_only():
+    # a blocking stream (one that the legacy default stream waits for) is busy with other work
+    hip = ctypes.CDLL("libamdhip64.so")
+    s = ctypes.c_void_p()
+    assert hip.hipStreamCreate(ctypes.byref(s)) == 0
+    A, B, C = rnd(64 * 64), rnd(64 * 64), rnd(64 * 64)
+    other, done = torch.cuda.ExternalStream(s.value), torch.cuda.Event()
+    with oz2.Ozaki2(torch.cuda.Stream()) as oz:
+        torch.cuda.synchronize()
+        with torch.cuda.stream(other):
+            torch.cuda._sleep(1000000000)  # about 0.4 s
+            done.record()
+        oz.gemm("N", "N", 64, 64, 64, 1.0, A, 64, B, 64, 0.0, C, 64, 16)
+        st = oz.stage_times()
+        waited = done.query()
+        torch.cuda.synchronize()
+    del other
+    assert hip.hipStreamDestroy(s) == 0
+    assert st.gemm_ms > 0 and not waited
