@@ -3,6 +3,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <functional>
 #include <limits>
 #include <stdexcept>
@@ -19,15 +20,19 @@ void hip_check(hipError_t e, const char* what) {
 }  // namespace
 
 Engine::Engine(hipStream_t stream) : stream_(stream) {
-    // the tables and, behind them, the first block of stamps (zeros), in one allocation and one copy
-    constexpr size_t kTabs = (kMaxModuli + 1) * sizeof(TabSet), kStampsAt = (kTabs + 255) / 256 * 256;
-    std::vector<uint64_t> host((kStampsAt + kStampSlots0 * k::kStampWords * sizeof(uint64_t)) / sizeof(uint64_t), 0);
+    // the tables and, behind them, the sums and stamps of the stage times (zeros), in one allocation and one copy
+    constexpr size_t kTabs = (kMaxModuli + 1) * sizeof(TabSet), kSumsAt = (kTabs + 255) / 256 * 256;
+    constexpr size_t kStamps = (1 + k::kStampSlots) * k::kStampWords * sizeof(uint64_t);  // the sums in the first
+    static_assert(k::kStageSums * sizeof(double) <= k::kStampWords * sizeof(uint64_t));
+    std::vector<uint64_t> host((kSumsAt + kStamps) / sizeof(uint64_t), 0);
     make_tabsets(reinterpret_cast<TabSet*>(host.data()));
     const size_t bytes = host.size() * sizeof(uint64_t);
     void* p = nullptr;
     hip_check(hipMalloc(&p, bytes), "table allocation");
     dtabs_ = static_cast<TabSet*>(p);
-    stamps_.push_back({reinterpret_cast<uint64_t*>(static_cast<std::byte*>(p) + kStampsAt), 0, kStampSlots0});
+    stage_sums_ = reinterpret_cast<double*>(static_cast<std::byte*>(p) + kSumsAt);
+    stamps_ = reinterpret_cast<uint64_t*>(stage_sums_) + k::kStampWords;
+    marks_.reserve(k::kStampSlots);
     const hipError_t e = hipMemcpy(p, host.data(), bytes, hipMemcpyHostToDevice);
     if (e != hipSuccess) {
         (void)hipFree(dtabs_);
@@ -57,7 +62,6 @@ Engine::~Engine() {
     if (aux_) (void)hipStreamSynchronize(aux_);
     release_workspace();
     if (aux_) (void)hipStreamDestroy(aux_);
-    for (size_t i = 1; i < stamps_.size(); ++i) (void)hipFree(stamps_[i].p);
     for (auto e : sync_events_) (void)hipEventDestroy(e);
     if (switch_ev_) (void)hipEventDestroy(switch_ev_);
     if (dtabs_) (void)hipFree(dtabs_);
@@ -106,23 +110,6 @@ const Plan& Engine::plan_for(int s, int64_t k) {
     return plan_;
 }
 
-uint64_t* Engine::stamp_slot(size_t mark) {
-    for (const StampBlock& b : stamps_)
-        if (mark - b.first < b.slots) return b.p + (mark - b.first) * k::kStampWords;
-    // the end stamps are maxima: a block starts at zero (a copy from pageable memory has landed when it returns)
-    const std::vector<uint64_t> zero(k::kStampWords * kStampSlots, 0);
-    const size_t bytes = zero.size() * sizeof(uint64_t);
-    void* p = nullptr;
-    hip_check(hipMalloc(&p, bytes), "stage time allocation");
-    const hipError_t e = hipMemcpy(p, zero.data(), bytes, hipMemcpyHostToDevice);
-    if (e != hipSuccess) {
-        (void)hipFree(p);
-        hip_check(e, "stage time allocation");
-    }
-    stamps_.push_back({static_cast<uint64_t*>(p), mark, kStampSlots});
-    return stamps_.back().p;
-}
-
 bool Engine::capturing() const {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream_, &cap) != hipSuccess) {
@@ -133,9 +120,20 @@ bool Engine::capturing() const {
 }
 
 uint64_t* Engine::StageTimer::next() {
-    uint64_t* ts = e.stamp_slot(e.marks_.size());
+    if (e.marks_.size() == k::kStampSlots) e.sum_marks();
     e.marks_.push_back(st);
-    return ts;
+    return e.stamps_ + (e.marks_.size() - 1) * k::kStampWords;
+}
+
+// All stamps are taken: the stages are summed behind the launches of both streams, and the slots are free again.
+void Engine::sum_marks() {
+    k::StampStages stages;
+    std::copy(marks_.begin(), marks_.end(), stages.s);
+    order_after(stream_, aux_);
+    k::sum_stamps(stream_, stamps_, stages, static_cast<uint32_t>(marks_.size()), stage_sums_, !summed_);
+    order_after(aux_, stream_);
+    summed_ = true;
+    marks_.clear();
 }
 
 hipEvent_t Engine::sync_event() {
@@ -156,48 +154,27 @@ void Engine::order_after(hipStream_t to, hipStream_t from) {
 
 StageTimes Engine::stage_times() {
     StageTimes t;
-    if (!profiling_ || marks_.empty()) return t;
+    if (!profiling_ || (marks_.empty() && !summed_)) return t;
     if (capturing()) return t;  // (a stream under capture cannot be waited for)
     constexpr size_t kW = k::kStampWords;
-    std::vector<uint64_t> ts(marks_.size() * kW);
+    std::vector<uint64_t> w((1 + marks_.size()) * kW);
     // copied on the call's own stream: a plain hipMemcpy waits for every blocking stream of the process
-    bool ok = true;
-    for (const StampBlock& b : stamps_) {
-        if (b.first >= marks_.size()) break;
-        const size_t n = std::min(b.slots, marks_.size() - b.first);
-        ok = ok && hipMemcpyAsync(ts.data() + b.first * kW, b.p, n * kW * sizeof(uint64_t), hipMemcpyDeviceToHost, stream_) == hipSuccess;
-    }
+    bool ok = hipMemcpyAsync(w.data(), stage_sums_, w.size() * sizeof(uint64_t), hipMemcpyDeviceToHost, stream_) == hipSuccess;
     ok = hipStreamSynchronize(stream_) == hipSuccess && ok;
     if (!ok) {
         (void)hipGetLastError();
         return t;
     }
-    for (size_t i = 0; i < marks_.size(); ++i) {
-        const uint64_t* w = ts.data() + i * kW;
-        const uint64_t b = w[0], e = *std::max_element(w + 1, w + 1 + k::kStampEnds);
-        const double ms = e > b ? static_cast<double>(e - b) / static_cast<double>(clock_khz_) : 0.0;
-        switch (marks_[i]) {
-            case Stage::Scale: t.scale_ms += ms; break;
-            case Stage::Split: t.split_ms += ms; break;
-            case Stage::Gemm: t.gemm_ms += ms; break;
-            case Stage::Crt: t.crt_ms += ms; break;
-            case Stage::Fused:
-            case Stage::ScaleSplit: {
-                // divided as the launch's first workgroup divided its time
-                const uint64_t second = w[k::kStampInner], end = w[k::kStampInner + 1];
-                const double f = end > second && second > b ? static_cast<double>(end - second) / static_cast<double>(end - b) : 0.0;
-                const bool fused = marks_[i] == Stage::Fused;
-                (fused ? t.gemm_ms : t.scale_ms) += ms * (1.0 - f);
-                (fused ? t.crt_ms : t.split_ms) += ms * f;
-                break;
-            }
-        }
-    }
-    return t;
+    double sums[k::kStageSums] = {};
+    if (summed_) std::memcpy(sums, w.data(), sizeof(sums));
+    for (size_t i = 0; i < marks_.size(); ++i) k::add_stage_ticks(w.data() + (1 + i) * kW, marks_[i], sums);
+    const double khz = static_cast<double>(clock_khz_);
+    return {sums[0] / khz, sums[1] / khz, sums[2] / khz, sums[3] / khz};
 }
 
 void Engine::profile_begin() {
     marks_.clear();
+    summed_ = false;
     calls_ = 0;
     accumulate_ = true;
 }
@@ -292,7 +269,10 @@ void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, doubl
     // synchronization and an allocation)
     const bool capture = capturing();
     const bool timed = profiling_ && !fixed_ws && !capture;
-    if (!accumulate_) marks_.clear();
+    if (!accumulate_) {
+        marks_.clear();
+        summed_ = false;
+    }
     sync_used_ = 0;
     ++calls_;
     // validation (hpp:745-748)

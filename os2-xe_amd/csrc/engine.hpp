@@ -88,7 +88,7 @@ public:
     int compute_units() const { return cus_; }
 
 private:
-    enum class Stage { Scale, Split, Gemm, Crt, Fused, ScaleSplit };  // Fused: GEMM and CRT in one launch
+    using Stage = k::Stage;
     // hands every launch of one stage its own stamps
     struct StageTimer final : k::LaunchTimer {
         Engine& e;
@@ -99,7 +99,7 @@ private:
     void run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, double ai, const double* A, int64_t lda,
              const double* B, int64_t ldb, double br, double bi, double* C, int64_t ldc, int s, bool cplx,
              std::byte* fixed_ws, size_t fixed_bytes);
-    uint64_t* stamp_slot(size_t mark);
+    void sum_marks();
     bool capturing() const;
     hipEvent_t sync_event();  // from a pool reused by every call (a wait binds the record before it)
     void order_after(hipStream_t to, hipStream_t from);
@@ -128,16 +128,12 @@ private:
     TileInfo memo_ti_{};
     k::Tile tile_ = k::Tile::T256;
     hipStream_t aux_ = nullptr;  // second stream of the column-block overlap
-    // stamps of the timed launches, kStampWords words each, in device blocks: the first behind the tables
-    // (enough for any call of a few panels), more when many panels or profile_begin() need them
-    static constexpr size_t kStampSlots0 = 256, kStampSlots = 4096;
-    struct StampBlock {
-        uint64_t* p;
-        size_t first, slots;  // stamps of marks first .. first + slots - 1
-    };
-    std::vector<StampBlock> stamps_;
+    // behind the tables: the sums of the stages over the marks that were summed, and the stamps of the marks since
+    double* stage_sums_ = nullptr;
+    uint64_t* stamps_ = nullptr;            // kStampSlots of kStampWords words each
+    bool summed_ = false;
     int64_t clock_khz_ = 100000;
-    std::vector<Stage> marks_;              // stage of every timed launch; mark i has entry i of stamps_
+    std::vector<Stage> marks_;              // stage of every timed launch since; mark i has entry i of stamps_
     std::vector<hipEvent_t> sync_events_;   // ordering events between the two streams
     size_t sync_used_ = 0;
     bool accumulate_ = false;

@@ -28,6 +28,36 @@ protected:
     ~LaunchTimer() = default;
 };
 
+// The stages that launches are timed as.  Fused: GEMM and CRT in one launch, ScaleSplit: scale and split; their time is
+// divided as the launch's first workgroup divided its own.
+enum class Stage : uint8_t { Scale, Split, Gemm, Crt, Fused, ScaleSplit };
+inline constexpr int kStageSums = 4;  // scale, split, GEMM, CRT
+
+// adds the time of one launch, in ticks of the clock, from its stamps
+__host__ __device__ inline void add_stage_ticks(const uint64_t* w, Stage st, double* sums) {
+    uint64_t e = 0;
+    for (uint32_t i = 1; i <= kStampEnds; ++i) e = e > w[i] ? e : w[i];
+    const uint64_t b = w[0], second = w[kStampInner], end = w[kStampInner + 1];
+    const double ticks = e > b ? static_cast<double>(e - b) : 0.0;
+    if (st != Stage::Fused && st != Stage::ScaleSplit) {
+        sums[static_cast<int>(st)] += ticks;
+        return;
+    }
+    const double f = end > second && second > b ? static_cast<double>(end - second) / static_cast<double>(end - b) : 0.0;
+    const int first = st == Stage::Fused ? static_cast<int>(Stage::Gemm) : static_cast<int>(Stage::Scale);
+    sums[first] += ticks * (1.0 - f);
+    sums[first + 1] += ticks * f;
+}
+
+// Sums of the stages over the first n of the stamps at ts, added to sums (first: stored).  A handle has the stamps of
+// kStampSlots launches; a longer region is summed on the stream, a launch of 3 us in 256, so that no call allocates
+// for its stamps or waits for the GPU.
+inline constexpr uint32_t kStampSlots = 256;
+struct StampStages {
+    Stage s[kStampSlots];
+};
+void sum_stamps(hipStream_t st, const uint64_t* ts, const StampStages& stages, uint32_t n, double* sums, bool first);
+
 // Where a launch goes: a stream and, for timed calls, the timer of its stage.  The kernel stamps the
 // GPU's constant-rate clock itself (Stamp below).  Events recorded around the launches are barrier
 // packets of their own, about 10 us of idle GPU between any two stages (DGEMM 64^3 s = 16: 68 us a call
