@@ -303,7 +303,7 @@ void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, doubl
     const size_t limit = fixed_ws ? fixed_bytes : capture && ws_limit_ == 0 ? ws_size_ : budget();
     const TileInfo ti = plan_for_call(cs, limit);
     const int64_t mb = ti.mb, nb = ti.nb;
-    const Layout L = layout(cs, mb, nb);
+    const Layout L = layout(cs, mb, nb, ti.tile);
     const int64_t kp = L.kp, kch = L.kch, klen = L.klen;
     if (!fixed_ws) ensure_workspace(L.total);
     tiling_ = ti;

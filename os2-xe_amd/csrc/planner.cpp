@@ -188,17 +188,23 @@ k::Tile call_tile(int64_t mb, int64_t nb, int64_t klen, int planes, int forced_c
     return best;
 }
 
-Layout layout(const CallShape& c, int64_t mb, int64_t nb) {
+k::Tile panel_tile(const CallShape& c, int64_t mb, int64_t nb) {
+    const int planes = (c.cplx ? 3 : 1) * c.s;
+    const int64_t klen = k_chunk_len(round_up(c.k, kKStep));
+    // (panels of a call that does not fit keep the simpler rule, whose cost the search over them can rely on to
+    // fall with larger panels)
+    return mb == c.m && nb == c.n ? call_tile(mb, nb, klen, planes, c.forced_tile, c.cus)
+                                  : pick_tile(mb, nb, klen, planes, c.forced_tile);
+}
+
+Layout layout(const CallShape& c, int64_t mb, int64_t nb, k::Tile tile) {
     Layout L;
     L.g = c.cplx ? 3 : 1;
     L.planes = L.g * c.s;
     L.kp = round_up(c.k, kKStep);
     L.klen = k_chunk_len(L.kp);
     L.kch = k_chunks(L.kp);
-    // (panels of a call that does not fit keep the simpler rule, whose cost the search over them can rely on to
-    // fall with larger panels)
-    L.tile = mb == c.m && nb == c.n ? call_tile(mb, nb, L.klen, L.planes, c.forced_tile, c.cus)
-                                    : pick_tile(mb, nb, L.klen, L.planes, c.forced_tile);
+    L.tile = tile;
     L.TM = k::tile_m(L.tile);
     L.TN = k::tile_n(L.tile);
     L.mpad = round_up(mb, L.TM);
@@ -223,8 +229,8 @@ Layout layout(const CallShape& c, int64_t mb, int64_t nb) {
     return L;
 }
 
-double panel_cost(const CallShape& c, int64_t mb, int64_t nb) {
-    const Layout L = layout(c, mb, nb);
+double panel_cost(const CallShape& c, int64_t mb, int64_t nb, k::Tile layout_tile) {
+    const Layout L = layout(c, mb, nb, layout_tile);
     const int64_t pm = ceil_div(c.m, mb), pn = ceil_div(c.n, nb);
     const int64_t mlast = c.m - (pm - 1) * mb, nlast = c.n - (pn - 1) * nb;
     // GEMM launches: (pm - 1) x (pn - 1) full panel pairs, the ragged last row and column
@@ -251,17 +257,24 @@ double panel_cost(const CallShape& c, int64_t mb, int64_t nb) {
 }
 
 TileInfo plan_tiling(const CallShape& c, size_t limit) {
-    auto fits = [&](int64_t mb, int64_t nb) { return layout(c, mb, nb).total <= limit; };
+    // A call that fits whole only with the padding of pick_tile's tile takes that one: 294 x 525 x 87 s = 16 needs 4.6 MiB
+    // with 64 x 64 tiles, 5.8 with call_tile's.  At limits between, us, in panels / whole: this one 31.8 / 17.7, 783 x 507
+    // x 73 s = 24 41.1 / 27.2, complex 163 x 180 x 414 s = 20 48.7 / 31.6, 2404 x 655 x 10945 s = 8 362 / 335.
+    const k::Tile small = pick_tile(c.m, c.n, k_chunk_len(round_up(c.k, kKStep)), (c.cplx ? 3 : 1) * c.s, c.forced_tile);
+    const k::Tile whole = layout(c, c.m, c.n).total <= limit ? panel_tile(c, c.m, c.n) : small;
+    auto tile_of = [&](int64_t mb, int64_t nb) { return mb == c.m && nb == c.n ? whole : panel_tile(c, mb, nb); };
+    auto fits = [&](int64_t mb, int64_t nb) { return layout(c, mb, nb, tile_of(mb, nb)).total <= limit; };
     double best = std::numeric_limits<double>::infinity();
     TileInfo bt;
     auto consider = [&](int64_t mb, int64_t nb) {
         if (!fits(mb, nb)) return;
-        const double t = panel_cost(c, mb, nb);
+        const k::Tile tile = tile_of(mb, nb);
+        const double t = panel_cost(c, mb, nb, tile);
         // strictly cheaper only: among equal costs the first (fewest panels) stays
         if (t < best * (1.0 - 1e-12)) {
             best = t;
-            bt = TileInfo{mb, nb, ceil_div(c.m, mb), ceil_div(c.n, nb), layout(c, mb, nb).kch,
-                          layout(c, mb, nb).total};
+            const Layout L = layout(c, mb, nb, tile);
+            bt = TileInfo{mb, nb, ceil_div(c.m, mb), ceil_div(c.n, nb), L.kch, L.total, tile};
         }
     };
     auto try_rows = [&](int64_t mb) {

@@ -15,13 +15,6 @@
 
 namespace oz2 {
 
-struct TileInfo {
-    int64_t mb = 0, nb = 0;
-    int64_t pm = 0, pn = 0;
-    int64_t k_chunks = 0;
-    size_t workspace_bytes = 0;
-};
-
 namespace k {
 // Macro tiles of the INT8 GEMM (rows of op(A) x columns of op(B) per workgroup of
 // 4 waves).  T256: one workgroup per CU, 4 LDS stages (long k).  T256x128: two
@@ -47,6 +40,14 @@ inline bool tile_from_code(int code, Tile& t) {
     }
 }
 }  // namespace k
+
+struct TileInfo {
+    int64_t mb = 0, nb = 0;
+    int64_t pm = 0, pn = 0;
+    int64_t k_chunks = 0;
+    size_t workspace_bytes = 0;
+    k::Tile tile = k::Tile::T256;  // of the GEMM
+};
 
 // What the planner needs to know of a call.
 struct CallShape {
@@ -76,9 +77,13 @@ struct Layout {
 // panel has the chip to itself; pick_tile: one of a batch.
 k::Tile call_tile(int64_t mb, int64_t nb, int64_t klen, int planes, int forced_code, int cus);
 k::Tile pick_tile(int64_t mb, int64_t nb, int64_t klen, int planes, int forced_code);
-Layout layout(const CallShape& c, int64_t mb, int64_t nb);
+// the tile of a call's panels where memory does not matter: call_tile for all of C in one, else pick_tile
+k::Tile panel_tile(const CallShape& c, int64_t mb, int64_t nb);
+Layout layout(const CallShape& c, int64_t mb, int64_t nb, k::Tile tile);
+inline Layout layout(const CallShape& c, int64_t mb, int64_t nb) { return layout(c, mb, nb, panel_tile(c, mb, nb)); }
 // modelled seconds of the whole call with mb x nb panels on MI355X
-double panel_cost(const CallShape& c, int64_t mb, int64_t nb);
+double panel_cost(const CallShape& c, int64_t mb, int64_t nb, k::Tile tile);
+inline double panel_cost(const CallShape& c, int64_t mb, int64_t nb) { return panel_cost(c, mb, nb, panel_tile(c, mb, nb)); }
 // Tile of the fused GEMM + CRT kernel for panels of mb x nb, 128 or 64, or 0 where the separate kernels are
 // ahead (or the product is complex or has several k-chunks); the panels' planes are laid out as L
 int fused_tile(const CallShape& c, const Layout& L, int64_t mb, int64_t nb);

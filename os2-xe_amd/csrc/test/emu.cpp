@@ -210,5 +210,12 @@ int emu_plan_tiling(const int64_t* sh, uint64_t limit, int64_t* out) {
     }
 }
 uint64_t emu_layout_total(const int64_t* sh, int64_t mb, int64_t nb) { return layout(emu_shape(sh), mb, nb).total; }
+// the tile code of the call's panels in a batch or under a limit (pick_tile), with the chip to itself (call_tile)
+int emu_tile_code(const int64_t* sh, int64_t mb, int64_t nb, int alone) {
+    const CallShape c = emu_shape(sh);
+    const int planes = (c.cplx ? 3 : 1) * c.s;
+    const int64_t klen = layout(c, mb, nb).klen;
+    return k::tile_code(alone ? call_tile(mb, nb, klen, planes, c.forced_tile, c.cus) : pick_tile(mb, nb, klen, planes, c.forced_tile));
+}
 double emu_panel_cost(const int64_t* sh, int64_t mb, int64_t nb) { return panel_cost(emu_shape(sh), mb, nb); }
 }
