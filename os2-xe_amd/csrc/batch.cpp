@@ -86,8 +86,10 @@ BatchPlan::BatchPlan(Engine& eng, std::vector<GemmDesc> descs, const std::vector
         P& q = pp[i];
         const int planes = s_[i];
         if (q.ftile && rounds[{q.ftile, q.plan.NL}] < kFusedRounds) q.ftile = 0;
-        q.mpad = round_up(g.m, k::tile_m(q.tile));
-        q.npad = round_up(g.n, k::tile_n(q.tile));
+        // (the fused kernel's tiles, whatever the problem's own: the split writes the rows of the planes up to a multiple
+        // of 64, and a tile past them would run all its moduli on bytes that nobody wrote)
+        q.mpad = round_up(g.m, q.ftile ? q.ftile : k::tile_m(q.tile));
+        q.npad = round_up(g.n, q.ftile ? q.ftile : k::tile_n(q.tile));
         q.planeA = q.mpad * q.kp;
         q.planeB = q.npad * q.kp;
         q.planeR = q.npad * q.mpad;
