@@ -217,5 +217,10 @@ int emu_tile_code(const int64_t* sh, int64_t mb, int64_t nb, int alone) {
     const int64_t klen = layout(c, mb, nb).klen;
     return k::tile_code(alone ? call_tile(mb, nb, klen, planes, c.forced_tile, c.cus) : pick_tile(mb, nb, klen, planes, c.forced_tile));
 }
+// the fused kernel's tile for the call's panels, or 0
+int emu_fused_tile(const int64_t* sh, int64_t mb, int64_t nb) {
+    const CallShape c = emu_shape(sh);
+    return fused_tile(c, layout(c, mb, nb), mb, nb);
+}
 double emu_panel_cost(const int64_t* sh, int64_t mb, int64_t nb) { return panel_cost(emu_shape(sh), mb, nb); }
 }
