@@ -82,7 +82,10 @@ int oz2_reserve_workspace(oz2_handle h, size_t bytes);
 int oz2_workspace_query(oz2_handle h, int ta, int tb, int64_t m, int64_t n, int64_t k, int num_moduli, int cplx,
                         size_t* bytes);
 
-/* Ozaki2::stage_times / last_tiling / set_tuning / tuning (hpp:712-737) */
+/* Ozaki2::stage_times / last_tiling / set_tuning / tuning (hpp:712-737).  Stage times are the time in the stage's
+ * kernels, by clock stamps that their workgroups write: without the gaps between launches, and with overlap_blocks the
+ * sum over both streams.  A launch that does two stages is divided as its first workgroup divided its time.
+ * oz2_stage_times waits for the handle's stream. */
 int oz2_stage_times(oz2_handle h, oz2_stage_times_t* out);
 int oz2_last_tiling(oz2_handle h, oz2_tile_info_t* out);
 int oz2_set_tuning(oz2_handle h, const oz2_tuning_t* t);

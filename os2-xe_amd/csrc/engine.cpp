@@ -237,9 +237,9 @@ size_t Engine::workspace_for(Op ta, Op tb, int64_t m, int64_t n, int64_t k, int 
 }
 
 int Engine::overlap_blocks() const {
-    // automatic: none.  Measured on MI355X at DGEMM 8192^3 s = 16 (8.56 ms per call in one
-    // stream): 2 blocks 8.62 ms, 4 blocks 8.75, 8 blocks 8.95 - the GEMM, power-limited at
-    // about 1.7 GHz, slows by more than the split and CRT time it hides.
+    // automatic: none.  Measured on MI355X at DGEMM 8192^3 s = 16 (7.57 ms per call in one
+    // stream): 2 blocks 7.73 ms, 4 blocks 7.93, 8 blocks 8.06 - the GEMM, power-limited at
+    // about 1.6 GHz, slows by more than the split and CRT time it hides.
     if (tune_.overlap_blocks >= 0) return std::min(std::max(tune_.overlap_blocks, 1), kMaxOverlapBlocks);
     return 1;
 }

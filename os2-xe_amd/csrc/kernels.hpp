@@ -1,9 +1,11 @@
 // kernels.hpp - host-side launch interface of the gfx950 kernels.
 //
 // Data layout in HBM (all owned by the engine's workspace):
-//   planes   int8  [group][t] then blocked: 1 KB per 16 rows x 64 k of op(A) (or op(B)^T),
-//                  1 KB blocks of 16 rows x 64 k (PlaneMap); rows padded with zeros to
-//                  the GEMM tile, k to kp
+//   planes   int8  [group][t] of op(A) and op(B)^T in 1 KB blocks of 16 rows x 64 k (PlaneMap).  The split writes
+//                  zeros up to kp along k and up to a multiple of the half tile of the GEMM (tile_pad_m, tile_pad_n; 64
+//                  for the fused kernel) along the rows; a plane has room for whole tiles.  A tile may read the rows
+//                  behind those written, whatever they hold: they only enter sums of rows or columns that lie outside C
+//                  and are not stored to it.
 //   residues uint8 [chunk][group][t][j][ldr]  GEMM results reduced mod m_t, i contiguous
 //   D, E     int32 exponents per row of op(A) / column of op(B)
 #pragma once
@@ -180,7 +182,7 @@ struct SplitArgs {
     const double* X;      // op(X) rows start at row r0 (already offset)
     int64_t ldx;
     int64_t rows;         // valid rows of this block
-    int64_t rows_pad;     // rows written (>= rows, multiple of 32)
+    int64_t rows_pad;     // rows written (>= rows, multiple of 32, in scale_split of 64)
     int64_t k;            // valid k
     int64_t kp;           // padded k (multiple of 128)
     const int32_t* ex;    // exponent per row (already offset); unused with part
@@ -190,11 +192,11 @@ struct SplitArgs {
     int32_t* ex_out;      // with part, and in scale_split: the exponents are written here
     int8_t* P;            // planes
     PlaneMap map;
-    int64_t plane;        // bytes per plane (rows_pad * kp)
+    int64_t plane;        // bytes from plane to plane (at least rows_pad * kp)
     int64_t group;        // bytes per group of s planes (complex)
     int s;
     bool kcontig, cplx, conj;
-    int form;             // limb_form(tk): octets of the offset value 8, 12 or 14
+    int form;             // limb_form(tk): two, three or four words of base 2^31
     const TabSet* tab;    // device tables of this s
 };
 void split(const Stream& st, const SplitArgs& a);

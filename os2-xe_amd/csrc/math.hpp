@@ -123,11 +123,11 @@ OZ2_HD uint64_t scaled_mag62(uint64_t bits, int e) {
 }
 
 // Words of x = RNE(v 2^e) in base 2^31, x = sum_w (a[w] - 2^31) 2^(31 w): the residue chain takes one v_dot4 a word
-//   Octets8  two words, |x| <= 2^61;   Octets12  three, |x| <= 2^92 (every plan has tk <= 91);
-//   Octets14 four, |x| <= 2^100.
-enum class Limbs { Octets8, Octets12, Octets14 };
+//   Words2  two words, |x| <= 2^61;   Words3  three, |x| <= 2^92 (every plan has tk <= 91);
+//   Words4  four, |x| <= 2^100.
+enum class Limbs { Words2, Words3, Words4 };
 template <Limbs F>
-inline constexpr int kLimbWords = F == Limbs::Octets8 ? 2 : F == Limbs::Octets12 ? 3 : 4;
+inline constexpr int kLimbWords = F == Limbs::Words2 ? 2 : F == Limbs::Words3 ? 3 : 4;
 
 // Adding 1.5 2^52 + 2^31 units of 2^(31 w) leaves word w, rounded to nearest, in the low half of the sum's bits;
 // subtracting that is exact, and the remainder of at most half a unit goes to the next word.  So the top word is
@@ -180,9 +180,9 @@ OZ2_HD uint32_t sym_float(uint32_t F, uint32_t m, float rm) {
     return mad_i24(static_cast<int32_t>(q), -static_cast<int32_t>(m), F);
 }
 
-// Chain of x's words for modulus index t from `start`: start + sum over the octets of (2^(31 w + 8 j) mod m)
+// Chain of x's words for modulus index t from `start`: start + sum over the words' bytes of byte (2^(31 w + 8 j) mod m)
 template <Limbs F, typename Tab>
-OZ2_HD uint32_t octet_chain(const uint32_t (&a)[4], Tab tb, int t, uint32_t start) {
+OZ2_HD uint32_t word_chain(const uint32_t (&a)[4], Tab tb, int t, uint32_t start) {
     uint32_t w = udot4(a[0], tb->c8[t][0], start);
     w = udot4(a[1], tb->c8[t][1], w);
     if (kLimbWords<F> > 2) w = udot4(a[2], tb->c8[t][2], w);
@@ -194,12 +194,12 @@ OZ2_HD uint32_t octet_chain(const uint32_t (&a)[4], Tab tb, int t, uint32_t star
 //   EXACT, t = 1 (m = 255 in the sets of up to six moduli) and four words: w = v - h by sym_m23 with v = x + h (mod m), v < 2^20;
 //   else sym_float: one instruction less, also for the sum.
 template <Limbs F>
-inline constexpr bool kFloatResidues = F != Limbs::Octets14;
+inline constexpr bool kFloatResidues = F != Limbs::Words4;
 template <Limbs F, bool EXACT, typename Tab>
 OZ2_HD uint32_t sym_residue(const uint32_t (&a)[4], Tab tb, int t) {
     constexpr int f = static_cast<int>(F);
-    if (EXACT) return sym_m23(octet_chain<F>(a, tb, t, tb->offh[f][t]), tb->m[t], tb->mu[t], tb->h2[t]);
-    return sym_float(octet_chain<F>(a, tb, t, tb->fstart[f][t]), tb->m[t], tb->rm[t]);
+    if (EXACT) return sym_m23(word_chain<F>(a, tb, t, tb->offh[f][t]), tb->m[t], tb->mu[t], tb->h2[t]);
+    return sym_float(word_chain<F>(a, tb, t, tb->fstart[f][t]), tb->m[t], tb->rm[t]);
 }
 template <Limbs F, bool EXACT, typename Tab>
 OZ2_HD void sym_residues(const uint32_t (&a)[4], const uint32_t (&b)[4], Tab tb, int t, uint32_t (&out)[3]) {
@@ -207,12 +207,12 @@ OZ2_HD void sym_residues(const uint32_t (&a)[4], const uint32_t (&b)[4], Tab tb,
     const uint32_t m = tb->m[t];
     if (EXACT) {
         const uint32_t mu = tb->mu[t], h2 = tb->h2[t];
-        out[0] = sym_m23(octet_chain<F>(a, tb, t, tb->offh[f][t]), m, mu, h2);
-        out[1] = sym_m23(octet_chain<F>(b, tb, t, tb->offh[f][t]), m, mu, h2);
+        out[0] = sym_m23(word_chain<F>(a, tb, t, tb->offh[f][t]), m, mu, h2);
+        out[1] = sym_m23(word_chain<F>(b, tb, t, tb->offh[f][t]), m, mu, h2);
         out[2] = sym_m23(out[0] + out[1] + m, m, mu, h2);  // both in [-h, h]: v = the sum + m + h > 0
         return;
     }
-    const uint32_t x = octet_chain<F>(a, tb, t, tb->fstart[f][t]), y = octet_chain<F>(b, tb, t, tb->fstart[f][t]);
+    const uint32_t x = word_chain<F>(a, tb, t, tb->fstart[f][t]), y = word_chain<F>(b, tb, t, tb->fstart[f][t]);
     const float rm = tb->rm[t];
     out[0] = sym_float(x, m, rm);
     out[1] = sym_float(y, m, rm);
@@ -260,12 +260,12 @@ OZ2_HD uint32_t acc_residue(uint32_t x, Tab tb, int t) {
     return residue_word(x + tb->c30[t], tb->m[t], tb->mg[t]) & 0xFFu;
 }
 
-// Exact reconstruction of one entry from its limb and quotient sums (as rows of the
-// matrix product of TabSet::Wd and Kc, or by dot products); NL = 32-bit words of M.  The quotient q = round(sum_t r_t y_t / m_t) is taken in 16.16 fixed point: with
-// F_t = round(2^16 y_t / m_t) the sum sum_t r_t F_t / 2^16 is within s * 255 * 2^-17 < 0.05 of
-// the exact one, which lies within 1/4 of q whenever |C'| <= M/4 (the scaling guarantees it),
-// so rounding it gives q (the reference's fp32 estimate gives the same q for the same reason).
-//
+// Exact reconstruction of one entry from its limb and quotient sums (as rows of the matrix product of TabSet::Wd and
+// Kc, or by dot products); NL = 32-bit words of M.  The quotient q = round(sum_t r_t y_t / m_t) is taken in 16.16 fixed
+// point: with F_t = round(2^16 y_t / m_t) the sum sum_t r_t F_t / 2^16 is within s * 255 * 2^-17 < 0.05 of the exact
+// one, which lies within 1/4 of q whenever |C'| <= M/4 (the scaling guarantees it), so rounding it gives q (the
+// reference's fp32 estimate gives the same q for the same reason).
+
 // keeps the compiler from merging the operations before and after
 OZ2_HD void settle(int32_t& x) {
 #if defined(__HIP_DEVICE_COMPILE__)

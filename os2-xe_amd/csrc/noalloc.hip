@@ -9,9 +9,10 @@
 // rejected with OZ2_INVALID_ARGUMENT before anything is enqueued.
 //
 // Every call on one GPU shares that GPU's array and leaves its contents behind.
-// Nothing in it needs to start at zero: each launch writes all it reads later
-// (the split writes its padding rows and k as zeros, the GEMM every residue of
-// its padded tiles).  Calls that overlap on one GPU - from two handles on two
+// Nothing in it needs to start at zero: the split writes its padding rows and k
+// as zeros, the GEMM every residue that the CRT reads.  What a tile reads past
+// the padding rows (kernels.hpp) are bytes of the array that an earlier call left;
+// they enter no stored result.  Calls that overlap on one GPU - from two handles on two
 // streams, or two threads - race on the array; one in-order stream per GPU, or
 // the caller's own ordering, keeps them apart.
 #include <hip/hip_runtime.h>

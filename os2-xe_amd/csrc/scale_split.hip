@@ -497,7 +497,7 @@ __device__ __forceinline__ void split_cplx_body(const SplitItem& it, uint32_t l)
         plane(t, [&](words x, words y, bytes r) { sym_residues<F, !kFloatResidues<F>>(x, y, tb, t, r); });
 }
 
-// bytes per thread slot: half chunks for wide complex values (their 2 x 4 octet words
+// bytes per thread slot: half chunks for wide complex values (their 2 x 4 words
 // per element would not fit 16 elements in registers), whole chunks otherwise
 constexpr int split_q(int form, bool cplx) { return form != 0 && cplx ? 8 : 16; }
 template <int FORM, bool CPLX>

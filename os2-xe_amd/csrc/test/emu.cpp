@@ -60,12 +60,12 @@ void split_cplx_form(const double* re, const double* im, const int32_t* e, int64
 extern "C" {
 
 // symmetric int8 residues of RNE(v_i * 2^e_i): planes[t * n + i]; e = INT32_MIN gives 0.
-// the octets of u = 2^OFF + x: 8 bytes for tk <= 62, else 14
+// two to four words of base 2^31 (limb_form of tk)
 void emu_split(const double* v, const int32_t* e, int64_t n, int s, int tk, int8_t* planes) {
     switch (limb_form(tk)) {
-        case 0: split_form<math::Limbs::Octets8>(v, e, n, s, planes); break;
-        case 1: split_form<math::Limbs::Octets12>(v, e, n, s, planes); break;
-        default: split_form<math::Limbs::Octets14>(v, e, n, s, planes); break;
+        case 0: split_form<math::Limbs::Words2>(v, e, n, s, planes); break;
+        case 1: split_form<math::Limbs::Words3>(v, e, n, s, planes); break;
+        default: split_form<math::Limbs::Words4>(v, e, n, s, planes); break;
     }
 }
 
@@ -73,9 +73,9 @@ void emu_split(const double* v, const int32_t* e, int64_t n, int s, int tk, int8
 void emu_split_cplx(const double* re, const double* im, const int32_t* e, int64_t n, int s, int tk, int conj,
                     int8_t* planes) {
     switch (limb_form(tk)) {
-        case 0: split_cplx_form<math::Limbs::Octets8>(re, im, e, n, s, conj, planes); break;
-        case 1: split_cplx_form<math::Limbs::Octets12>(re, im, e, n, s, conj, planes); break;
-        default: split_cplx_form<math::Limbs::Octets14>(re, im, e, n, s, conj, planes); break;
+        case 0: split_cplx_form<math::Limbs::Words2>(re, im, e, n, s, conj, planes); break;
+        case 1: split_cplx_form<math::Limbs::Words3>(re, im, e, n, s, conj, planes); break;
+        default: split_cplx_form<math::Limbs::Words4>(re, im, e, n, s, conj, planes); break;
     }
 }
 
