@@ -4,6 +4,7 @@
 // fixed-point CRT quotient estimate, whose error is bounded far below its margin.
 #pragma once
 #include <cstdint>
+#include <type_traits>
 
 #include "plan.hpp"
 
@@ -219,11 +220,13 @@ OZ2_HD void sym_residues(const uint32_t (&a)[4], const uint32_t (&b)[4], Tab tb,
     out[2] = sym_float(x + y - tb->fb[t], m, rm);
 }
 
-// int8 byte of the symmetric residue of x for modulus index t (m = 256 only at t = 0, m = 255 only at t = 1)
-template <Limbs F, typename Tab>
-OZ2_HD uint32_t sym_byte(const uint32_t (&a)[4], Tab tb, int t) {
-    if (t == 0) return a[0] & 0xFFu;  // m = 256: the words' units are multiples of it
-    return (t == 1 || !kFloatResidues<F> ? sym_residue<F, true>(a, tb, t) : sym_residue<F, false>(a, tb, t)) & 0xFFu;
+// The moduli t0 .. t1 - 1 of a split, by the form of their residues: low() for t = 0 (m = 256: the words' units are
+// multiples of it, the low byte of word 0 is the residue), plane(t, exact) for the others (sym_residue).
+template <Limbs F, typename Low, typename Plane>
+OZ2_HD void for_moduli(int t0, int t1, const Low& low, const Plane& plane) {
+    if (t0 == 0) low();
+    if (t0 <= 1 && t1 > 1) plane(1, std::true_type{});
+    for (int t = t0 > 2 ? t0 : 2; t < t1; ++t) plane(t, std::bool_constant<!kFloatResidues<F>>{});
 }
 
 // the low bytes of b0..b3 packed into one word (b0 lowest): two v_perm_b32 (each
@@ -254,10 +257,6 @@ OZ2_HD uint32_t pack_lo_halves(uint32_t a, uint32_t b) {
 // byte of the returned word is u - q m.  m = 256 has mg = c30 = 0: the low byte of x.
 OZ2_HD uint32_t residue_word(uint32_t u, uint32_t m, uint32_t mg) {
     return mad_i24(static_cast<int32_t>(mulhi32(u, mg) >> 7), -static_cast<int32_t>(m), u);
-}
-template <typename Tab>
-OZ2_HD uint32_t acc_residue(uint32_t x, Tab tb, int t) {
-    return residue_word(x + tb->c30[t], tb->m[t], tb->mg[t]) & 0xFFu;
 }
 
 // Exact reconstruction of one entry from its limb and quotient sums (as rows of the matrix product of TabSet::Wd and

@@ -152,7 +152,6 @@ void make_tabsets(TabSet* out) {
             const uint32_t h = (m - 1) / 2;
             tb.m[t] = m;
             tb.mu[t] = static_cast<uint32_t>(((uint64_t{1} << 31) + m - 1) / m);
-            tb.h[t] = h;
             tb.rm[t] = 1.0f / static_cast<float>(m);
             tb.fb[t] = 0x4B000000u + (m * (((1u << 23) + m - 1) / m) - (1u << 23));
             uint32_t K = pow2_mod(31, m) + pow2_mod(62, m);  // two words

@@ -87,10 +87,9 @@ struct TabSet {
     // split (hpp:202-220): Barrett constants and symmetric offsets
     uint32_t m[kMaxModuli];
     uint32_t mu[kMaxModuli];                // ceil(2^31 / m): exact quotients of values below 2^23 (mod_m23)
-    uint32_t h[kMaxModuli];                 // (m - 1) / 2
     uint32_t offh[3][kMaxModuli];           // (h - K mod m) mod m - h (mod 2^32), K = the words' offsets 2^31 2^(31 w) of
                                             // limb_form 0, 1, 2: start of the dot chain that ends at sym_m23
-    uint32_t h2[kMaxModuli];                // 2 h
+    uint32_t h2[kMaxModuli];                // 2 h, h = (m - 1) / 2
     uint32_t c8[kMaxModuli][4];             // [word w] bytes 2^(31 w + 8 j) mod m, j = 0..3 (low first)
     // the chain that ends at sym_float (m <= 253): float 1 / m, bits of the float B = m ceil(2^23 / m), and the
     // chain's start, those bits + (-K mod m)

@@ -404,13 +404,12 @@ __device__ __forceinline__ void split_real_body(const SplitItem& it, uint32_t l,
     for (int q = 0; q < Q; ++q) to_limbs<F>(rowzero ? 0 : bits[q], e, false, limbs[q]);
     int8_t* out = a.P + chunk_offset(th.r, sl.blk, sl.c, a.map) + sl.q0;
     uint32_t w[4] = {0, 0, 0, 0};
-    // plane 0 has m = 256 in every moduli set (the low byte), plane 1 m = 255 (sym_residue)
-    if (th.t0 == 0) {
+    auto low = [&] {
 #pragma unroll
         for (int g = 0; g < Q / 4; ++g)
             w[g] = pack_lo_bytes(limbs[4 * g][0], limbs[4 * g + 1][0], limbs[4 * g + 2][0], limbs[4 * g + 3][0]);
         store_bytes<Q>(out, w);
-    }
+    };
     auto plane = [&](int t, auto exact) {
         constexpr bool E = decltype(exact)::value;
 #pragma unroll
@@ -419,8 +418,7 @@ __device__ __forceinline__ void split_real_body(const SplitItem& it, uint32_t l,
                                  sym_residue<F, E>(limbs[4 * g + 2], tb, t), sym_residue<F, E>(limbs[4 * g + 3], tb, t));
         store_bytes<Q>(out + t * a.plane, w);
     };
-    if (th.t0 <= 1 && th.t1 > 1) plane(1, std::true_type{});
-    for (int t = max(th.t0, 2); t < th.t1; ++t) plane(t, std::bool_constant<!kFloatResidues<F>>{});
+    for_moduli<F>(th.t0, th.t1, low, plane);
 }
 
 // Complex split: three plane groups Re, Im (negated for conj: the sign of the bits), Re+Im, each
@@ -486,15 +484,18 @@ __device__ __forceinline__ void split_cplx_body(const SplitItem& it, uint32_t l)
     };
     typedef const uint32_t (&words)[4];
     typedef uint32_t (&bytes)[3];
-    if (th.t0 == 0)  // m = 256: low bytes
-        plane(0, [](words x, words y, bytes r) {
-            r[0] = x[0];
-            r[1] = y[0];
-            r[2] = x[0] + y[0];
+    for_moduli<F>(
+        th.t0, th.t1,
+        [&] {
+            plane(0, [](words x, words y, bytes r) {
+                r[0] = x[0];
+                r[1] = y[0];
+                r[2] = x[0] + y[0];
+            });
+        },
+        [&](int t, auto exact) {
+            plane(t, [&](words x, words y, bytes r) { sym_residues<F, decltype(exact)::value>(x, y, tb, t, r); });
         });
-    if (th.t0 <= 1 && th.t1 > 1) plane(1, [&](words x, words y, bytes r) { sym_residues<F, true>(x, y, tb, 1, r); });
-    for (int t = max(th.t0, 2); t < th.t1; ++t)
-        plane(t, [&](words x, words y, bytes r) { sym_residues<F, !kFloatResidues<F>>(x, y, tb, t, r); });
 }
 
 // bytes per thread slot: half chunks for wide complex values (their 2 x 4 words

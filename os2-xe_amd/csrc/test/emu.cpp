@@ -29,7 +29,9 @@ void split_form(const double* v, const int32_t* e, int64_t n, int s, int8_t* pla
         __builtin_memcpy(&bits, v + i, 8);
         const bool zero = e[i] == INT32_MIN;
         math::to_limbs<F>(bits, zero ? 0 : e[i], zero, a);
-        for (int t = 0; t < s; ++t) planes[t * n + i] = static_cast<int8_t>(math::sym_byte<F>(a, tb, t));
+        math::for_moduli<F>(
+            0, s, [&] { planes[i] = static_cast<int8_t>(a[0]); },
+            [&](int t, auto exact) { planes[t * n + i] = static_cast<int8_t>(math::sym_residue<F, decltype(exact)::value>(a, tb, t)); });
     }
 }
 
@@ -46,12 +48,20 @@ void split_cplx_form(const double* re, const double* im, const int32_t* e, int64
         const int ee = zero ? 0 : e[i];
         math::to_limbs<F>(br, ee, zero, ar);
         math::to_limbs<F>(conj ? bi ^ (uint64_t{1} << 63) : bi, ee, zero, ai);
-        for (int t = 0; t < s; ++t) {
-            uint32_t r[3] = {ar[0], ai[0], ar[0] + ai[0]};
-            if (t == 1 || (t && !math::kFloatResidues<F>)) math::sym_residues<F, true>(ar, ai, tb, t, r);
-            else if (t) math::sym_residues<F, false>(ar, ai, tb, t, r);
+        auto store = [&](int t, const uint32_t (&r)[3]) {
             for (int g = 0; g < 3; ++g) planes[(g * s + t) * n + i] = static_cast<int8_t>(r[g]);
-        }
+        };
+        math::for_moduli<F>(
+            0, s,
+            [&] {
+                const uint32_t r[3] = {ar[0], ai[0], ar[0] + ai[0]};
+                store(0, r);
+            },
+            [&](int t, auto exact) {
+                uint32_t r[3];
+                math::sym_residues<F, decltype(exact)::value>(ar, ai, tb, t, r);
+                store(t, r);
+            });
     }
 }
 
@@ -93,7 +103,7 @@ int64_t emu_mod_m23_mismatches(int s, int t) {
 // a chain of three words and of the sum of two, where it is used
 int64_t emu_sym_m23_mismatches(int s, int t) {
     const TabSet* tb = tables() + s;
-    const uint32_t m = tb->m[t], h = tb->h[t];
+    const uint32_t m = tb->m[t], h = (m - 1) / 2;
     int64_t bad = 0;
     for (uint32_t v = 0; v < (1u << 20) + 256; ++v) {
         const int32_t got = static_cast<int32_t>(math::sym_m23(v - h, m, tb->mu[t], tb->h2[t]));
@@ -114,7 +124,7 @@ int64_t emu_sym_m23_mismatches(int s, int t) {
 void emu_acc_residue(const int32_t* x, int64_t n, int s, uint8_t* out) {
     const TabSet* tb = tables() + s;
     for (int t = 0; t < s; ++t)
-        for (int64_t i = 0; i < n; ++i) out[t * n + i] = static_cast<uint8_t>(math::acc_residue(static_cast<uint32_t>(x[i]), tb, t));
+        for (int64_t i = 0; i < n; ++i) out[t * n + i] = static_cast<uint8_t>(math::residue_word(static_cast<uint32_t>(x[i]) + tb->c30[t], tb->m[t], tb->mg[t]));
 }
 
 // CRT of residues res[i * s + t] in [0, m_t): out[i] = RNE(C') * 2^-shift[i]
