@@ -125,13 +125,14 @@ uint64_t* Engine::StageTimer::next() {
     return e.stamps_ + (e.marks_.size() - 1) * k::kStampWords;
 }
 
-// All stamps are taken: the stages are summed behind the launches of both streams, and the slots are free again.
+// All stamps are taken: the stages are summed behind the launches of both streams (the second has work of a call only
+// while forked_), and the slots are free again.
 void Engine::sum_marks() {
     k::StampStages stages;
     std::copy(marks_.begin(), marks_.end(), stages.s);
-    order_after(stream_, aux_);
+    if (forked_) order_after(stream_, aux_);
     k::sum_stamps(stream_, stamps_, stages, static_cast<uint32_t>(marks_.size()), stage_sums_, !summed_);
-    order_after(aux_, stream_);
+    if (forked_) order_after(aux_, stream_);
     summed_ = true;
     marks_.clear();
 }
@@ -461,7 +462,7 @@ void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, doubl
     if (!scales) timed_on(Stage::Scale, stream_, [&](const k::Stream& on) {
         k::scale(on, {A, lda, m, k, ta != Op::N, cplx, tk, PA, D, fold_a}, {B, ldb, n, k, tb == Op::N, cplx, tk, PB, E, fold_b});
     });
-    bool forked = false;
+    forked_ = false;
     for (int64_t j0 = 0; j0 < n; j0 += nb) {
         const int64_t nbj = std::min(nb, n - j0);
         const int64_t wb = nblocks > 1 ? round_up((nbj + nblocks - 1) / nblocks, L.TN) : nbj;
@@ -481,9 +482,9 @@ void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, doubl
                 timed_on(Stage::Crt, stream_, [&](const k::Stream& on) { crt_block(on, i0, mbi, j0, 0, nbj); });
                 continue;
             }
-            if (!forked) {  // the second stream starts after everything before it on the caller's
+            if (!forked_) {  // the second stream starts after everything before it on the caller's
                 order_after(aux_, stream_);
-                forked = true;
+                forked_ = true;
             }
             hipEvent_t split_done[kMaxOverlapBlocks], gemm_done[kMaxOverlapBlocks];
             if (i0 == 0)  // the B panel's blocks, once per panel column, ahead of the CRTs
@@ -510,7 +511,7 @@ void Engine::run(Op ta, Op tb, int64_t m, int64_t n, int64_t k, double ar, doubl
             if (i0 + mb < m || j0 + nb < n) order_after(stream_, aux_);
         }
     }
-    if (forked) order_after(stream_, aux_);  // the call ends on the caller's stream
+    if (forked_) order_after(stream_, aux_);  // the call ends on the caller's stream
     hip_check(hipGetLastError(), "kernel launch");
 }
 

@@ -132,6 +132,7 @@ private:
     double* stage_sums_ = nullptr;
     uint64_t* stamps_ = nullptr;            // kStampSlots of kStampWords words each
     bool summed_ = false;
+    bool forked_ = false;                   // the call has work on aux_
     int64_t clock_khz_ = 100000;
     std::vector<Stage> marks_;              // stage of every timed launch since; mark i has entry i of stamps_
     std::vector<hipEvent_t> sync_events_;   // ordering events between the two streams

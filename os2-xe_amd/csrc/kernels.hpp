@@ -52,7 +52,7 @@ __host__ __device__ inline void add_stage_ticks(const uint64_t* w, Stage st, dou
 }
 
 // Sums of the stages over the first n of the stamps at ts, added to sums (first: stored).  A handle has the stamps of
-// kStampSlots launches; a longer region is summed on the stream, a launch of 3 us in 256, so that no call allocates
+// kStampSlots launches; a longer region is summed on the stream, a launch of 3.4 us in 256, so that no call allocates
 // for its stamps or waits for the GPU.
 inline constexpr uint32_t kStampSlots = 256;
 struct StampStages {
