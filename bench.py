@@ -32,7 +32,7 @@ HBM_PEAK_GBS = 8000.0    # MI355X HBM3E, 8 TB/s
 # HBM bytes per INT8 GEMM launch measured with rocprofv3 (FETCH_SIZE and WRITE_SIZE passes of this
 # build's bench.py workloads on one MI355X, each scaled by its reading for a 1 GiB copy kernel).
 # A bench run cannot count its own traffic (the counters need rocprofv3 around the process), so the
-# line quotes these with their source; the GEMM's fetch (its L2 misses) differs by a few % between boxes.
+# line quotes these with their source; the GEMM's fetch (its L2 misses) differs by a few % between GPUs.
 MEASURED_GEMM_TRAFFIC = {
     ("dgemm", 8192, 8192, 8192, 16): (1.5146e10, "profiles/dgemm8192_s16_hbm_traffic.txt (one MI355X, 2026-12-05)"),
     ("zgemm", 4096, 4096, 4096, 16): (5.6596e9, "profiles/zgemm4096_s16_hbm_traffic.txt (one MI355X, 2026-12-05)"),

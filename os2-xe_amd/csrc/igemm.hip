@@ -30,7 +30,8 @@
 // the residue epilogue of one workgroup then overlaps the MFMAs of the other.
 //
 // The large tiles are bound by power: a loop of this instruction on random registers alone runs at 3.53 Pop/s
-// (1.76 GHz), on constant ones at 4.8 (8192^3, 16 planes, on the same box: 2.76, 1.63 GHz).  So consecutive MFMAs share an operand: the column blocks
+// (1.76 GHz), on constant ones at 4.8 (8192^3, 16 planes, on the same GPU: 2.76, 1.63 GHz).  So consecutive MFMAs share
+// an operand: the column blocks
 // go back and forth under the row blocks (register loop 3.20 -> 3.27 Pop/s; 4096 x 4096 x 1536 s = 16 444 ->
 // 434 us, 4096^3 s = 16 940 -> 929).
 //

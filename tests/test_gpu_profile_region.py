@@ -41,7 +41,7 @@ def test_calls_do_not_wait(per_plane):
 
 
 # Sums over 100 calls (300 launches and more) and over 20: per call alike.  1024^3 with 14 moduli takes about 42 us of
-# kernels; the clock of a box and the gaps' share move that by a few percent, a lost block of 256 launches by 60 % and more.
+# kernels; a GPU's clock and the gaps' share move that by a few percent, a lost block of 256 launches by 60 % and more.
 @pytest.mark.parametrize("overlap", [1, 4])
 def test_long_region_adds_up(overlap):
     size, s = 1024, 14
